@@ -188,8 +188,7 @@ int mista_das_device(mista_handle* h, float* d_value, float* d_factor, void* str
 /* No counterpart in the reference (frames of NetworkSyncSTAMethod.cpp:93-140
  * each run their own processor): the DAS of n prepared handles, up to 16
  * frames in one launch of the tiled kernel when their launches agree in
- * storage, coherence factor, transmit block and workgroup size and their
- * geometries have been tuned (a frame each handle ran through
+ * storage and tile size and their geometries have been tuned (a frame each handle ran through
  * mista_das_device/mista_process_device); others run one by one.  Every
  * frame writes the images it writes alone.  Work goes on `stream` (NULL:
  * the first handle's), which must be ordered after each handle's
@@ -202,10 +201,11 @@ int mista_das_batch_device(mista_handle* const* handles, uint32_t n, float* cons
  * harnesses that forbid hipMalloc).  Same inputs and outputs and the same
  * images as mista_das_device with the tiled kernel; it calls no hipMalloc
  * or hipFree.  The handle must hold a prepared frame (the preparation sizes
- * every buffer the DAS reads).  The window tables of the launch live in a
- * static device array of 80 MiB that each GPU holds once per process and
- * that every call on that GPU rebuilds: a geometry whose tables need more
- * is refused with MISTA_E_INVALID_PARAM, and calls that overlap on one GPU
+ * every buffer the DAS reads).  The tile delays, window tables and per-rx
+ * sums of the launch live in a static device array of 256 MiB that each GPU
+ * holds once per process and that every call on that GPU rebuilds, a run of
+ * tiles at a time: a geometry whose window tables need more than 80 MiB is
+ * refused with MISTA_E_INVALID_PARAM, and calls that overlap on one GPU
  * (from several threads or streams) race.  Uses the tile shape tuned for the
  * geometry when there is one, else a default; it never tunes.  Stage timing
  * (mista_last_timing) is recorded only if an earlier frame created the
@@ -231,8 +231,9 @@ int mista_query(const mista_handle* h, uint32_t* signal_length, uint32_t* fft_si
 
 /* Select the DAS kernel variant (0 = automatic/tuned, 1 = reference-shaped
  * one-pixel-per-lane gather, 2 = LDS-tiled).  Tile parameters 0 = default;
- * tile_param1 = pairs per chunk (4, 8, or 16 on 512-lane tiles over 128
- * transmits) | ring buffers << 8 | LDS budget in KiB << 16.  Where the
+ * tile_param1 = pairs per transmit step (the receive elements of a
+ * workgroup: 4, 8, or 16 on 512-point tiles) | ring buffers << 8 | LDS budget
+ * in KiB << 16.  Where the
  * variant's tiles do not fit, the rx-parallel form runs instead. */
 int mista_set_kernel(mista_handle* h, int variant, int tile_param0, int tile_param1);
 
@@ -257,7 +258,7 @@ int mista_tuned_kernel(const mista_handle* h, int* tile_param0, int* tile_param1
 /* The configuration of the last DAS launch: tile shape (-1 when the gather
  * kernel ran, -2 the rx-parallel form that runs where no tile fits: per-rx
  * sums a lane per (pixel, rx), then the statistics a lane per pixel) and
- * pairs per chunk | ring buffers << 8 | LDS budget in KiB << 16.  No
+ * pairs per transmit step | ring buffers << 8 | LDS budget in KiB << 16.  No
  * counterpart in the reference. */
 int mista_last_kernel(const mista_handle* h, int* tile_param0, int* tile_param1);
 

@@ -176,7 +176,6 @@ void set_frame_geom(mista_handle* h, uint32_t ns, uint32_t L, hipStream_t s)
 	g.num_elements = h->rows;
 	g.first_tx = h->tx_row0;
 	g.ntx = ntx_of(c);
-	g.ntx_pad = pad_ntx(g.ntx);
 	g.nrx = c.num_elements;
 	g.ns = ns;
 	g.up = c.upsampling_factor;
@@ -205,7 +204,7 @@ void set_frame_geom(mista_handle* h, uint32_t ns, uint32_t L, hipStream_t s)
 	// captured frame graph reuses a tail that an eager frame has cleared)
 	if (!h->capturing) HIP_CHECK(hipMemsetAsync(t + tbytes, 0, tensor_tail_padding(), s));
 	h->d_scale.reserve(nch * sizeof(float));
-	h->d_w.reserve(static_cast<size_t>(g.ntx_pad) * g.nrx * sizeof(float));
+	h->d_w.reserve(static_cast<size_t>(g.ntx) * pad_nrx(g.nrx) * sizeof(float));
 	// apodization buffers too, so that the DAS of a prepared frame allocates nothing
 	h->d_rx_apod.reserve(static_cast<size_t>(g.nrx) * sizeof(float));
 	h->d_tx_apod.reserve(static_cast<size_t>(g.ntx) * sizeof(float));
@@ -403,7 +402,8 @@ size_t handle_device_bytes(const mista_handle* h)
 			h->d_grid.capacity() + h->d_delay.capacity() + h->d_raw.capacity() + h->d_tensor.capacity() +
 			h->d_scale.capacity() + h->d_hpoly.capacity() + h->d_tmp.capacity() + h->d_value.capacity() +
 			h->d_factor.capacity() + h->das_scratch.partial.capacity() + h->das_scratch.bounds.capacity() +
-			h->das_scratch.params.capacity() + prep_device_bytes(h->prep);
+			h->das_scratch.params.capacity() + h->das_scratch.delays.capacity() + h->das_scratch.slots.capacity() +
+			h->das_scratch.partials.capacity() + prep_device_bytes(h->prep);
 }
 }  // namespace mista
 

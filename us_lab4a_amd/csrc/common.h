@@ -85,7 +85,6 @@ struct FrameGeom {
 	uint32_t num_elements;  // rows of the delay table
 	uint32_t first_tx;      // row of transmit 0
 	uint32_t ntx;
-	uint32_t ntx_pad;   // transmits padded to 32/64/128 (multiple of 8 above)
 	uint32_t nrx;
 	uint32_t ns;        // raw samples per channel
 	uint32_t up;        // upsampling factor
@@ -114,13 +113,15 @@ inline uint32_t hilbert_fft_size(uint32_t n)
 // Interpolator.h:64-111 low-pass design (double precision).
 std::vector<double> upsampling_filter(uint32_t up, double half_tw);
 
-// Transmit count padded to the DAS kernel's instantiated sizes.
-inline uint32_t pad_ntx(uint32_t ntx)
+// Receive elements padded to the most that a workgroup of the tiled kernel takes.
+inline uint32_t pad_nrx(uint32_t nrx) { return (nrx + 15) / 16 * 16; }
+// Padded transmit count that table budgets are stated in: 32, 64, 128, above
+// that ceil(ntx / 128) equal blocks of whole 8-transmit chunks.
+inline uint32_t budget_pad_ntx(uint32_t ntx)
 {
 	if (ntx <= 32) return 32;
 	if (ntx <= 64) return 64;
 	if (ntx <= 128) return 128;
-	// above 128: ceil(ntx / 128) equal blocks of whole 8-pair chunks, run in turn
 	const uint32_t nblk = (ntx + 127) / 128;
 	const uint32_t bt = ((ntx + nblk - 1) / nblk + 7) / 8 * 8;
 	return nblk * bt;
@@ -189,9 +190,11 @@ struct DasTuning {
 };
 struct DasScratch {
 	DeviceBuffer partial;           // small device scalars (max window slots)
-	DeviceBuffer bounds;            // per-tile element delay bounds
+	DeviceBuffer delays;            // the tiles' delays in lane order
+	DeviceBuffer bounds;            // their bounds per tile and row
 	DeviceBuffer params;            // per (tile, rx, tx) window words
-	DeviceBuffer partials;          // per-rx sums between transmit blocks (more than 128 transmits)
+	DeviceBuffer slots;             // per tile: slots of its longest window
+	DeviceBuffer partials;          // per-rx sums (tiled: of a slab of tiles; rx-parallel form: of the frame)
 	uint64_t bounds_version = ~0ull;
 	uint64_t params_key = 0;
 	float params_offset = 0.0f;
@@ -202,9 +205,12 @@ struct DasScratch {
 };
 // Bytes of zeroed padding after the analytic tensor (window over-read).
 size_t tensor_tail_padding();
-// Device scratch of the no-allocation DAS entry point (per GPU, static).
-constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(80) << 20;
-// DAS over the handle's resident tensor with its window tables in that
+// The no-allocation DAS entry point: its limit on a geometry's window tables,
+// and its device scratch (per GPU, static), which holds the tables and sums of
+// as many tiles at a time as fit.
+constexpr size_t kNoAllocTableBytes = static_cast<size_t>(80) << 20;
+constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(256) << 20;
+// DAS over the handle's resident tensor with its tables and sums in that
 // scratch: no device allocation; the tuned tile shape when there is one.
 void launch_das_noalloc(const FrameGeom& g, int tuned_p0, int tuned_p1, DasScratch& last, const void* d_tensor,
 		const float* d_delay, const float* d_w, float* d_value, float* d_factor, hipStream_t s);
@@ -220,8 +226,7 @@ struct DasBatchItem {
 	float* factor;
 };
 // The DAS of several prepared frames: frames whose tiled launches agree in
-// storage, coherence factor, transmit block and workgroup size (and whose
-// geometry has been tuned) share one launch of the tiled kernel, up to 16 a
+// storage and tile size (and whose geometry has been tuned) share one launch of the tiled kernel, up to 16 a
 // launch; the rest run one by one.  Returns the number of shared launches.
 uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s);
 void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, const void* d_tensor,

@@ -15,14 +15,15 @@
 //  das_rx_sums_kernel + das_rx_stats_kernel  the fallback where no tile
 //                     fits: a lane per (pixel, rx) sums over the transmits,
 //                     then a lane per pixel folds the per-rx sums in rx order.
-//  das_tile_kernel    a workgroup owns a pixel tile for the whole frame; the
-//                     tx delays of each lane's pixel stay in registers; for
-//                     every (rx, tx) pair the tile's signal window is copied
-//                     HBM -> LDS with direct loads (global_load_lds_dwordx4,
-//                     double-buffered), so each sample pair costs one LDS
-//                     read.  Window start / length / record-end flag per
-//                     (tile, rx, tx) come from a table built once per
-//                     geometry.
+//  das_tile_kernel + das_tile_stats_kernel  the tiled form: a workgroup forms
+//                     the per-rx sums of a tile of pixels for a few receive
+//                     elements; for every (rx, tx) pair the tile's signal
+//                     window is copied HBM -> LDS with direct loads
+//                     (global_load_lds_dwordx4, a ring of buffers), so each
+//                     sample pair costs one LDS read.  Tile delays, window
+//                     starts, lengths and record-end flags come from tables
+//                     built once per geometry.  Then a lane per pixel folds
+//                     the sums in rx order.
 #include "das_common.h"
 
 #include <algorithm>
@@ -34,10 +35,10 @@
 namespace mista {
 
 namespace das {
-extern template void launch_tile_storage<MISTA_STORAGE_F32>(int, const TileBatch&, uint32_t, uint32_t, hipStream_t);
-extern template void launch_tile_storage<MISTA_STORAGE_F16>(int, const TileBatch&, uint32_t, uint32_t, hipStream_t);
-extern template void launch_tile_storage<MISTA_STORAGE_BF16>(int, const TileBatch&, uint32_t, uint32_t, hipStream_t);
-extern template void launch_tile_storage<kStorageReal>(int, const TileBatch&, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<MISTA_STORAGE_F32>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<MISTA_STORAGE_F16>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<MISTA_STORAGE_BF16>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<kStorageReal>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
 }  // namespace das
 
 using namespace das;
@@ -50,7 +51,8 @@ namespace {
 // tx outer, rx inner into one accumulator (VectorialSTAProcessor.h:312-325).
 // CF != NONE: rx outer, tx inner, which yields the same per-rx sums
 // (VectorialSTAProcessor.h:269-284) one rx at a time.
-template<int STORAGE, int CF>
+// RX_OUTER: rx outer without a coherence factor too, the tiled kernel's order.
+template<int STORAGE, int CF, bool RX_OUTER>
 __global__ void __launch_bounds__(256) das_gather_kernel(const DasArgs a)
 {
 	const uint64_t p = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -60,7 +62,7 @@ __global__ void __launch_bounds__(256) das_gather_kernel(const DasArgs a)
 	// pos in [0, L-1) <=> i = trunc(pos) satisfies i + 1 < L; the float
 	// compare also rejects NaN and values past 2^32
 	const float lim = static_cast<float>(L - 1u);
-	if constexpr (CF == MISTA_CF_NONE) {
+	if constexpr (CF == MISTA_CF_NONE && !RX_OUTER) {
 		float sr = 0.0f, si = 0.0f;
 		for (uint32_t t = 0; t < a.ntx; ++t) {
 			const float txo = a.offset + dcol[static_cast<uint64_t>(a.first_tx + t) * a.npix];
@@ -72,7 +74,7 @@ __global__ void __launch_bounds__(256) das_gather_kernel(const DasArgs a)
 					const uint64_t ch = (static_cast<uint64_t>(t) * a.nrx + r) * L + i;
 					const float2 v0 = load_sample<STORAGE>(a.tensor, ch);
 					const float2 v1 = load_sample<STORAGE>(a.tensor, ch + 1);
-					const float w = a.w[static_cast<uint64_t>(r) * a.w_stride + t];
+					const float w = a.weight(r, t);
 					sr = fmaf(fmaf(k, v1.x - v0.x, v0.x), w, sr);
 					si = fmaf(fmaf(k, v1.y - v0.y, v0.y), w, si);
 				}
@@ -93,7 +95,7 @@ __global__ void __launch_bounds__(256) das_gather_kernel(const DasArgs a)
 					const uint64_t ch = (static_cast<uint64_t>(t) * a.nrx + r) * L + i;
 					const float2 v0 = load_sample<STORAGE>(a.tensor, ch);
 					const float2 v1 = load_sample<STORAGE>(a.tensor, ch + 1);
-					const float w = a.w[static_cast<uint64_t>(r) * a.w_stride + t];
+					const float w = a.weight(r, t);
 					ar = fmaf(fmaf(k, v1.x - v0.x, v0.x), w, ar);
 					ai = fmaf(fmaf(k, v1.y - v0.y, v0.y), w, ai);
 				}
@@ -121,7 +123,6 @@ __global__ void __launch_bounds__(256) das_rx_sums_kernel(const DasArgs a)
 	const float* dcol = a.delay + p;
 	const float lim = static_cast<float>(a.L - 1u);
 	const float drx = dcol[static_cast<uint64_t>(r) * a.npix];
-	const float* wrow = a.w + static_cast<uint64_t>(r) * a.w_stride;
 	float ar = 0.0f, ai = 0.0f;
 	for (uint32_t t = 0; t < a.ntx; ++t) {
 		const float pos = (a.offset + dcol[static_cast<uint64_t>(a.first_tx + t) * a.npix]) + drx;
@@ -131,7 +132,7 @@ __global__ void __launch_bounds__(256) das_rx_sums_kernel(const DasArgs a)
 			const uint64_t ch = (static_cast<uint64_t>(t) * a.nrx + r) * a.L + i;
 			const float2 v0 = load_sample<STORAGE>(a.tensor, ch);
 			const float2 v1 = load_sample<STORAGE>(a.tensor, ch + 1);
-			const float w = wrow[t];
+			const float w = a.weight(r, t);
 			ar = fmaf(fmaf(k, v1.x - v0.x, v0.x), w, ar);
 			ai = fmaf(fmaf(k, v1.y - v0.y, v0.y), w, ai);
 		}
@@ -166,82 +167,128 @@ void launch_rx_parallel(const FrameGeom& g, const DasArgs& a, hipStream_t s)
 	}
 }
 
-template<int STORAGE>
+template<int STORAGE, bool RX_OUTER>
 void launch_gather(const FrameGeom& g, const DasArgs& a, hipStream_t s)
 {
 	const dim3 grid(static_cast<uint32_t>((g.npix + 255) / 256));
 	switch (g.cf_kind) {
 	case MISTA_CF_NONE:
-		hipLaunchKernelGGL((das_gather_kernel<STORAGE, MISTA_CF_NONE>), grid, dim3(256), 0, s, a);
+		hipLaunchKernelGGL((das_gather_kernel<STORAGE, MISTA_CF_NONE, RX_OUTER>), grid, dim3(256), 0, s, a);
 		break;
 	case MISTA_CF_PCF:
-		hipLaunchKernelGGL((das_gather_kernel<STORAGE, MISTA_CF_PCF>), grid, dim3(256), 0, s, a);
+		hipLaunchKernelGGL((das_gather_kernel<STORAGE, MISTA_CF_PCF, true>), grid, dim3(256), 0, s, a);
 		break;
 	default:
-		hipLaunchKernelGGL((das_gather_kernel<STORAGE, MISTA_CF_SCF>), grid, dim3(256), 0, s, a);
+		hipLaunchKernelGGL((das_gather_kernel<STORAGE, MISTA_CF_SCF, true>), grid, dim3(256), 0, s, a);
 		break;
 	}
+	HIP_CHECK(hipGetLastError());
 }
 
-// Per-tile (min, max) of every element's delay.  One workgroup per tile.
-__global__ void __launch_bounds__(256) tile_bounds_kernel(const float* __restrict__ delay, uint64_t npix,
-		uint32_t num_elements, TileGeom tg, float2* __restrict__ bounds)
+template<bool RX_OUTER>
+void launch_gather_any(const FrameGeom& g, const DasArgs& a, hipStream_t s)
 {
-	// Each wave takes every fourth element and reduces over the tile's
-	// points with shuffles (no workgroup barrier per element); the points'
-	// table offsets are computed once.  Lanes outside the grid read the point
-	// they shadow, as in the DAS kernels.
-	constexpr uint32_t kMaxPts = 512 / 64;
+	switch (g.storage) {
+	case MISTA_STORAGE_F32: launch_gather<MISTA_STORAGE_F32, RX_OUTER>(g, a, s); break;
+	case MISTA_STORAGE_F16: launch_gather<MISTA_STORAGE_F16, RX_OUTER>(g, a, s); break;
+	case kStorageReal: launch_gather<kStorageReal, RX_OUTER>(g, a, s); break;
+	default: launch_gather<MISTA_STORAGE_BF16, RX_OUTER>(g, a, s); break;
+	}
+}
+
+// A lane per tile point: its per-rx sums (the tiled kernel's, [tiles][nrx]
+// [tile points]) in rx order through the same statistics as the other forms.
+// Bound by reading the sums once (8 bytes per pixel and receive element).
+template<int CF>
+__global__ void __launch_bounds__(256) das_tile_stats_kernel(const DasArgs a, const TileGeom tg, uint32_t tile0,
+		uint32_t npts)
+{
+	const uint32_t per = npts / 256;
+	const uint32_t tl = blockIdx.x / per, q = (blockIdx.x % per) * 256 + threadIdx.x;
+	uint32_t col, row;
+	bool valid;
+	tg.pixel(tile0 + tl, q, col, row, valid);
+	if (!valid) return;
+	const float2* src = a.partial + static_cast<uint64_t>(tl) * a.nrx * npts + q;
+	PixelStats<CF> st;
+	uint32_t r = 0;
+	for (; r + 4 <= a.nrx; r += 4) {   // four loads in flight
+		float2 v[4];
+#pragma unroll
+		for (uint32_t k = 0; k < 4; ++k) v[k] = src[static_cast<uint64_t>(r + k) * npts];
+#pragma unroll
+		for (uint32_t k = 0; k < 4; ++k) st.add_rx(v[k].x, v[k].y, r + k == 0);
+	}
+	for (; r < a.nrx; ++r) {
+		const float2 v = src[static_cast<uint64_t>(r) * npts];
+		st.add_rx(v.x, v.y, r == 0);
+	}
+	st.write(a, static_cast<uint64_t>(col) * tg.n2 + row);
+}
+
+// Delays of a run of tiles in lane order: [tiles][nrx + ntx][npts], the rx
+// rows as in the delay table, the tx rows with the offset added (the first
+// add of every position).  Points outside the grid hold the point they shadow.
+__global__ void __launch_bounds__(256) tile_delays_kernel(const float* __restrict__ delay, uint64_t npix, TileGeom tg,
+		uint32_t tile0, uint32_t npts, uint32_t nrx, uint32_t first_tx, uint32_t rows, float offset,
+		float* __restrict__ td)
+{
+	const uint32_t per = npts / 256;
+	const uint32_t tl = blockIdx.x / per, q = (blockIdx.x % per) * 256 + threadIdx.x;
+	uint32_t col, row;
+	bool valid;
+	tg.pixel(tile0 + tl, q, col, row, valid);
+	const float* src = delay + static_cast<uint64_t>(col) * tg.n2 + row;
+	float* dst = td + static_cast<uint64_t>(tl) * rows * npts + q;
+	for (uint32_t e = blockIdx.y; e < rows; e += gridDim.y) {
+		float d;
+		if (e < nrx) d = src[static_cast<uint64_t>(e) * npix];
+		else d = offset + src[static_cast<uint64_t>(first_tx + e - nrx) * npix];
+		dst[static_cast<uint64_t>(e) * npts] = d;
+	}
+}
+
+// (min, max) of every row of the tile delays: a wave per (tile, row).
+__global__ void __launch_bounds__(256) tile_bounds_kernel(const float* __restrict__ td, uint64_t nrows, uint32_t npts,
+		float2* __restrict__ bounds)
+{
+	const uint64_t i = static_cast<uint64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+	if (i >= nrows) return;
+	const uint32_t lane = threadIdx.x & 63;
+	const float* src = td + i * npts;
+	float mn = 3.4e38f, mx = -3.4e38f;
+	for (uint32_t k = lane; k < npts; k += 64) {
+		const float d = src[k];
+		mn = fminf(mn, d);
+		mx = fmaxf(mx, d);
+	}
+	for (int o = 32; o > 0; o >>= 1) {
+		mn = fminf(mn, __shfl_xor(mn, o, 64));
+		mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+	}
+	if (lane == 0) bounds[i] = make_float2(mn, mx);
+}
+
+// Window words of a tile ([rx groups][ntx][kRxGroup]) and the slots of
+// its longest window; max_slots takes the longest of all tiles.  A workgroup
+// per tile.
+__global__ void __launch_bounds__(256) window_params_kernel(const float2* __restrict__ bounds, uint32_t ntx,
+		uint32_t nrx, uint32_t nrx_pad, uint32_t L, uint32_t esz, uint32_t* __restrict__ words,
+		uint32_t* __restrict__ slots, uint32_t* __restrict__ max_slots)
+{
+	__shared__ uint32_t red[4];
 	const uint32_t tile = blockIdx.x;
-	const uint32_t npt = tg.tw1 * tg.tw2 * tg.tzh;
-	const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	uint64_t off[kMaxPts];
-#pragma unroll
-	for (uint32_t k = 0; k < kMaxPts; ++k) {
-		const uint32_t l = lane + 64 * k;
-		uint32_t col = 0, row = 0;
-		bool valid;
-		tg.pixel(tile, l < npt ? l : 0u, col, row, valid);
-		off[k] = static_cast<uint64_t>(col) * tg.n2 + row;
-	}
-	for (uint32_t e = wave; e < num_elements; e += 4) {
-		const float* de = delay + static_cast<uint64_t>(e) * npix;
-		float mn = 3.4e38f, mx = -3.4e38f;
-#pragma unroll
-		for (uint32_t k = 0; k < kMaxPts; ++k) {
-			if (lane + 64 * k < npt) {
-				const float d = de[off[k]];
-				mn = fminf(mn, d);
-				mx = fmaxf(mx, d);
-			}
-		}
-		for (int o = 32; o > 0; o >>= 1) {
-			mn = fminf(mn, __shfl_xor(mn, o, 64));
-			mx = fmaxf(mx, __shfl_xor(mx, o, 64));
-		}
-		if (lane == 0) bounds[static_cast<uint64_t>(tile) * num_elements + e] = make_float2(mn, mx);
-	}
-}
-
-__global__ void __launch_bounds__(256) window_params_kernel(const float2* __restrict__ bounds, uint32_t ntiles,
-		uint32_t num_elements, uint32_t first_tx, uint32_t ntx, uint32_t ntx_pad, uint32_t nrx, uint32_t L, float offset,
-		uint32_t esz, uint32_t* __restrict__ words, uint32_t* __restrict__ max_need)
-{
-	// Grid-stride over the entries (a capped grid): each lane folds the
-	// window lengths of many entries, then one atomic per wave.
-	const uint64_t n = static_cast<uint64_t>(ntiles) * nrx * ntx_pad;
-	uint32_t mneed = 0;   // every lane reaches the wave reduction below
-	for (uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;
-			i += static_cast<uint64_t>(gridDim.x) * blockDim.x) {
-		const uint32_t t = static_cast<uint32_t>(i % ntx_pad);
-		const uint32_t r = static_cast<uint32_t>((i / ntx_pad) % nrx);
-		const uint32_t tile = static_cast<uint32_t>(i / (static_cast<uint64_t>(ntx_pad) * nrx));
-		uint32_t word = kEdgeBit;   // padded transmit or nothing to stage: the channel's start, excluded
-		if (t < ntx) {
-			const float2 bt = bounds[static_cast<uint64_t>(tile) * num_elements + first_tx + t];
-			const float2 br = bounds[static_cast<uint64_t>(tile) * num_elements + r];
-			const float lo = (offset + bt.x) + br.x;
-			const float hi = (offset + bt.y) + br.y;
+	const float2* tb = bounds + static_cast<uint64_t>(tile) * (nrx + ntx);
+	const uint32_t n = nrx_pad * ntx;
+	uint32_t* out = words + static_cast<uint64_t>(tile) * n;
+	uint32_t mslots = 1;
+	for (uint32_t i = threadIdx.x; i < n; i += 256) {
+		const uint32_t t = i / kRxGroup % ntx, r = i / (kRxGroup * ntx) * kRxGroup + i % kRxGroup;
+		uint32_t word = kEdgeBit;   // padding or nothing to stage: excluded
+		if (r < nrx) {
+			const float2 bt = tb[nrx + t], br = tb[r];
+			const float lo = bt.x + br.x;
+			const float hi = bt.y + br.y;
 			// lo past the record end or NaN: nothing staged, every lane of
 			// the pair is excluded by the predicated path.  (lo is never
 			// negative: delays are >= 0 and the peak offset is >= 0.)
@@ -251,28 +298,27 @@ __global__ void __launch_bounds__(256) window_params_kernel(const float2* __rest
 				// entries [ws, floor(hi) + 1], never past index L (one past the record)
 				uint32_t need = (fhi >= static_cast<float>(L)) ? L + 1u - ws : static_cast<uint32_t>(fhi) + 2u - ws;
 				need = min(need, L + 1u - ws);
-				mneed = max(mneed, need);
+				const uint32_t k = (need * esz + 1023u) / 1024u;
+				mslots = max(mslots, k);
 				const bool edge = fhi + 1.0f >= static_cast<float>(L - 1u);
-				word = ws * esz | (edge ? kEdgeBit : 0u);
+				word = ws * esz | (min(k, 127u) << kSlotShift) | (edge ? kEdgeBit : 0u);
 			}
 		}
-		words[i] = word;
+		out[i] = word;
 	}
-	for (int o = 32; o > 0; o >>= 1) mneed = max(mneed, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mneed), o, 64)));
-	if ((threadIdx.x & 63) == 0 && mneed) atomicMax(max_need, mneed);
+	for (int o = 32; o > 0; o >>= 1)
+		mslots = max(mslots, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mslots), o, 64)));
+	if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mslots;
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		for (int w = 1; w < 4; ++w) mslots = max(mslots, red[w]);
+		slots[tile] = mslots;
+		atomicMax(max_slots, mslots);
+	}
 }
 
 }  // namespace
 
-// Builds (or reuses) the window tables for tile shape p0 and launches the
-// tiled kernel with the chunking p1.  p0: 0/1 = 16x16 (planes) or 8x8x4
-// (volumes), 2 = 8x32, 3 = 32x8, 4 = 8x8x4; 512-point tiles (512-lane
-// workgroups, 8 pairs per chunk): 5 = 16x32, 6 = 32x16, 7 = 8x8x8.  p1:
-// byte 0 pairs per chunk
-// (4 or 8), byte 1 chunk buffers, byte 2 LDS budget in KiB (default: the
-// smallest of 52 (three workgroups per CU: the kernel is compiled for three
-// waves per SIMD), 76 (two) and 150 (one) in which the windows fit).
-// Returns false when the tables do not fit the tiled kernel.
 namespace {
 
 __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
@@ -280,7 +326,7 @@ __global__ void zero_u32_kernel(uint32_t* p) { *p = 0u; }
 // Tile shape p0 (see launch_tiled) of a geometry.
 struct TilePlan {
 	TileGeom tg;
-	uint32_t ntiles = 0, nt = 0, nw = 0, esz = 0;
+	uint32_t ntiles = 0, npts = 0, esz = 0;
 	uint64_t key = 0;        // what the window tables depend on, besides grid and offset
 	bool ok = false;
 };
@@ -291,159 +337,216 @@ TilePlan tile_plan(const FrameGeom& g, int p0)
 	const uint32_t ny = g.ny ? g.ny : 1u;
 	uint32_t tw1 = 16, tw2 = 1, tzh = 16;
 	if (ny > 1) { tw1 = 8; tw2 = 8; tzh = 4; }
-	if (p0 == 2) { tw1 = 8; tw2 = 1; tzh = 32; }
-	else if (p0 == 3) { tw1 = 32; tw2 = 1; tzh = 8; }
-	else if (p0 == 4) { tw1 = 8; tw2 = 8; tzh = 4; }
-	else if (p0 == 5) { tw1 = 16; tw2 = 1; tzh = 32; }
-	else if (p0 == 6) { tw1 = 32; tw2 = 1; tzh = 16; }
-	else if (p0 == 7) { tw1 = 8; tw2 = 8; tzh = 8; }
-	tp.nt = tw1 * tw2 * tzh;
-	tp.nw = tp.nt / 64;
-	// More than 128 transmits: 512-lane tiles only.  A lane holds a block's
-	// 128 transmit delays in registers, which leaves a 256-lane tile (three
-	// waves per SIMD, 168 registers) spilling; 512-lane tiles have 256.
-	if (g.ntx_pad > 128 && tp.nt != 512) return tp;
+	switch (p0) {
+	case 2: tw1 = 8; tw2 = 1; tzh = 32; break;
+	case 3: tw1 = 32; tw2 = 1; tzh = 8; break;
+	case 4: tw1 = 8; tw2 = 8; tzh = 4; break;
+	case 5: tw1 = 16; tw2 = 1; tzh = 32; break;
+	case 6: tw1 = 32; tw2 = 1; tzh = 16; break;
+	case 7: tw1 = 8; tw2 = 8; tzh = 8; break;
+	case 8: tw1 = 32; tw2 = 1; tzh = 32; break;
+	case 9: tw1 = 64; tw2 = 1; tzh = 32; break;
+	case 10: tw1 = 16; tw2 = 8; tzh = 8; break;
+	case 11: tw1 = 16; tw2 = 16; tzh = 8; break;
+	default: break;
+	}
+	tp.npts = tw1 * tw2 * tzh;
+	// More than 128 transmits: 256-point tiles, which copy the most bytes per
+	// pixel and pair, are not offered.
+	if (g.ntx > 128 && tp.npts < 512) return tp;
+	if (g.L >= kMaxWindowL) return tp;
 	tp.esz = static_cast<uint32_t>(storage_bytes(g.storage));
 	const uint32_t nx = g.n1 / ny;
 	tp.tg = TileGeom{g.n1, g.n2, ny, nx, tw1, tw2, tzh, (nx + tw1 - 1) / tw1, (ny + tw2 - 1) / tw2, (g.n2 + tzh - 1) / tzh};
 	const uint64_t ntiles64 = static_cast<uint64_t>(tp.tg.tiles_x) * tp.tg.tiles_y * tp.tg.tiles_z;
-	if (ntiles64 >= (1ull << 31)) return tp;
+	if (ntiles64 * (pad_nrx(g.nrx) / kRxGroup) >= (1ull << 31)) return tp;
 	tp.ntiles = static_cast<uint32_t>(ntiles64);
-	tp.key = (static_cast<uint64_t>(tw1) << 56) ^ (static_cast<uint64_t>(tw2) << 52) ^
-			(static_cast<uint64_t>(tzh) << 44) ^ (static_cast<uint64_t>(ny) << 40) ^
-			(static_cast<uint64_t>(tp.esz) << 36) ^ (static_cast<uint64_t>(g.L) << 8) ^ g.first_tx ^
-			(static_cast<uint64_t>(g.ntx) << 20) ^ (static_cast<uint64_t>(g.ntx_pad) << 28);
+	tp.key = 0x9E3779B97F4A7C15ull;
+	for (uint64_t v : {static_cast<uint64_t>(p0), static_cast<uint64_t>(ny), static_cast<uint64_t>(tp.esz),
+				static_cast<uint64_t>(g.L), static_cast<uint64_t>(g.first_tx), static_cast<uint64_t>(g.ntx)})
+		tp.key = (tp.key ^ v) * 0x100000001B3ull;
 	tp.ok = true;
 	return tp;
 }
 
-size_t bounds_bytes(const FrameGeom& g, const TilePlan& tp)
+size_t bounds_bytes(const FrameGeom& g, const TilePlan& tp, uint32_t ntiles)
 {
-	return static_cast<size_t>(tp.ntiles) * g.num_elements * sizeof(float2);
+	return static_cast<size_t>(ntiles) * (g.nrx + g.ntx) * sizeof(float2);
 }
-size_t words_bytes(const FrameGeom& g, const TilePlan& tp)
+size_t words_bytes(const FrameGeom& g, const TilePlan& tp, uint32_t ntiles)
 {
-	return static_cast<size_t>(tp.ntiles) * g.nrx * g.ntx_pad * sizeof(uint32_t);
+	return static_cast<size_t>(ntiles) * pad_nrx(g.nrx) * g.ntx * sizeof(uint32_t);
+}
+size_t delays_bytes(const FrameGeom& g, const TilePlan& tp, uint32_t ntiles)
+{
+	return static_cast<size_t>(ntiles) * (g.nrx + g.ntx) * tp.npts * sizeof(float);
+}
+// Per-rx sums of one tile.
+size_t sums_bytes(const FrameGeom& g, const TilePlan& tp)
+{
+	return static_cast<size_t>(g.nrx) * tp.npts * sizeof(float2);
 }
 
-// Builds the per-tile delay bounds and the window words; returns the window
-// size in 1 KiB slots (reads back the longest window: synchronises s).
-uint32_t build_window_tables(const FrameGeom& g, const TilePlan& tp, const float* d_delay, float2* bounds,
-		uint32_t* words, uint32_t* d_max, hipStream_t s)
+// Delays, their bounds, window words and longest windows of the tiles
+// [tile0, tile0 + n) into the given buffers; max_slots keeps the longest.
+void build_window_tables(const FrameGeom& g, const TilePlan& tp, uint32_t tile0, uint32_t n, const float* d_delay,
+		float* td, float2* bounds, uint32_t* words, uint32_t* slots, uint32_t* max_slots, hipStream_t s)
 {
-	hipLaunchKernelGGL(tile_bounds_kernel, dim3(tp.ntiles), dim3(256), 0, s, d_delay, g.npix, g.num_elements, tp.tg,
+	const uint32_t rows = g.nrx + g.ntx;
+	const uint32_t nb = n * (tp.npts / 256);
+	hipLaunchKernelGGL(tile_delays_kernel, dim3(nb, std::max(1u, std::min(rows, 16384u / std::max(1u, nb)))), dim3(256), 0, s,
+			d_delay, g.npix, tp.tg, tile0, tp.npts, g.nrx, g.first_tx, rows, g.offset, td);
+	HIP_CHECK(hipGetLastError());
+	const uint64_t nrows = static_cast<uint64_t>(n) * rows;
+	hipLaunchKernelGGL(tile_bounds_kernel, dim3(static_cast<uint32_t>((nrows + 3) / 4)), dim3(256), 0, s, td, nrows, tp.npts,
 			bounds);
 	HIP_CHECK(hipGetLastError());
-	const uint64_t np = static_cast<uint64_t>(tp.ntiles) * g.nrx * g.ntx_pad;
-	hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, d_max);
+	hipLaunchKernelGGL(window_params_kernel, dim3(n), dim3(256), 0, s, bounds, g.ntx, g.nrx, pad_nrx(g.nrx), g.L, tp.esz, words,
+			slots, max_slots);
 	HIP_CHECK(hipGetLastError());
-	hipLaunchKernelGGL(window_params_kernel, dim3(static_cast<uint32_t>(std::min<uint64_t>((np + 255) / 256, 4096))),
-			dim3(256), 0, s, bounds, tp.ntiles, g.num_elements, g.first_tx, g.ntx, g.ntx_pad, g.nrx, g.L, g.offset,
-			tp.esz, words, d_max);
-	HIP_CHECK(hipGetLastError());
-	uint32_t max_need = 0;
-	HIP_CHECK(hipMemcpyAsync(&max_need, d_max, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-	HIP_CHECK(hipStreamSynchronize(s));
-	const uint32_t slot = 1024u / tp.esz;   // entries per 1 KiB load slot
-	return std::max(1u, (max_need + slot - 1) / slot);
 }
 
-// Chunking and launch of the tiled kernel over window tables with S slots.
-// p1: byte 0 pairs per chunk (4 or 8), byte 1 chunk buffers, byte 2 LDS
-// budget in KiB (default: the smallest of 52 (three workgroups per CU: the
-// kernel is compiled for three waves per SIMD), 76 (two) and 150 (one) in
-// which the windows fit).  Returns false when nothing fits.
-bool choose_chunking(const FrameGeom& g, uint32_t nt, int p1, uint32_t S, uint32_t& tc, uint32_t& nbuf)
+uint32_t read_u32(const uint32_t* d, hipStream_t s)
 {
-	tc = 0;
-	nbuf = 0;
-	if (S > kMaxSlots) return false;
-	const uint32_t nw = nt / 64;
-	// Pairs per chunk (tc) and chunk buffers in the LDS ring (nbuf): the most
-	// pairs in flight, (nbuf - 1) * tc, that fit the budget and the 6-bit
-	// vmcnt of the per-chunk waits.
-	const uint32_t want_tc = static_cast<uint32_t>(p1) & 0xFF, want_nb = (static_cast<uint32_t>(p1) >> 8) & 0xFF;
-	const uint32_t want_kb = (static_cast<uint32_t>(p1) >> 16) & 0xFF;
-	for (uint32_t kb : {52u, 76u, 150u}) {
-		if (want_kb && kb != 52u) break;
-		const size_t budget = static_cast<size_t>(want_kb ? std::min(want_kb, 158u) : kb) * 1024 -
-				tile_stats_bytes(g.cf_kind, nt);
-		auto fit = [&](uint32_t c) -> uint32_t {
-			if (c % nw != 0) return 0u;   // every wave copies whole windows
-			const size_t bb = tile_buffer_bytes(c, S, nt);
-			uint32_t nb = static_cast<uint32_t>(std::min<size_t>(16, budget / bb));
-			if (want_nb) nb = std::min(nb, want_nb);
-			const uint32_t per = c / nw * S + 1;   // copies per wave per chunk, at most
-			while (nb > 2 && (nb - 2) * per > 63) --nb;
-			return (nb >= 2 && 2 * per <= 63) ? nb : 0u;
-		};
-		for (uint32_t c : {16u, 8u, 4u}) {
-			if (want_tc && c != want_tc) continue;
-			if (c == 16 && (nt != 512 || want_tc != 16 || g.ntx_pad != 128)) continue;   // 16 pairs: asked for, 512-lane tiles, 128-transmit blocks
-			if (nt == 512 && c == 4) continue;
-			const uint32_t nb = fit(c);
-			if (nb && (nb - 1) * c > (nbuf ? (nbuf - 1) * tc : 0u)) { tc = c; nbuf = nb; }
-		}
-		if (nbuf) break;
-	}
-	return nbuf != 0;
+	uint32_t v = 0;
+	HIP_CHECK(hipMemcpyAsync(&v, d, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+	HIP_CHECK(hipStreamSynchronize(s));
+	return v;
 }
 
-TileArgs tile_args(const FrameGeom& g, const TilePlan& tp, const DasArgs& a, const uint32_t* words, uint32_t S,
-		uint32_t nbuf)
+// How a tile's sums are formed (das_tile's template parameters).
+struct Chunking {
+	uint32_t r = 0;       // receive elements per workgroup: pairs per transmit step
+	uint32_t nt = 0;      // lanes
+	uint32_t nbmax = 0;   // most chunk buffers
+	uint32_t lds = 0;     // LDS bytes
+	uint32_t nbuf = 0;    // chunk buffers of the tile with the longest window
+	int p1(int asked) const { return static_cast<int>(r | (nbuf << 8)) | (asked & 0xFF0000); }
+};
+
+// Chunking of the tiled kernel over windows of at most S slots.  p1: byte 0
+// pairs per transmit step (4, 8, or 16 on 512-point tiles), byte 1 most chunk
+// buffers, byte 2 LDS budget in KiB (default: the smallest in which two
+// buffers of the longest window fit, of those that put 4, 3, 2 or 1
+// workgroups on a CU).  Returns false when nothing fits.
+bool choose_chunking(uint32_t npts, int p1, uint32_t S, Chunking& c)
+{
+	if (S > kMaxSlots) return false;
+	const uint32_t want_r = static_cast<uint32_t>(p1) & 0xFF, want_nb = (static_cast<uint32_t>(p1) >> 8) & 0xFF;
+	const uint32_t want_kb = (static_cast<uint32_t>(p1) >> 16) & 0xFF;
+	c.nbmax = want_nb ? std::max(2u, std::min(want_nb, 4u)) : 4u;
+	for (uint32_t kb : {40u, 53u, 80u, 160u}) {
+		if (want_kb) {
+			if (kb != 40u) break;
+			kb = std::min(want_kb, 160u);
+		}
+		// lanes per workgroup; no more workgroups than the CU's registers hold
+		c.nt = npts <= 512 ? 256u : npts == 1024 ? 512u : kb <= 80u ? 512u : 1024u;
+		if (!want_kb && c.nt == 512u && kb < 80u) continue;
+		c.lds = kb * 1024u;
+		for (uint32_t r : {4u, 8u, 16u}) {
+			if (want_r ? r != want_r : r == 16u) continue;
+			if ((r == 16u && npts != 512u) || (r == 8u && (npts == 256u || (npts == 2048u && c.nt == 512u)))) continue;
+			const uint32_t rc = npts == 2048u && c.nt == 512u ? 2u : 4u;
+			c.r = r;
+			if (r == 16u) c.nt = 512u;
+			c.nbuf = tile_buffers(c.nbmax, c.lds, S, rc, r / rc, npts);
+			if (c.nbuf) return true;
+		}
+	}
+	return false;
+}
+
+TileArgs tile_args(const FrameGeom& g, const DasArgs& a, uint32_t ntiles, const Chunking& c)
 {
 	TileArgs A;
-	A.d = a;
-	A.tg = tp.tg;
-	A.words = words;
-	A.S = S;
-	A.ntx_pad = g.ntx_pad;
-	A.nbuf = nbuf;
+	A.tensor = a.tensor;
+	A.td = nullptr;
+	A.words = nullptr;
+	A.slots = nullptr;
+	A.w = a.w;
+	A.partial = a.partial;
+	A.ntx = g.ntx;
+	A.nrx = g.nrx;
+	A.L = g.L;
+	A.ntiles = ntiles;
+	A.ngrp = (g.nrx + c.r - 1) / c.r;
+	A.ngrp4 = pad_nrx(g.nrx) / kRxGroup;
+	A.lds = c.lds;
+	A.nbmax = c.nbmax;
 	return A;
 }
 
 // Launches the tiled kernel of the batch's storage.
-void launch_batch(int storage, int cf, const TileBatch& B, uint32_t nt, uint32_t tc, hipStream_t s)
+void launch_batch(int storage, const TileBatch& B, uint32_t npts, const Chunking& c, hipStream_t s)
 {
 	switch (storage) {
-	case MISTA_STORAGE_F32: launch_tile_storage<MISTA_STORAGE_F32>(cf, B, nt, tc, s); break;
-	case MISTA_STORAGE_F16: launch_tile_storage<MISTA_STORAGE_F16>(cf, B, nt, tc, s); break;
-	case kStorageReal: launch_tile_storage<kStorageReal>(cf, B, nt, tc, s); break;
-	default: launch_tile_storage<MISTA_STORAGE_BF16>(cf, B, nt, tc, s); break;
+	case MISTA_STORAGE_F32: launch_tile_storage<MISTA_STORAGE_F32>(B, npts, c.r, c.nt, s); break;
+	case MISTA_STORAGE_F16: launch_tile_storage<MISTA_STORAGE_F16>(B, npts, c.r, c.nt, s); break;
+	case kStorageReal: launch_tile_storage<kStorageReal>(B, npts, c.r, c.nt, s); break;
+	default: launch_tile_storage<MISTA_STORAGE_BF16>(B, npts, c.r, c.nt, s); break;
 	}
 	HIP_CHECK(hipGetLastError());
 }
 
-// One frame's tiled launch over window tables with S slots.  Returns false
-// when nothing fits.
-bool launch_tiles(const FrameGeom& g, const TilePlan& tp, int p0, int p1, uint32_t S, const uint32_t* words,
-		const DasArgs& a, DasScratch& scratch, hipStream_t s)
+// The statistics of the tiles [tile0, tile0 + n), whose sums start at a.partial.
+void launch_tile_stats(const FrameGeom& g, const TilePlan& tp, const DasArgs& a, uint32_t tile0, uint32_t n, hipStream_t s)
 {
-	uint32_t tc = 0, nbuf = 0;
-	if (!choose_chunking(g, tp.nt, p1, S, tc, nbuf)) return false;
-	TileBatch B{};
-	B.jobs[0] = tile_args(g, tp, a, words, S, nbuf);
-	B.first[0] = 0;
-	B.first[1] = tp.ntiles;
-	B.njobs = 1;
-	B.total = tp.ntiles;
-	scratch.last_p0 = p0 == 0 ? (tp.tg.ny > 1 ? 4 : 1) : p0;
-	scratch.last_p1 = static_cast<int>(tc | (nbuf << 8) | (((static_cast<uint32_t>(p1) >> 16) & 0xFF) << 16));
-	launch_batch(g.storage, g.cf_kind, B, tp.nt, tc, s);
-	return true;
+	const dim3 grid(n * (tp.npts / 256));
+	switch (g.cf_kind) {
+	case MISTA_CF_NONE:
+		hipLaunchKernelGGL(das_tile_stats_kernel<MISTA_CF_NONE>, grid, dim3(256), 0, s, a, tp.tg, tile0, tp.npts);
+		break;
+	case MISTA_CF_PCF:
+		hipLaunchKernelGGL(das_tile_stats_kernel<MISTA_CF_PCF>, grid, dim3(256), 0, s, a, tp.tg, tile0, tp.npts);
+		break;
+	default:
+		hipLaunchKernelGGL(das_tile_stats_kernel<MISTA_CF_SCF>, grid, dim3(256), 0, s, a, tp.tg, tile0, tp.npts);
+		break;
+	}
+	HIP_CHECK(hipGetLastError());
 }
 
-// Window tables of tile shape p0 in the handle's scratch (built when the
-// grid, shape or offset changed: synchronises s); false when the shape does
-// not apply.
+// Most bytes of per-rx sums held at a time: a frame whose sums need more runs
+// its tiles in several launches.
+constexpr size_t kSumsBytes = static_cast<size_t>(1) << 30;
+
+uint32_t slab_tiles(const FrameGeom& g, const TilePlan& tp)
+{
+	return static_cast<uint32_t>(std::max<size_t>(1, std::min<size_t>(tp.ntiles, kSumsBytes / sums_bytes(g, tp))));
+}
+
+// The tiles [tile0, tile0 + n) of a frame: per-rx sums, then statistics.
+void run_tiles(const FrameGeom& g, const TilePlan& tp, const TileArgs& first, const DasArgs& a, uint32_t tile0, uint32_t n,
+		const Chunking& c, hipStream_t s)
+{
+	TileBatch B{};
+	B.jobs[0] = first;
+	B.njobs = 1;
+	B.total = B.first[1] = n * first.ngrp;
+	launch_batch(g.storage, B, tp.npts, c, s);
+	launch_tile_stats(g, tp, a, tile0, n, s);
+}
+
+// The shape that is reported for p0 (0: the default).
+int reported_shape(const TilePlan& tp, int p0) { return p0 == 0 ? (tp.tg.ny > 1 ? 4 : 1) : p0; }
+
+// Tables of tile shape p0 in the handle's scratch (built when the grid, shape
+// or offset changed: synchronises s); false when the shape does not apply.
 bool ensure_tables(const FrameGeom& g, const TilePlan& tp, DasScratch& scratch, const float* d_delay, hipStream_t s)
 {
 	if (!tp.ok) return false;
 	if (scratch.bounds_version != g.grid_version || scratch.params_key != tp.key || scratch.params_offset != g.offset) {
-		float2* b = static_cast<float2*>(scratch.bounds.reserve(bounds_bytes(g, tp)));
-		uint32_t* words = static_cast<uint32_t*>(scratch.params.reserve(words_bytes(g, tp)));
+		float* td = static_cast<float*>(scratch.delays.reserve(delays_bytes(g, tp, tp.ntiles)));
+		float2* b = static_cast<float2*>(scratch.bounds.reserve(bounds_bytes(g, tp, tp.ntiles)));
+		uint32_t* words = static_cast<uint32_t*>(scratch.params.reserve(words_bytes(g, tp, tp.ntiles)));
+		uint32_t* slots = static_cast<uint32_t*>(scratch.slots.reserve(static_cast<size_t>(tp.ntiles) * sizeof(uint32_t)));
 		uint32_t* d_max = static_cast<uint32_t*>(scratch.partial.reserve(256));
-		scratch.max_slots = build_window_tables(g, tp, d_delay, b, words, d_max, s);
+		scratch.bounds_version = ~0ull;   // nothing half-built is kept
+		hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, d_max);
+		HIP_CHECK(hipGetLastError());
+		build_window_tables(g, tp, 0, tp.ntiles, d_delay, td, b, words, slots, d_max, s);
+		scratch.max_slots = read_u32(d_max, s);
 		scratch.bounds_version = g.grid_version;
 		scratch.params_key = tp.key;
 		scratch.params_offset = g.offset;
@@ -453,38 +556,40 @@ bool ensure_tables(const FrameGeom& g, const TilePlan& tp, DasScratch& scratch, 
 
 }  // namespace
 
-// Builds (or reuses) the window tables for tile shape p0 and launches the
-// tiled kernel with the chunking p1.  p0: 0/1 = 16x16 (planes) or 8x8x4
-// (volumes), 2 = 8x32, 3 = 32x8, 4 = 8x8x4; 512-point tiles (512-lane
-// workgroups, 8 pairs per chunk): 5 = 16x32, 6 = 32x16, 7 = 8x8x8.  p1: see
-// launch_tiles.  Returns false when the tables do not fit the tiled kernel.
-bool launch_tiled(const FrameGeom& g, int p0, int p1, DasScratch& scratch, const DasArgs& a, const float* d_delay,
+// Builds (or reuses) the tables for tile shape p0 and runs the tiled kernel
+// with the chunking p1 (see choose_chunking).  p0: 0/1 = 16x16 (planes) or
+// 8x8x4 (volumes), 2 = 8x32, 3 = 32x8, 4 = 8x8x4; 512 points: 5 = 16x32,
+// 6 = 32x16, 7 = 8x8x8; 1024 points: 8 = 32x32, 10 = 16x8x8; 2048 points:
+// 9 = 64x32, 11 = 16x16x8.  Returns false when the windows do not fit.
+bool launch_tiled(const FrameGeom& g, int p0, int p1, DasScratch& scratch, const DasArgs& args, const float* d_delay,
 		hipStream_t s)
 {
 	const TilePlan tp = tile_plan(g, p0);
 	if (!ensure_tables(g, tp, scratch, d_delay, s)) return false;
-	return launch_tiles(g, tp, p0, p1, scratch.max_slots, scratch.params.as<const uint32_t>(), a, scratch, s);
-}
-
-// Bytes of the per-rx partial sums a frame with several transmit blocks
-// keeps between blocks (tiled kernel), 0 with one block.
-size_t partial_bytes(const FrameGeom& g)
-{
-	return g.ntx_pad > 128 ? static_cast<size_t>(g.nrx) * g.npix * sizeof(float2) : 0;
-}
-
-float2* scratch_partial(const FrameGeom& g, DasScratch& scratch)
-{
-	const size_t b = partial_bytes(g);
-	return b ? static_cast<float2*>(scratch.partials.reserve(b)) : nullptr;
+	Chunking c;
+	if (!choose_chunking(tp.npts, p1, scratch.max_slots, c)) return false;
+	const uint32_t slab = slab_tiles(g, tp);
+	DasArgs a = args;
+	a.partial = static_cast<float2*>(scratch.partials.reserve(slab * sums_bytes(g, tp)));
+	for (uint32_t t0 = 0; t0 < tp.ntiles; t0 += slab) {
+		const uint32_t n = std::min(slab, tp.ntiles - t0);
+		TileArgs A = tile_args(g, a, n, c);
+		A.td = scratch.delays.as<const float>() + delays_bytes(g, tp, t0) / sizeof(float);
+		A.words = scratch.params.as<const uint32_t>() + words_bytes(g, tp, t0) / sizeof(uint32_t);
+		A.slots = scratch.slots.as<const uint32_t>() + t0;
+		run_tiles(g, tp, A, a, t0, n, c, s);
+	}
+	scratch.last_p0 = reported_shape(tp, p0);
+	scratch.last_p1 = c.p1(p1);
+	return true;
 }
 
 // Kernel arguments of a frame.
 DasArgs das_args(const FrameGeom& g, const void* d_tensor, const float* d_delay, const float* d_w, float* d_value,
-		float* d_factor, float2* d_partial)
+		float* d_factor)
 {
 	DasArgs a;
-	a.partial = d_partial;
+	a.partial = nullptr;
 	a.tensor = d_tensor;
 	a.delay = d_delay;
 	a.w = d_w;
@@ -495,7 +600,6 @@ DasArgs das_args(const FrameGeom& g, const void* d_tensor, const float* d_delay,
 	a.ntx = g.ntx;
 	a.nrx = g.nrx;
 	a.L = g.L;
-	a.w_stride = g.ntx_pad;
 	a.offset = g.offset;
 	if (g.cf_kind == MISTA_CF_PCF) {
 		// CoherenceFactor.h:243-246: sigma0 = pi/sqrt(3) (stored as float),
@@ -512,13 +616,12 @@ DasArgs das_args(const FrameGeom& g, const void* d_tensor, const float* d_delay,
 
 // ---------------------------------------------------------------- no allocation
 
-// Device scratch of the no-allocation DAS: the per-tile delay bounds, the
-// window words and the longest-window counter of one launch, and, for more
-// than 128 transmits, the per-rx partial sums.  Every call on
-// a GPU shares that GPU's copy (each GPU the library runs on holds one until
-// the process ends) and rebuilds what it needs: calls that overlap on one GPU
-// race.  In host code `scratch` names a host-side stand-in; kernels get the
-// device address from hipGetSymbolAddress.
+// Device scratch of the no-allocation DAS: the tile delays, window tables and
+// per-rx sums of as many tiles as fit.  Every call on a GPU shares that GPU's
+// copy (each GPU the library runs on holds one until the process ends) and
+// rebuilds what it needs: calls that overlap on one GPU race.  In host code
+// `scratch` names a host-side stand-in; kernels get the device address from
+// hipGetSymbolAddress.
 static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
 
 namespace {
@@ -541,36 +644,89 @@ static unsigned char* noalloc_scratch()
 	return static_cast<unsigned char*>(ptr);
 }
 
+// Bytes of the window tables that decide whether the entry point takes a
+// geometry (its documented limit): transmits padded to 32, 64, 128 or equal
+// blocks of whole 8-pair chunks, and the sums between those blocks.
+static size_t noalloc_table_bytes(const FrameGeom& g, const TilePlan& tp)
+{
+	const size_t pad = budget_pad_ntx(g.ntx);
+	auto up = [](size_t b) { return (b + 255) / 256 * 256; };
+	return up(pad > 128 ? static_cast<size_t>(g.nrx) * g.npix * sizeof(float2) : 0) +
+			up(static_cast<size_t>(tp.ntiles) * g.num_elements * sizeof(float2)) +
+			up(static_cast<size_t>(tp.ntiles) * g.nrx * pad * sizeof(uint32_t)) + 256;
+}
+
 void launch_das_noalloc(const FrameGeom& g, int tuned_p0, int tuned_p1, DasScratch& last, const void* d_tensor,
 		const float* d_delay, const float* d_w, float* d_value, float* d_factor, hipStream_t s)
 {
-	if (!((g.ntx_pad <= 128 || g.ntx_pad % 8 == 0) && static_cast<uint64_t>(g.L) * storage_bytes(g.storage) < (1ull << 31)))
-		MISTA_THROW(MISTA_E_INVALID_PARAM, "This geometry has no tiled DAS form, which the no-allocation entry point needs.");
 	unsigned char* base = noalloc_scratch();
-	const size_t pb = (partial_bytes(g) + 255) / 256 * 256;   // per-rx sums between transmit blocks
-	DasArgs a = das_args(g, d_tensor, d_delay, d_w, d_value, d_factor, pb ? reinterpret_cast<float2*>(base) : nullptr);
+	DasArgs a = das_args(g, d_tensor, d_delay, d_w, d_value, d_factor);
 	// the tuned tile shape when it fits, else the default, else the larger tiles
 	std::vector<std::pair<int, int>> shapes;
 	if (tuned_p0 >= 0) shapes.emplace_back(tuned_p0, tuned_p1);
-	for (int p0 : (g.ny > 1 ? std::vector<int>{4, 7} : std::vector<int>{1, 5, 6})) shapes.emplace_back(p0, 0);
+	const std::vector<int> defaults = g.ny > 1 ? std::vector<int>{4, 7} : std::vector<int>{1, 5, 6};
+	for (int p0 : defaults) shapes.emplace_back(p0, 0);
 	size_t need_min = ~size_t(0);
+	for (int p0 : defaults) {
+		FrameGeom gl = g;
+		gl.L = std::min(g.L, kMaxWindowL - 1);   // (the shape alone, whatever the record)
+		const TilePlan tp = tile_plan(gl, p0);
+		if (tp.ok) need_min = std::min(need_min, noalloc_table_bytes(g, tp));
+	}
+	if (need_min != ~size_t(0) && need_min > kNoAllocTableBytes)
+		MISTA_THROW(MISTA_E_INVALID_PARAM, "The DAS window tables of this geometry need " << need_min
+				<< " bytes; the no-allocation entry point holds at most " << kNoAllocTableBytes << '.');
+	bool too_large = g.L >= kMaxWindowL;   // no tile of the frame fits the scratch (or the record the window words)
 	for (const auto& sh : shapes) {
 		const TilePlan tp = tile_plan(g, sh.first);
 		if (!tp.ok) continue;
-		const size_t bb = (bounds_bytes(g, tp) + 255) / 256 * 256, wb = (words_bytes(g, tp) + 255) / 256 * 256;
-		const size_t need = pb + bb + wb + 256;
-		need_min = std::min(need_min, need);
-		if (need > kNoAllocScratchBytes) continue;
-		float2* bounds = reinterpret_cast<float2*>(base + pb);
-		uint32_t* words = reinterpret_cast<uint32_t*>(base + pb + bb);
-		uint32_t* d_max = reinterpret_cast<uint32_t*>(base + pb + bb + wb);
-		const uint32_t S = build_window_tables(g, tp, d_delay, bounds, words, d_max, s);
-		if (launch_tiles(g, tp, sh.first, sh.second, S, words, a, last, s)) return;
+		// the scratch: longest window, then the tables and sums of `slab` tiles
+		size_t off[6] = {256, 0, 0, 0, 0, 0};
+		auto layout = [&](uint32_t n) {
+			const size_t bytes[5] = {delays_bytes(g, tp, n), bounds_bytes(g, tp, n), words_bytes(g, tp, n),
+					static_cast<size_t>(n) * sizeof(uint32_t), n * sums_bytes(g, tp)};
+			for (int k = 0; k < 5; ++k) off[k + 1] = off[k] + (bytes[k] + 255) / 256 * 256;
+			return off[5] <= kNoAllocScratchBytes;
+		};
+		if (!layout(1)) {
+			too_large = true;
+			continue;
+		}
+		const size_t per = off[5] - 256;   // an upper bound per tile
+		const uint32_t slab = static_cast<uint32_t>(std::min<size_t>(tp.ntiles, (kNoAllocScratchBytes - 256) / per));
+		if (!layout(slab)) MISTA_THROW(MISTA_E_INVALID_STATE, "no-allocation DAS scratch layout");
+		uint32_t* d_max = reinterpret_cast<uint32_t*>(base);
+		float* td = reinterpret_cast<float*>(base + off[0]);
+		uint32_t* words = reinterpret_cast<uint32_t*>(base + off[2]);
+		uint32_t* slots = reinterpret_cast<uint32_t*>(base + off[3]);
+		a.partial = reinterpret_cast<float2*>(base + off[4]);
+		auto build = [&](uint32_t t0, uint32_t n) {
+			build_window_tables(g, tp, t0, n, d_delay, td, reinterpret_cast<float2*>(base + off[1]), words, slots, d_max, s);
+		};
+		hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, d_max);
+		HIP_CHECK(hipGetLastError());
+		for (uint32_t t0 = 0; t0 < tp.ntiles; t0 += slab) build(t0, std::min(slab, tp.ntiles - t0));
+		Chunking c;
+		if (!choose_chunking(tp.npts, sh.second, read_u32(d_max, s), c)) continue;
+		for (uint32_t t0 = 0; t0 < tp.ntiles; t0 += slab) {
+			const uint32_t n = std::min(slab, tp.ntiles - t0);
+			if (slab < tp.ntiles) build(t0, n);
+			TileArgs A = tile_args(g, a, n, c);
+			A.td = td;
+			A.words = words;
+			A.slots = slots;
+			run_tiles(g, tp, A, a, t0, n, c, s);
+		}
+		last.last_p0 = reported_shape(tp, sh.first);
+		last.last_p1 = c.p1(sh.second);
+		return;
 	}
-	if (need_min != ~size_t(0) && need_min > kNoAllocScratchBytes)
-		MISTA_THROW(MISTA_E_INVALID_PARAM, "The DAS window tables of this geometry need " << need_min
-				<< " bytes; the no-allocation entry point holds at most " << kNoAllocScratchBytes << '.');
-	MISTA_THROW(MISTA_E_INVALID_PARAM, "The signal windows of this geometry do not fit the tiled DAS kernel.");
+	if (!too_large)
+		MISTA_THROW(MISTA_E_INVALID_PARAM, "The signal windows of this geometry do not fit the tiled DAS kernel.");
+	// a tile's tables alone pass the scratch: one pixel per lane, which needs none
+	launch_gather_any<true>(g, a, s);
+	last.last_p0 = -1;
+	last.last_p1 = 0;
 }
 
 // ---------------------------------------------------------------- batches
@@ -589,24 +745,21 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 		const DasBatchItem& it = items[i];
 		const FrameGeom& g = *it.g;
 		int p0 = -1, p1 = 0;
-		const bool can_tile = it.t->variant != 1 && (g.ntx_pad <= 128 || g.ntx_pad % 8 == 0) &&
-				static_cast<uint64_t>(g.L) * storage_bytes(g.storage) < (1ull << 31);
-		if (can_tile && (it.t->variant == 2 || it.t->p0 || it.t->p1)) {
+		if (it.t->variant != 1 && (it.t->variant == 2 || it.t->p0 || it.t->p1)) {
 			p0 = it.t->p0;
 			p1 = it.t->p1;
-		} else if (can_tile && it.scratch->tuned_p0 >= 0) {
+		} else if (it.t->variant != 1 && it.scratch->tuned_p0 >= 0) {
 			p0 = it.scratch->tuned_p0;
 			p1 = it.scratch->tuned_p1;
 		}
 		TilePlan tp;
 		if (p0 >= 0) tp = tile_plan(g, p0);
-		if (p0 < 0 || !ensure_tables(g, tp, *it.scratch, it.delay, s) || it.scratch->max_slots > kMaxSlots) {
-			alone.push_back(i);   // untuned geometry (it tunes alone), gather kernel, or no tiled form
+		if (p0 < 0 || !ensure_tables(g, tp, *it.scratch, it.delay, s) || it.scratch->max_slots > kMaxSlots ||
+				slab_tiles(g, tp) < tp.ntiles) {
+			alone.push_back(i);   // untuned geometry (it tunes alone), gather kernel, no tiled form, or more than one slab of sums
 			continue;
 		}
-		const uint32_t ncls = g.ntx_pad > 128 ? 256u : g.ntx_pad;   // transmit block instantiation
-		const uint64_t cls = static_cast<uint64_t>(g.storage) | (static_cast<uint64_t>(g.cf_kind) << 8) |
-				(static_cast<uint64_t>(ncls) << 16) | (static_cast<uint64_t>(tp.nt) << 32);
+		const uint64_t cls = static_cast<uint64_t>(g.storage) | (static_cast<uint64_t>(tp.npts) << 32);
 		ready.push_back({i, tp, p0, p1, cls});
 	}
 	uint32_t shared = 0;
@@ -615,8 +768,13 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 		if (done[a0]) continue;
 		// the next group: frames of a0's class, in order, at most kMaxBatch
 		std::vector<size_t> grp;
-		for (size_t b = a0; b < ready.size() && grp.size() < kMaxBatch; ++b)
-			if (!done[b] && ready[b].cls == ready[a0].cls) grp.push_back(b);
+		uint64_t total = 0;
+		for (size_t b = a0; b < ready.size() && grp.size() < kMaxBatch; ++b) {
+			const uint64_t n = static_cast<uint64_t>(ready[b].tp.ntiles) * (pad_nrx(items[ready[b].i].g->nrx) / kRxGroup);
+			if (done[b] || ready[b].cls != ready[a0].cls || total + n >= (1ull << 31)) continue;
+			grp.push_back(b);
+			total += n;
+		}
 		uint32_t S = 0;
 		bool same_p1 = true;
 		for (size_t b : grp) {
@@ -624,10 +782,10 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 			same_p1 = same_p1 && ready[b].p1 == ready[grp[0]].p1;
 		}
 		const FrameGeom& g0 = *items[ready[grp[0]].i].g;
-		uint32_t tc = 0, nbuf = 0;
-		const uint32_t nt = ready[grp[0]].tp.nt;
-		bool fits = choose_chunking(g0, nt, same_p1 ? ready[grp[0]].p1 : 0, S, tc, nbuf);
-		if (!fits) fits = choose_chunking(g0, nt, 0, S, tc, nbuf);
+		Chunking c;
+		const uint32_t npts = ready[grp[0]].tp.npts;
+		bool fits = choose_chunking(npts, same_p1 ? ready[grp[0]].p1 : 0, S, c);
+		if (!fits) fits = choose_chunking(npts, 0, S, c);
 		for (size_t b : grp) done[b] = true;
 		if (!fits || grp.size() == 1) {
 			for (size_t b : grp) alone.push_back(ready[b].i);
@@ -635,21 +793,31 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 		}
 		TileBatch B{};
 		B.njobs = static_cast<uint32_t>(grp.size());
-		uint32_t total = 0;
+		uint32_t first = 0;
+		std::vector<DasArgs> args;
 		for (uint32_t k = 0; k < B.njobs; ++k) {
 			const Ready& r = ready[grp[k]];
 			const DasBatchItem& it = items[r.i];
-			const DasArgs a = das_args(*it.g, it.tensor, it.delay, it.w, it.value, it.factor,
-					scratch_partial(*it.g, *it.scratch));
-			B.jobs[k] = tile_args(*it.g, r.tp, a, it.scratch->params.as<const uint32_t>(), S, nbuf);
-			B.first[k] = total;
-			total += r.tp.ntiles;
-			it.scratch->last_p0 = r.p0 == 0 ? (r.tp.tg.ny > 1 ? 4 : 1) : r.p0;
-			it.scratch->last_p1 = static_cast<int>(tc | (nbuf << 8));
+			DasArgs a = das_args(*it.g, it.tensor, it.delay, it.w, it.value, it.factor);
+			a.partial = static_cast<float2*>(it.scratch->partials.reserve(r.tp.ntiles * sums_bytes(*it.g, r.tp)));
+			TileArgs& A = B.jobs[k];
+			A = tile_args(*it.g, a, r.tp.ntiles, c);
+			A.td = it.scratch->delays.as<const float>();
+			A.words = it.scratch->params.as<const uint32_t>();
+			A.slots = it.scratch->slots.as<const uint32_t>();
+			B.first[k] = first;
+			first += r.tp.ntiles * A.ngrp;
+			args.push_back(a);
+			it.scratch->last_p0 = reported_shape(r.tp, r.p0);
+			it.scratch->last_p1 = c.p1(0);
 		}
-		B.first[B.njobs] = total;
-		B.total = total;
-		launch_batch(g0.storage, g0.cf_kind, B, nt, tc, s);
+		B.first[B.njobs] = first;
+		B.total = first;
+		launch_batch(g0.storage, B, npts, c, s);
+		for (uint32_t k = 0; k < B.njobs; ++k) {
+			const Ready& r = ready[grp[k]];
+			launch_tile_stats(*items[r.i].g, r.tp, args[k], 0, r.tp.ntiles, s);
+		}
 		++shared;
 	}
 	for (size_t i : alone) {
@@ -667,11 +835,9 @@ size_t tensor_tail_padding() { return static_cast<size_t>(kMaxSlots) * 1024; }
 void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, const void* d_tensor,
 		const float* d_delay, const float* d_w, float* d_value, float* d_factor, hipStream_t s)
 {
-	const DasArgs a = das_args(g, d_tensor, d_delay, d_w, d_value, d_factor, scratch_partial(g, scratch));
+	const DasArgs a = das_args(g, d_tensor, d_delay, d_w, d_value, d_factor);
 
-	// window words hold ws * ESZ in 31 bits (L <= 2^20 samples)
-	const bool can_tile = (t.variant != 1) && (g.ntx_pad <= 128 || g.ntx_pad % 8 == 0) &&
-			static_cast<uint64_t>(g.L) * storage_bytes(g.storage) < (1ull << 31);
+	const bool can_tile = t.variant != 1 && g.L < kMaxWindowL;
 	if (can_tile) {
 		if (t.variant == 2 || t.p0 || t.p1) {
 			if (launch_tiled(g, t.p0, t.p1, scratch, a, d_delay, s)) return;
@@ -685,7 +851,23 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 					(static_cast<uint64_t>(g.nrx) << 50) ^ (static_cast<uint64_t>(g.storage) << 60) ^
 					(static_cast<uint64_t>(g.cf_kind) << 62) ^ static_cast<uint64_t>(g.offset * 1024.0f);
 			if (scratch.tuned_key != key) {
-				const std::vector<int> shapes = g.ny > 1 ? std::vector<int>{7, 4} : std::vector<int>{1, 2, 3, 5, 6};
+				// The larger tiles copy fewer bytes per pixel and pair (64x32
+				// points: 0.67 window entries per point and pair against 1.63
+				// at 16x32, 128-element frame; DAS 5.8 ms at 64x32, 8.3 at
+				// 32x32, 9.1 at 32x16).  The large ones go first, where they
+				// give every CU several workgroups; smaller planes are tried
+				// only where no large one fits, 256-point tiles only where
+				// nothing larger than 512 points won.
+				auto work = [&](int p0) {
+					const TilePlan tp = tile_plan(g, p0);
+					return static_cast<uint64_t>(tp.ntiles) * (pad_nrx(g.nrx) / kRxGroup);
+				};
+				std::vector<int> shapes;
+				const std::vector<int> large = g.ny > 1 ? std::vector<int>{11, 10} : std::vector<int>{9, 8};
+				for (int p0 : large)
+					if (tile_plan(g, p0).ok && work(p0) >= 1024u) shapes.push_back(p0);
+				for (int p0 : (g.ny > 1 ? std::vector<int>{7} : std::vector<int>{6, 5})) shapes.push_back(p0);
+				for (int p0 : (g.ny > 1 ? std::vector<int>{4} : std::vector<int>{1, 3, 2})) shapes.push_back(p0);
 				hipEvent_t e0 = nullptr, e1 = nullptr;
 				HIP_CHECK(hipEventCreate(&e0));
 				HIP_CHECK(hipEventCreate(&e1));
@@ -706,67 +888,32 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 					return run;
 				};
 				for (int p0 : shapes) {
-					// 256-lane tiles: three or two workgroups per CU; 512-lane
-					// tiles: one
-					const int kbs[2] = {p0 >= 5 ? 76 : 52, p0 >= 5 ? 150 : 76};
-					// untimed for comparison (it builds the shape's tables)
+					const uint32_t npts = tile_plan(g, p0).npts;
+					const uint32_t won = bp0 >= 0 ? tile_plan(g, bp0).npts : 0u;
+					if (won > 512 && (npts == 256 || (npts == 512 && g.ny <= 1))) continue;
+					// the first run builds the shape's tables; not compared
 					HIP_CHECK(hipEventRecord(e0, s));
-					// the last try takes the smallest LDS budget the windows
-					// fit, up to a CU's whole LDS (long windows: steep angles,
-					// coarse grids); 512-lane tiles, one per CU whatever the
-					// budget, try the whole LDS first
-					int tries[4] = {8 | (kbs[0] << 16), 4 | (kbs[0] << 16), kbs[1] << 16, 0};
-					if (p0 >= 5) {
-						tries[0] = 8 | (kbs[1] << 16);
-						tries[1] = 8 | (kbs[0] << 16);
-					}
-					int built = 0;
-					bool ok = false;
-					for (int k = 0; k < 4 && !ok; ++k) {
-						built = tries[k];
-						ok = launch_tiled(g, p0, built, scratch, a, d_delay, s);
-					}
+					if (!launch_tiled(g, p0, 0, scratch, a, d_delay, s)) continue;
 					HIP_CHECK(hipEventRecord(e1, s));
-					if (!ok) continue;
 					last_p0 = p0;
 					HIP_CHECK(hipEventSynchronize(e1));
 					float first_ms = 0.0f;
 					HIP_CHECK(hipEventElapsedTime(&first_ms, e0, e1));
 					if (first_ms > 2.0f * kTuneLimitMs) long_frame = true;
-					if (long_frame) {
-						float ms = 0.0f;
-						if (timed(p0, built, ms) && (bp0 < 0 || ms < best)) {
-							best = ms;
-							bp0 = p0;
-							bp1 = built;
-						}
-						continue;
-					}
-					// pairs per chunk (8 first: the better one when it fits) in
-					// each budget, then the smallest budget that fits
+					// pairs per transmit step (4 or 8) in the LDS budgets worth
+					// a try, then the smallest budget that fits; a long frame
+					// takes that alone
 					std::vector<int> cands;
-					for (int kb : kbs)
-						for (int tc : {8, 4}) cands.push_back(tc | (kb << 16));
-					// 512-lane tiles over 128-transmit blocks: also 16 pairs per
-					// chunk in the whole LDS (half the barriers; windows of up to
-					// 4 slots, FP16/BF16)
-					if (p0 >= 5 && g.ntx_pad == 128) cands.push_back(16 | (kbs[1] << 16));
-					cands.push_back(0);
+					if (!long_frame && npts == 2048) cands = {4 | (80 << 16), 8 | (160 << 16)};
+					else if (!long_frame && npts == 512) cands = {4 | (52 << 16), 8 | (52 << 16)};
+					if (npts != 2048 || long_frame) cands.push_back(0);
 					for (const int p1 : cands) {
-						if (bp0 >= 0 && best > kTuneLimitMs) {
-							long_frame = true;
-							break;
-						}
 						// the better of two runs (the first may find cold caches)
 						float ms = 0.0f;
 						bool run = false;
 						for (int rep = 0; rep < 2; ++rep) {
-							HIP_CHECK(hipEventRecord(e0, s));
-							run = launch_tiled(g, p0, p1, scratch, a, d_delay, s);
-							HIP_CHECK(hipEventRecord(e1, s));
-							HIP_CHECK(hipEventSynchronize(e1));
 							float t = 0.0f;
-							HIP_CHECK(hipEventElapsedTime(&t, e0, e1));
+							run = timed(p0, p1, t);
 							ms = rep == 0 ? t : std::min(ms, t);
 							if (!run || t > kTuneLimitMs) break;
 						}
@@ -811,13 +958,7 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 		return;
 	}
 	scratch.last_p0 = -1;
-	switch (g.storage) {
-	case MISTA_STORAGE_F32: launch_gather<MISTA_STORAGE_F32>(g, a, s); break;
-	case MISTA_STORAGE_F16: launch_gather<MISTA_STORAGE_F16>(g, a, s); break;
-	case kStorageReal: launch_gather<kStorageReal>(g, a, s); break;
-	default: launch_gather<MISTA_STORAGE_BF16>(g, a, s); break;
-	}
-	HIP_CHECK(hipGetLastError());
+	launch_gather_any<false>(g, a, s);
 }
 
 }  // namespace mista

@@ -6,6 +6,8 @@
 
 #include "common.h"
 
+#include <type_traits>
+
 namespace mista {
 namespace das {
 
@@ -105,20 +107,27 @@ template<> struct Entry<kStorageReal> {
 	}
 };
 
+// Receive elements whose sums one workgroup forms together, and the group
+// that the weights and window words are laid out by: [rx group][tx][kRxGroup].
+constexpr uint32_t kRxGroup = 4;
+
 struct DasArgs {
 	const void* tensor;   // [ntx][nrx][L] complex, storage type
 	const float* delay;   // [num_elements][npix]
-	const float* w;       // [nrx][ntx]
+	const float* w;       // [rx groups][ntx][kRxGroup]
 	float* value;         // [npix]
 	float* factor;        // [npix] or null
-	float2* partial;      // [nrx][npix] per-rx sums between transmit blocks (tiled, more than 128 transmits)
+	float2* partial;      // per-rx sums: [nrx][npix] (rx-parallel form) or [tiles][nrx][tile points]
 	uint64_t npix;
 	uint32_t first_tx, ntx, nrx, L;
-	uint32_t w_stride;    // row stride of w (transmits padded)
 	float offset;
 	float cf_factor;      // PCF: gamma / sigma0; SCF: p
 	float inv_num;        // 1 / (Ntx * Nrx)
 	int signed_value;     // RF samples: value = sum / (Ntx * Nrx), not |sum|
+	__device__ __forceinline__ float weight(uint32_t r, uint32_t t) const
+	{
+		return w[(static_cast<uint64_t>(r / kRxGroup) * ntx + t) * kRxGroup + r % kRxGroup];
+	}
 };
 
 // Shifted single-pass moments for the two-pass population sigma of
@@ -184,67 +193,6 @@ struct PixelStats {
 	}
 };
 
-// Per-rx statistics of the tiled kernel: PixelStats with the PCF moments (4
-// doubles per lane) kept in LDS at m.  They change once per rx, and in
-// registers they would push the kernel past its register budget (128
-// registers hold the lane's transmit delays).  The arithmetic is
-// PixelStats's, so both kernels give the same bits.
-template<int CF>
-struct TileStats {
-	float sr = 0.0f, si = 0.0f;
-	float k0 = 0.0f, k1 = 0.0f;   // the moments' shifts (first phase, first aux)
-	int sign_sum = 0;
-	double* m = nullptr;          // LDS: s1 and s2 of the phases, then of the aux phases
-	__device__ __forceinline__ void add_rx(float ar, float ai, bool first)
-	{
-		sr += ar;
-		si += ai;
-		if constexpr (CF == MISTA_CF_PCF) {
-			const float phi = atan2f(ai, ar);
-			const float aux = phi + ((phi < 0.0f) ? kPi : -kPi);
-			if (first) {
-				k0 = phi;
-				k1 = aux;
-			}
-			Moments m0, m1;
-			m0.k = k0;
-			m1.k = k1;
-			if (!first) {
-				m0.s1 = m[0];
-				m0.s2 = m[1];
-				m1.s1 = m[2];
-				m1.s2 = m[3];
-			}
-			m0.add(phi, false);
-			m1.add(aux, false);
-			m[0] = m0.s1;
-			m[1] = m0.s2;
-			m[2] = m1.s1;
-			m[3] = m1.s2;
-		} else if constexpr (CF == MISTA_CF_SCF) {
-			sign_sum += (ar >= 0.0f) ? 1 : -1;
-		}
-	}
-	__device__ __forceinline__ void write(const DasArgs& a, uint64_t p) const
-	{
-		PixelStats<CF> ps;
-		ps.sr = sr;
-		ps.si = si;
-		ps.sign_sum = sign_sum;
-		if constexpr (CF == MISTA_CF_PCF) {
-			ps.m0.k = k0;
-			ps.m1.k = k1;
-			ps.m0.s1 = m[0];
-			ps.m0.s2 = m[1];
-			ps.m1.s1 = m[2];
-			ps.m1.s2 = m[3];
-		}
-		ps.write(a, p);
-	}
-};
-// LDS bytes of the tiled kernel's per-lane statistics
-inline size_t tile_stats_bytes(int cf, uint32_t nt) { return cf == MISTA_CF_PCF ? static_cast<size_t>(nt) * 32 : 0; }
-
 // Tile geometry: a tw1 (x) by tw2 (y) by tzh (z) block of grid points, one
 // point per lane.  A plane has ny = tw2 = 1; a volume is laid out as
 // n1 = nx * ny columns (y fastest) by n2 = nz rows.  In a plane tile each wave
@@ -283,17 +231,21 @@ struct TileGeom {
 };
 
 // Window word per (tile, rx, tx):
-//   bits 0..30  ws * ESZ: byte offset in the channel of the first staged entry
-//               (ws = floor of the tile's lowest position for the pair)
-//   bit  31     record-end flag: some lane may have pos < 0 or i + 1 >= L,
-//               or the pair has nothing to stage (padded transmit, window
-//               past the record end)
+//   bits 0..23   ws * ESZ: byte offset in the channel of the first staged
+//                entry (ws = floor of the tile's lowest position for the pair)
+//   bits 24..30  1 KiB slots to copy (0: nothing to stage)
+//   bit  31      record-end flag: some lane may have pos < 0 or i + 1 >= L,
+//                or the pair has nothing to stage (padded transmit or receive
+//                element, window past the record end)
 // The lowest and highest positions use the same float expression order as
 // the lanes', (offset + d_tx) + d_rx, so by monotonic rounding every lane's
 // floor(pos) lies in [ws, floor(hi)], and floor(pos) + 1 in the staged
-// window of wcap entries.  The channel itself (t * nrx + r) is not stored:
-// the kernel forms its 64-bit address, so tensors of any size are tiled.
+// slots.  The channel itself (t * nrx + r) is not stored: the kernel forms
+// its 64-bit address, so tensors of any size are tiled.
 constexpr uint32_t kEdgeBit = 1u << 31;
+constexpr uint32_t kWsMask = (1u << 24) - 1u;
+constexpr uint32_t kSlotShift = 24;
+constexpr uint32_t kMaxWindowL = 1u << 21;   // records up to here: every ws * ESZ fits the word
 
 typedef __attribute__((address_space(1))) const void* gptr_t;
 typedef __attribute__((address_space(3))) void* lptr_t;
@@ -302,19 +254,24 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 typedef __attribute__((address_space(4))) const uint32_t* cu32_t;
 typedef __attribute__((address_space(4))) const float* cf32_t;
 
+// One frame's per-rx sums, or those of a run of its tiles (every per-tile
+// pointer starts at the run's first tile).
 struct TileArgs {
-	DasArgs d;
-	TileGeom tg;
-	const uint32_t* words;    // [ntiles][nrx][ntx_pad]
-	uint32_t S;               // 1 KiB load slots per staged window (wcap = S * SLOT entries)
-	uint32_t ntx_pad;         // transmits padded to the instantiated count
-	uint32_t nbuf;            // chunk buffers in the LDS ring (>= 2)
+	const void* tensor;       // [ntx][nrx][L] complex, storage type
+	const float* td;          // [tiles][nrx + ntx][tile points]: rx delays, then offset + tx delays, in lane order
+	const uint32_t* words;    // [tiles][rx groups][ntx][kRxGroup]
+	const uint32_t* slots;    // [tiles] 1 KiB slots of the tile's longest window
+	const float* w;           // [rx groups][ntx][kRxGroup]
+	float2* partial;          // [tiles][nrx][tile points]
+	uint32_t ntx, nrx, L;
+	uint32_t ntiles, ngrp, ngrp4;   // tiles; workgroups per tile; groups of kRxGroup receive elements
+	uint32_t lds, nbmax;      // LDS bytes of the ring; most chunk buffers in it (2..4)
 };
 
 // The tiles of up to kMaxBatch frames (possibly of different shapes) in one
-// launch: frame j's tiles are global tiles first[j] .. first[j+1]-1.  Every
-// frame shares the kernel instantiation (storage, coherence factor, transmit
-// block, chunk size, workgroup size) and the window size S and ring depth.
+// launch: frame j's items are global items first[j] .. first[j+1]-1.  Every
+// frame shares the kernel instantiation (storage, tile points, chunk size)
+// and the LDS ring's size.
 constexpr uint32_t kMaxBatch = 16;
 struct TileBatch {
 	TileArgs jobs[kMaxBatch];
@@ -322,7 +279,6 @@ struct TileBatch {
 	uint32_t njobs, total;
 };
 
-constexpr uint32_t kTileThreads = 256;
 // Zeroed bytes after the analytic tensor: a window is staged as whole 1 KiB
 // slots from its first entry, so the last channel's copies may read up to
 // (slots per window) KiB past its end; the launcher keeps windows below this.
@@ -337,38 +293,30 @@ constexpr uint32_t kMaxSlots = 64;
 // kernels using these never rely on m0 themselves.
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_dma4(const void* g, uint32_t lds)
-{
-	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" :: "s"(lds), "v"(g) : "memory", "m0");
-}
-// n (1..4) consecutive 1 KiB slots: global g + k KiB -> LDS lds + k KiB.
+// The first n of four consecutive 1 KiB slots: global base + voff + k KiB -> LDS
+// lds + k KiB, the wave-uniform base in scalar registers, voff = 16 * lane.
 // The instruction offset of global_load_lds moves both the global and the
 // LDS address (measured on gfx950: offset:1024 with m0 = B lands the source
-// bytes [1024, 2048) at LDS B + 1024), so one m0 serves four slots.
-__device__ __forceinline__ void lds_dma16_slots(const void* g, uint32_t lds, uint32_t n)
+// bytes [1024, 2048) at LDS B + 1024), so one m0 serves four slots.  One asm
+// block: as C++ the cases come out as a ladder of flag registers and branches.
+__device__ __forceinline__ void lds_dma16_slots(const void* base, uint32_t voff, uint32_t lds, uint32_t n)
 {
-	switch (n) {
-	case 1:
-		asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-				:: "s"(lds), "v"(g) : "memory", "m0");
-		break;
-	case 2:
-		asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
-				"global_load_lds_dwordx4 %1, off offset:1024"
-				:: "s"(lds), "v"(g) : "memory", "m0");
-		break;
-	case 3:
-		asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
-				"global_load_lds_dwordx4 %1, off offset:1024\n\tglobal_load_lds_dwordx4 %1, off offset:2048"
-				:: "s"(lds), "v"(g) : "memory", "m0");
-		break;
-	default:
-		asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off\n\t"
-				"global_load_lds_dwordx4 %1, off offset:1024\n\tglobal_load_lds_dwordx4 %1, off offset:2048\n\t"
-				"global_load_lds_dwordx4 %1, off offset:3072"
-				:: "s"(lds), "v"(g) : "memory", "m0");
-		break;
-	}
+	asm volatile(
+			"s_mov_b32 m0, %0\n\t"
+			"s_cmp_lt_u32 %3, 1\n\t"
+			"s_cbranch_scc1 .Ldma_%=\n\t"
+			"global_load_lds_dwordx4 %1, %2\n\t"
+			"s_cmp_lt_u32 %3, 2\n\t"
+			"s_cbranch_scc1 .Ldma_%=\n\t"
+			"global_load_lds_dwordx4 %1, %2 offset:1024\n\t"
+			"s_cmp_lt_u32 %3, 3\n\t"
+			"s_cbranch_scc1 .Ldma_%=\n\t"
+			"global_load_lds_dwordx4 %1, %2 offset:2048\n\t"
+			"s_cmp_lt_u32 %3, 4\n\t"
+			"s_cbranch_scc1 .Ldma_%=\n\t"
+			"global_load_lds_dwordx4 %1, %2 offset:3072\n"
+			".Ldma_%=:"
+			:: "s"(lds), "v"(voff), "s"(base), "s"(n) : "memory", "m0", "scc");
 }
 #pragma clang diagnostic pop
 
@@ -447,433 +395,316 @@ __device__ __forceinline__ void lds_read_pairs(const uint32_t* addr, typename Ld
 	}
 }
 
-// Chunk i of a tile = pairs (rx r, tx c*TC .. c*TC+TC-1), r = i / CPR,
-// c = i % CPR.  Chunks stream through a ring of nbuf LDS buffers, each
-// holding TC windows of S 1 KiB slots plus the tile's rx delays (one float
-// per lane, copied with the first chunk of every rx).  Chunk i + nbuf - 1 is
-// copied while chunk i is computed.  Wave w copies the windows of pairs
-// w, w + NW, ... of each chunk, every one as S whole slots from its first
-// entry, so every wave issues the same number of copies per chunk and waits
-// for chunk i alone with s_waitcnt vmcnt.  The chunk's window words and
-// weights are scalar-loaded one chunk ahead; its TC LDS reads are issued
-// together, each pair waiting for its own.  Chunks in which no pair can reach a record
-// end (the common case) take a path without the range test.
-// Occupancy: 256-lane workgroups target three waves per SIMD (up to 170
-// registers each); a 512-lane workgroup with its large LDS ring holds a CU
-// alone (two waves per SIMD), so it may use up to 256 registers, which buys
-// all of a chunk's LDS reads in flight at once.
-template<int NTHREADS> constexpr int tile_waves_per_eu() { return NTHREADS >= 512 ? 2 : 3; }
+constexpr uint32_t kTileZeroBytes = 128;
 
-template<int STORAGE, int CF, int NTXMAX, int TC, int NTHREADS, bool MULTI>
-__device__ __forceinline__ void das_tile(const TileArgs& A, const uint32_t tile, unsigned char* smem)
+// Chunk buffers of the ring for a tile whose longest window has S slots: as many
+// as fit with their buffers of transmit delays (0: not even two).
+__host__ __device__ inline uint32_t tile_buffers(uint32_t nbmax, uint32_t lds, uint32_t S, uint32_t rc, uint32_t h, uint32_t npts)
+{
+	uint32_t nb = nbmax < 4u ? nbmax : 4u;
+	while (nb >= 2u && kTileZeroBytes + nb * rc * S * 1024u + (1u + (nb - 1u) / h) * npts * 4u > lds) --nb;
+	return nb >= 2u ? nb : 0u;
+}
+
+// Per-rx sums of one tile: a workgroup of NT lanes, P points a lane (point k
+// of lane l is tile point k * NT + l), forms the sums of RC * H receive
+// elements over all transmits.  A chunk = RC receive elements of one transmit:
+// RC signal windows, each copied HBM -> LDS with direct loads (only as many
+// 1 KiB slots as the pair needs).  Chunk i = transmit i / H, receive elements
+// RC * (i % H) ..; a transmit's delays of the tile's points are copied the same
+// way, once for its H chunks, with the last chunk of the transmit before, and
+// read during that chunk.  Chunks stream through a ring of 2..4 LDS buffers
+// (as many as the tile's longest window leaves room for); chunk i + NB - 1 is
+// copied while chunk i is computed.
+template<int STORAGE, int NT, int P, int RC, int H>
+__device__ __forceinline__ void das_tile(const TileArgs& A, const uint32_t tile, const uint32_t grp, unsigned char* smem)
 {
 	using E = typename Entry<STORAGE>::T;
-	constexpr uint32_t NT = NTHREADS;       // one tile point per lane
 	constexpr uint32_t ESZ = sizeof(E);
-	constexpr uint32_t SLOT = 64 * 16 / ESZ;   // entries per wave load instruction (1 KiB)
 	constexpr uint32_t NW = NT / 64;
-	static_assert(TC % NW == 0, "every wave copies whole windows");
-	constexpr uint32_t PPW = TC / NW;       // windows copied per wave per chunk
-	constexpr uint32_t CPB = NTXMAX / TC;   // chunks per block of NTXMAX transmits
-	// LDS reads issued together: a whole chunk's where the register budget
-	// allows it (two waves per SIMD), four with up to 64 transmit delays in
-	// registers, else one at a time (128 registers hold transmit delays)
-	constexpr int BATCH = NTHREADS >= 512 ? (TC > 8 ? 8 : TC) : (NTXMAX <= 64 ? 4 : 1);
-	static_assert(BATCH == 1 || TC % BATCH == 0, "whole read groups per chunk");
+	constexpr uint32_t NPTS = NT * P;
+	constexpr uint32_t R = RC * H;             // receive elements of the workgroup
+	constexpr uint32_t WPW = NW / RC;          // waves that share a window's copy
+	constexpr uint32_t DSLOTS = NPTS / 256;    // slots of a transmit's delays
+	static_assert(NW % RC == 0 && (RC == 4 || R == 4), "whole waves per window; words of a chunk consecutive");
 
-	const DasArgs& a = A.d;
 	const uint32_t tid = threadIdx.x, lane = tid % 64;
-	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);   // uniform: scalar copy loops
-	uint32_t col, row;
-	bool valid;
-	A.tg.pixel(tile, tid, col, row, valid);
-	const uint64_t npix = a.npix;
-	const uint64_t p = static_cast<uint64_t>(col) * A.tg.n2 + row;
-	const uint32_t L = a.L, ntx = a.ntx, nrx = a.nrx;
-	// Transmits run in blocks: one of NTXMAX, or (MULTI, more than 128
-	// transmits) nblk equal blocks of BT <= 128, block-major over the receive
-	// elements, each receive element's partial sum kept in HBM from one block
-	// to the next (the same fma chain as one pass over all transmits), so a
-	// lane loads each block's transmit delays once.  A segment is one
-	// (block, rx): CPS chunks, the first of which also brings the tile's rx
-	// delays.
-	const uint32_t nblk = MULTI ? (A.ntx_pad + NTXMAX - 1) / NTXMAX : 1u;
-	const uint32_t BT = MULTI ? A.ntx_pad / nblk : NTXMAX;   // transmits per block
-	const uint32_t CPS = MULTI ? BT / TC : CPB;               // chunks per segment
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / 64);
+	const uint32_t nrx = A.nrx, L = A.L, ntx = A.ntx;
+	const uint32_t nchunks = ntx * H;
 	const float lim = static_cast<float>(L - 1u);
-	const uint32_t S = A.S, NB = A.nbuf;
-	const uint32_t wcap = S * SLOT;
-	const uint32_t win_bytes = TC * S * 1024u;
-	const uint32_t buf_bytes = win_bytes + NT * 4;    // windows + rx delays
-	const cu32_t wtab = (cu32_t)(A.words + static_cast<uint64_t>(tile) * nrx * A.ntx_pad);
-	const unsigned char* tensor = static_cast<const unsigned char*>(a.tensor);
-	const uint64_t chan_bytes = static_cast<uint64_t>(L) * ESZ;        // one channel
-	const uint64_t tx_bytes = chan_bytes * nrx;                        // one transmit's channels
+	const uint32_t S = *(cu32_t)(A.slots + tile);
+	const uint32_t win = S * 1024u;
+	const uint32_t buf_bytes = RC * win;
+	const uint32_t NB = tile_buffers(A.nbmax, A.lds, S, RC, H, NPTS);
+	const uint32_t ring = NB * buf_bytes;
+	const uint32_t ND = 1 + (NB - 1) / H;      // buffers of transmit delays, after the ring
+	const uint64_t chan_bytes = static_cast<uint64_t>(L) * ESZ;
+	const uint64_t tx_bytes = chan_bytes * nrx;
+	const uint32_t rows = nrx + ntx;
+	const float* td = A.td + static_cast<uint64_t>(tile) * rows * NPTS;
+	// words and weights [groups of kRxGroup][ntx][kRxGroup]: chunk (t, h) at
+	// t * kRxGroup + h * hstride
+	const uint32_t hstride = RC == kRxGroup ? ntx * kRxGroup : static_cast<uint32_t>(RC);
+	const uint32_t g4 = grp * (R / kRxGroup);
+	const cu32_t wtab = (cu32_t)(A.words + (static_cast<uint64_t>(tile) * A.ngrp4 + g4) * ntx * kRxGroup);
+	const cf32_t weights = (cf32_t)(A.w + static_cast<uint64_t>(g4) * ntx * kRxGroup);
 	const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) void*)smem));
+	const uint32_t voff = lane * 16;
+	// The first bytes stay zero: the entries of lanes outside the record.
+	const uint32_t lds_ring = lds0 + kTileZeroBytes;
+	if (tid < kTileZeroBytes / 4) reinterpret_cast<uint32_t*>(smem)[tid] = 0u;   // seen after the first chunk's barrier
 
-	// tx delays of this lane's point for transmit block blk, offset folded
-	// in: (offset + d_tx).  Transmits are padded to whole chunks: padded ones
-	// have weight 0, position far below 0 and copy from the tensor's start,
-	// so they take the excluded path.
-	float dtx[NTXMAX];
-	auto load_dtx = [&](uint32_t blk) {
-		const int nvalid = static_cast<int>(min(BT, ntx - blk * BT));   // the block's transmits
+	// rx delays of this lane's points (receive elements past the last shadow it)
+	float drx[R][P];
 #pragma unroll
-		for (int t = 0; t < NTXMAX; ++t) {
-			const uint32_t tt = min(blk * BT + static_cast<uint32_t>(t), ntx - 1);   // unconditional load, no branch
-			const float d = a.delay[static_cast<uint64_t>(a.first_tx + tt) * npix + p];
-			// 0 for the block's transmits, <= -1e30 past them: arithmetic
-			// rather than a select, so no compare mask per transmit is held
-			// in scalar registers while the loads are in flight
-			const float pen = fminf(0.0f, static_cast<float>(nvalid - 1 - t)) * 1.0e30f;
-			dtx[t] = (a.offset + d) + pen;
-		}
-	};
-	load_dtx(0);
+	for (uint32_t q = 0; q < R; ++q)
+#pragma unroll
+		for (int k = 0; k < P; ++k)
+			drx[q][k] = td[static_cast<uint64_t>(min(grp * R + q, nrx - 1)) * NPTS + k * NT + tid];
+	// Fence: waited for here, before the first copy.  Left to their first use
+	// in the chunk loop, the compiler waits there, in every chunk, for all
+	// copies in flight (it does not see the copies).
+#pragma unroll
+	for (uint32_t q = 0; q < R; ++q)
+#pragma unroll
+		for (int k = 0; k < P; ++k) asm volatile("" : "+v"(drx[q][k]));
 
-	const uint32_t nchunks = nblk * nrx * CPS;
-	const uint32_t Q = PPW * S;   // window copies per wave per chunk (+1 for the rx delays at an rx start)
-	const uint32_t S4 = S & ~3u, SR = S & 3u;   // slots in groups of four, and the rest
-	// Window words and weights are laid out [rx][ntx_pad] (the transmit rows
-	// padded to whole chunks): the chunk of segment (blk, r), position c
-	// holds entries r * ntx_pad + blk * BT + c * TC .. + TC - 1 of the tile's
-	// table and of the weights (without blocks: chunk k at k * TC).
-	// Issue cursor: the next chunk to copy, its segment position, its table
-	// offset, its ring buffer and the address of its first window's channel.
-	uint32_t is_k = 0, is_c = 0, is_r = 0, is_b = 0, is_off = 0, is_lds = lds0;
-	const unsigned char* is_rbase = tensor;   // tensor + (block start) * tx_bytes + (rx) * chan_bytes
-	const unsigned char* is_cbase = tensor;   // + is_c * TC * tx_bytes
-	const float* is_drx = a.delay + p;        // rx delays of is_k's rx for this lane
-	uint32_t iw[PPW];                         // words of is_k's pairs that this wave copies
-	auto load_issue_words = [&]() {
-		const cu32_t pr = wtab + is_off + wave;
+	// Copy cursor: chunk is_t, is_h; its ring buffer and its delays' buffer; the
+	// channel of this wave's window.  WPW waves share a window: this one copies
+	// the sub-th part of window wj.
+	const uint32_t wj = wave / WPW, sub = wave % WPW;
+	uint32_t is_t = 0, is_h = 0, is_buf = 0, is_d = 0;
+	const unsigned char* is_base = static_cast<const unsigned char*>(A.tensor) + (static_cast<uint64_t>(grp) * R + wj) * chan_bytes;
+	uint32_t iw = 0;
+	auto load_issue_word = [&]() { iw = wtab[is_t * kRxGroup + is_h * hstride + wj]; };
+	auto issue_delays = [&](uint32_t t) -> uint32_t {   // transmit t's, a slot a wave
+		uint32_t count = 0;
 #pragma unroll
-		for (uint32_t q = 0; q < PPW; ++q) iw[q] = pr[q * NW];
-	};
-	uint32_t pend = 0;   // (MULTI) segment starts among the chunks issued and not yet computed
-	auto issue = [&]() {
-		if (MULTI && is_c == 0) ++pend;
-#pragma unroll
-		for (uint32_t k = 0; k < PPW; ++k) {
-			const uint32_t j = wave + k * NW;
-			// padded transmits copy from the tensor's start (weight 0)
-			const unsigned char* src = (is_b * BT + is_c * TC + j < ntx) ? is_cbase + j * tx_bytes + (iw[k] & ~kEdgeBit) : tensor;
-			src += lane * 16;
-			uint32_t dst = is_lds + j * S * 1024u;
-			for (uint32_t s0 = 0; s0 < S4; s0 += 4, src += 4096, dst += 4096) lds_dma16_slots(src, dst, 4);
-			if (SR) lds_dma16_slots(src, dst, SR);
-		}
-		if (is_c == 0) lds_dma4(is_drx, __builtin_amdgcn_readfirstlane(is_lds + win_bytes + wave * 256));
-		// advance to the next chunk
-		++is_k;
-		is_lds += buf_bytes;
-		if (is_lds == lds0 + NB * buf_bytes) is_lds = lds0;
-		is_cbase += TC * tx_bytes;
-		is_off += TC;
-		if (++is_c == CPS) {
-			is_c = 0;
-			if (MULTI && ++is_r == nrx) {   // next block
-				is_r = 0;
-				++is_b;
-				is_rbase = tensor + static_cast<uint64_t>(is_b) * BT * tx_bytes;
-				is_drx = a.delay + p;
-				is_off = is_b * BT;
-			} else {
-				is_rbase += chan_bytes;
-				is_drx += npix;
-				is_off += A.ntx_pad - BT;   // (0 without blocks)
+		for (uint32_t d0 = 0; d0 < DSLOTS; d0 += NW) {
+			const uint32_t d = d0 + (NW - 1 - wave);
+			if (d0 + NW <= DSLOTS || d < DSLOTS) {
+				lds_dma16_slots(td + static_cast<uint64_t>(nrx + t) * NPTS + d * 256u, voff,
+						lds_ring + ring + (is_d * DSLOTS + d) * 1024u, 1);
+				++count;
 			}
-			is_cbase = is_rbase;
 		}
+		if (++is_d == ND) is_d = 0;
+		return count;
 	};
-	const uint32_t pre = min(NB - 1, nchunks);
-	for (uint32_t k = 0; k < pre; ++k) {
-		load_issue_words();
-		issue();
+	// copies of the cursor's chunk; returns how many copy instructions this wave issued
+	auto issue = [&]() -> uint32_t {
+		const uint32_t n = (iw >> kSlotShift) & 127u;
+		const uint32_t h = (n + WPW - 1) / WPW, s0 = sub * h;
+		uint32_t left = s0 < n ? min(h, n - s0) : 0u;
+		uint32_t count = left;
+		const unsigned char* src = is_base + is_h * RC * chan_bytes + static_cast<uint64_t>((iw & kWsMask) + s0 * 1024u);
+		uint32_t dst = lds_ring + is_buf + wj * win + s0 * 1024u;
+		for (; left > 4; left -= 4, src += 4096, dst += 4096) lds_dma16_slots(src, voff, dst, 4);
+		lds_dma16_slots(src, voff, dst, left);
+		is_buf += buf_bytes;
+		if (is_buf == ring) is_buf = 0;
+		if (++is_h == H) {
+			is_h = 0;
+			++is_t;
+			is_base += tx_bytes;
+			if (is_t < ntx) count += issue_delays(is_t);
+		}
+		return count;
+	};
+	(void)issue_delays(0);
+	uint32_t c1 = 0, c2 = 0;   // copies of the last chunk issued, of the one before
+	for (uint32_t k = 0; k < NB - 1 && k < nchunks; ++k) {
+		load_issue_word();
+		c2 = c1;
+		c1 = issue();
 	}
-	if (is_k < nchunks) load_issue_words();
+	if (is_t < ntx) load_issue_word();
 	// window words and weights of the chunk to compute, one chunk ahead
-	uint32_t cw[TC];
-	float cwt[TC];
+	uint32_t cw[RC];
+	float cwt[RC];
 	auto load_chunk = [&](uint32_t off) {
-		const cu32_t pr = wtab + off;
-		const cf32_t wr = (cf32_t)(a.w + static_cast<uint64_t>(off));
 #pragma unroll
-		for (uint32_t j = 0; j < TC; ++j) {
-			cw[j] = pr[j];
-			cwt[j] = wr[j];
+		for (uint32_t j = 0; j < RC; ++j) {
+			cw[j] = wtab[off + j];
+			cwt[j] = weights[off + j];
 		}
 	};
 	load_chunk(0);
 
-	TileStats<CF> st;
-	st.m = reinterpret_cast<double*>(smem + NB * buf_bytes + tid * 32);
-	uint32_t i = 0, bbase = 0;   // chunk being computed, its buffer's LDS offset
-	for (uint32_t blk = 0; blk < nblk; ++blk) {
-		if (MULTI && blk > 0) load_dtx(blk);   // waited for at its first use
-		for (uint32_t r = 0; r < nrx; ++r) {
-			float drx = 0.0f, ar = 0.0f, ai = 0.0f;
-			if (MULTI && blk > 0) {   // the sums of the earlier blocks
-				const float2 ps = a.partial[static_cast<uint64_t>(r) * npix + p];
-				ar = ps.x;
-				ai = ps.y;
+	float ar[R][P], ai[R][P];
+#pragma unroll
+	for (uint32_t q = 0; q < R; ++q)
+#pragma unroll
+		for (int k = 0; k < P; ++k) ar[q][k] = ai[q][k] = 0.0f;
+	typedef __attribute__((address_space(3))) const float* lds_float_t;
+	float dt[P], dnext[P];   // this transmit's delays, the next one's
+	uint32_t rd_d = 0;       // buffer of the next delays to read
+	auto read_delays = [&]() {
+		const lds_float_t dl = (lds_float_t)(size_t)(lds_ring + ring + rd_d * (DSLOTS * 1024u) + tid * 4u);
+#pragma unroll
+		for (int k = 0; k < P; ++k) dnext[k] = dl[k * NT];
+		if (++rd_d == ND) rd_d = 0;
+	};
+
+	// the first transmit's delays: waited for with everything issued so far
+	MISTA_VMCNT(0);
+	__syncthreads();
+	read_delays();
+	uint32_t bbase = 0;   // ring offset of the buffer of the chunk being computed
+	for (uint32_t t = 0; t < ntx; ++t) {
+#pragma unroll
+		for (int h = 0; h < H; ++h) {
+			uint32_t w_[RC];
+			float wt[RC];
+#pragma unroll
+			for (uint32_t j = 0; j < RC; ++j) {
+				w_[j] = cw[j];
+				wt[j] = cwt[j];
 			}
-			// (MULTI) table offset of the next chunk to load and of the next
-			// segment's first chunk: the next rx's, or the next block's
-			uint32_t ld_off = r * A.ntx_pad + blk * BT;
-			const uint32_t seg_next = r + 1 < nrx ? ld_off + A.ntx_pad : (blk + 1) * BT;
-			uint32_t left = CPS;   // (MULTI) chunks of this segment still to compute
-#pragma clang loop unroll(full)
-			for (int c = 0; c < static_cast<int>(CPB); ++c) {
-				// A block shorter than NTXMAX skips its last chunks: a guard,
-				// not an exit, so the trip count stays constant, the loop
-				// unrolls and dtx keeps compile-time indices.  The count is
-				// opaque to the compiler, which would otherwise hoist one
-				// compare per chunk out of the rx loop into scalar registers.
-				if (MULTI) {
-					asm volatile("" : "+s"(left));
-					if (left == 0) continue;
+			// copies issued after this chunk: those of the NB - 2 chunks that follow
+			wait_vmcnt_at_most((NB > 2 ? c1 : 0u) + (NB > 3 ? c2 : 0u));
+			__syncthreads();
+			c2 = c1;
+			c1 = is_t < ntx ? issue() : 0u;
+			if (h == 0) {
+#pragma unroll
+				for (int k = 0; k < P; ++k) dt[k] = dnext[k];
+			}
+			// Register fence: this chunk's positions are computed here, not
+			// ahead of the barrier for all H chunks.
+#pragma unroll
+			for (int k = 0; k < P; ++k) asm volatile("" : "+v"(dt[k]));
+			uint32_t any_edge = 0;
+#pragma unroll
+			for (uint32_t j = 0; j < RC; ++j) any_edge |= w_[j];
+			const uint32_t lb = lds_ring + bbase;
+			// Positions and LDS addresses.  A chunk in which some lane may lie
+			// outside 0 <= pos < L - 1 (or with nothing staged for a pair)
+			// sends those lanes to the zero entries: they add zero.  The range
+			// test is one unsigned compare of the bit patterns: positions are
+			// never -0, and negative values and NaN compare above L - 1's.
+			constexpr int N = RC * P;
+			uint32_t addr[N];
+			float kf[N];
+#pragma unroll
+			for (uint32_t j = 0; j < RC; ++j) {
+				const uint32_t base = lb + j * win - (w_[j] & kWsMask);
+#pragma unroll
+				for (int k = 0; k < P; ++k) {
+					const float pos = dt[k] + drx[h * RC + j][k];
+					kf[j * P + k] = __builtin_amdgcn_fractf(pos);
+					addr[j * P + k] = static_cast<uint32_t>(pos) * ESZ + base;
 				}
-				// this chunk's words and weights (loaded one chunk ahead)
-				uint32_t w_[TC];
-				float wt[TC];
+			}
+			if (any_edge & kEdgeBit) {
 #pragma unroll
-				for (int j = 0; j < TC; ++j) {
-					w_[j] = cw[j];
-					wt[j] = cwt[j];
-				}
-				// copies issued after chunk i: chunks i+1 .. is_k-1, Q each
-				// plus one for every chunk that starts a segment (loads and
-				// stores of partial sums issued since only make the wait
-				// stricter)
-				uint32_t after;
-				if (MULTI) after = (is_k - 1 - i) * Q + pend - (c == 0 ? 1u : 0u);
-				else if (i + NB - 2 < nchunks) after = (NB - 2) * Q + (static_cast<uint32_t>(c) + NB - 2) / CPS;
-				else after = (nchunks - 1 - i) * Q + (nrx - 1 - r);
-				wait_vmcnt_at_most(after);         // this wave's copies of chunk i landed
-				__syncthreads();                   // everyone's did; buffer of chunk i-1 is free
-				// Waves still issuing copies, positions and LDS reads go
-				// before waves already accumulating (the reads then start
-				// sooner after the barrier): F32 DAS 9.97 -> 9.94 ms, F16
-				// 6.33 -> 6.26 ms.  Lowered once the chunk's last reads are issued.
-				if constexpr (BATCH > 1) __builtin_amdgcn_s_setprio(2);
-				if (MULTI && c == 0) --pend;
-				if (is_k < nchunks) issue();
-				if (c == 0) drx = *reinterpret_cast<const float*>(smem + bbase + win_bytes + tid * 4);
-				// Register fences: this chunk's positions are computed after
-				// the barrier, and its accumulation is finished before the
-				// next one, so only one chunk's temporaries are ever live.
-				asm volatile("" : "+v"(drx));
-				uint32_t any_edge = 0;
+				for (uint32_t j = 0; j < RC; ++j) {
+					const uint32_t limj = (w_[j] >> kSlotShift) & 127u ? __float_as_uint(lim) : 0u;
 #pragma unroll
-				for (int j = 0; j < TC; ++j) any_edge |= w_[j];
-				const uint32_t wbase = lds0 + bbase;
-				// entry address and weight of pair j for this lane
-				auto fast_pair = [&](int j, uint32_t& addr, float& kf, float& wv) {
-					// every lane of every pair of the chunk is inside 0 <= pos < L - 1
-					const float pos = dtx[c * TC + j] + drx;
-					kf = __builtin_amdgcn_fractf(pos);
-					addr = static_cast<uint32_t>(pos) * ESZ + (wbase + static_cast<uint32_t>(j) * S * 1024u - w_[j]);
-					wv = wt[j];
-				};
-				auto edge_pair = [&](int j, uint32_t& addr, float& kf, float& wv) {
-					// One form for every pair: lanes outside 0 <= pos < L-1
-					// get weight 0; the entry index floor(pos) - ws is
-					// clamped, as an unsigned value, to the window, which
-					// changes nothing for in-range lanes (it lies in
-					// [0, need - 2] by the window construction) and keeps
-					// excluded lanes' reads on staged (finite) entries, whose
-					// products with weight 0 leave the sums as they are (a sum
-					// is never -0).  0 <= pos < lim is one unsigned compare of
-					// the bit patterns: positions are never -0 (delays are
-					// >= +0), so non-negative ones order like their bits, and
-					// negative values and NaN compare above lim's.  (The
-					// fenced copy of drx keeps the compiler from computing
-					// both paths' positions ahead of the branch.)
-					float dr = drx;
-					asm volatile("" : "+v"(dr));
-					const float pos = dtx[c * TC + j] + dr;
-					kf = __builtin_amdgcn_fractf(pos);
-					const uint32_t ws = (w_[j] & ~kEdgeBit) / ESZ;
-					const bool ok = __float_as_uint(pos) < __float_as_uint(lim);
-					const float pc = __builtin_amdgcn_fmed3f(pos, 0.0f, lim);   // NaN-free, no int overflow
-					const uint32_t rel = min(static_cast<uint32_t>(static_cast<int>(pc)) - ws, wcap - 2u);
-					addr = rel * ESZ + wbase + static_cast<uint32_t>(j) * S * 1024u;
-					wv = ok ? wt[j] : 0.0f;
-				};
-				auto accumulate = [&](const float2 v, float wv) {
-					ar = fmaf(v.x, wv, ar);
-					ai = fmaf(v.y, wv, ai);
-				};
-				auto run = [&](auto&& pair) {
-					if constexpr (BATCH > 1) {
-						// groups of BATCH pairs: BATCH LDS reads in flight
-#pragma unroll
-						for (int g = 0; g < TC; g += BATCH) {
-							uint32_t addr[BATCH];
-							float kf[BATCH], wv[BATCH];
-#pragma unroll
-							for (int q = 0; q < BATCH; ++q) pair(g + q, addr[q], kf[q], wv[q]);
-							typename LdsPair<ESZ>::T e[BATCH];
-							lds_read_pairs<ESZ, BATCH>(addr, e);
-							if (g + BATCH >= TC) __builtin_amdgcn_s_setprio(0);
-#pragma unroll
-							for (int q = 0; q < BATCH; ++q) accumulate(Entry<STORAGE>::lerp2(e[q], kf[q]), wv[q]);
-						}
-					} else {
-#pragma unroll
-						for (int j = 0; j < TC; ++j) {
-							uint32_t addr;
-							float kf, wv;
-							pair(j, addr, kf, wv);
-							const E* e = reinterpret_cast<const E*>(smem + (addr - lds0));
-							accumulate(Entry<STORAGE>::lerp(e, kf), wv);
-						}
-					}
-				};
-				if (!(any_edge & kEdgeBit)) run(fast_pair);
-				else run(edge_pair);
-				asm volatile("" : "+v"(ar), "+v"(ai));
-				// the next chunks' scalars, after this chunk's LDS reads (a
-				// scalar load in flight would hold up their wait): in flight
-				// during the next barrier
-				if (is_k < nchunks) load_issue_words();
-				if (i + 1 < nchunks) {
-					if (MULTI) {
-						ld_off = left > 1 ? ld_off + TC : seg_next;
-						load_chunk(ld_off);
-					} else {
-						load_chunk((i + 1) * TC);
+					for (int k = 0; k < P; ++k) {
+						const float pos = dt[k] + drx[h * RC + j][k];
+						if (!(__float_as_uint(pos) < limj)) addr[j * P + k] = lds0;
 					}
 				}
-				bbase += buf_bytes;
-				if (bbase == NB * buf_bytes) bbase = 0;
-				++i;
-				if (MULTI) --left;
 			}
-			if (MULTI && blk + 1 < nblk) {
-				if (valid) a.partial[static_cast<uint64_t>(r) * npix + p] = make_float2(ar, ai);
-			} else {
-				st.add_rx(ar, ai, r == 0);
-			}
+			typename LdsPair<ESZ>::T v[N];
+			lds_read_pairs<ESZ, N>(addr, v);
+			if (h == H - 1) read_delays();
+#pragma unroll
+			for (uint32_t j = 0; j < RC; ++j)
+#pragma unroll
+				for (int k = 0; k < P; ++k) {
+					const uint32_t q = h * RC + j;
+					const float2 s = Entry<STORAGE>::lerp2(v[j * P + k], kf[j * P + k]);
+					ar[q][k] = fmaf(s.x, wt[j], ar[q][k]);
+					if constexpr (STORAGE != kStorageReal) ai[q][k] = fmaf(s.y, wt[j], ai[q][k]);
+				}
+			// ... and its sums are finished before the next chunk
+#pragma unroll
+			for (uint32_t q = h * RC; q < (h + 1) * RC; ++q)
+#pragma unroll
+				for (int k = 0; k < P; ++k) asm volatile("" : "+v"(ar[q][k]), "+v"(ai[q][k]));
+			// the next chunks' scalars, after this chunk's LDS reads (a scalar
+			// load in flight would hold up their wait): in flight during the
+			// next barrier
+			if (is_t < ntx) load_issue_word();
+			if (h + 1 < H) load_chunk(t * kRxGroup + (h + 1) * hstride);
+			else if (t + 1 < ntx) load_chunk((t + 1) * kRxGroup);
+			bbase += buf_bytes;
+			if (bbase == ring) bbase = 0;
 		}
 	}
-	MISTA_VMCNT(0);
-	if (valid) st.write(a, p);
+	float2* out = A.partial + (static_cast<uint64_t>(tile) * nrx + grp * R) * NPTS + tid;
+#pragma unroll
+	for (uint32_t q = 0; q < R; ++q)
+		if (grp * R + q < nrx)
+#pragma unroll
+			for (int k = 0; k < P; ++k) out[static_cast<uint64_t>(q) * NPTS + k * NT] = make_float2(ar[q][k], ai[q][k]);
 }
 
-// A workgroup per tile.  XCD-aware order: workgroups are dealt round-robin
-// to the 8 XCDs (block b runs on XCD b % 8), so XCD x gets one contiguous run
-// of the tiles; tiles running at the same time on one XCD then share windows
-// in its L2.
-__device__ __forceinline__ uint32_t xcd_tile()
+// Item (tile, rx group) of a launch of n items, XCD-aware: workgroups are
+// dealt round-robin to the 8 XCDs (block b runs on XCD b % 8), so XCD x gets
+// one contiguous run of the items.
+__device__ __forceinline__ uint32_t xcd_item()
 {
 	const uint32_t T = gridDim.x, q8 = T / 8, rm8 = T % 8, xcd = blockIdx.x % 8;
 	return xcd * q8 + min(xcd, rm8) + blockIdx.x / 8;
 }
 
-// Windows of pairs with nothing to stage are read (with weight 0): the ring
-// starts from zeros so that no stale bit pattern can be Inf/NaN.
-template<int TC, int NTHREADS>
-__device__ __forceinline__ void zero_ring(unsigned char* smem, uint32_t nbuf, uint32_t S)
-{
-	const uint32_t ring = nbuf * (TC * S * 1024u + NTHREADS * 4u);
-	for (uint32_t i = threadIdx.x; i < ring / 16; i += NTHREADS)
-		reinterpret_cast<uint4*>(smem)[i] = make_uint4(0u, 0u, 0u, 0u);
-	__syncthreads();
-}
-
 // One frame: its arguments arrive as the kernel's own, which the compiler
-// keeps in scalar registers for the whole tile.
-template<int STORAGE, int CF, int NTXMAX, int TC, int NTHREADS, bool MULTI>
-__global__ void __launch_bounds__(NTHREADS)
-__attribute__((amdgpu_waves_per_eu(tile_waves_per_eu<NTHREADS>(), tile_waves_per_eu<NTHREADS>())))
+// keeps in scalar registers.
+template<int STORAGE, int NT, int P, int RC, int H>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 das_tile_kernel(const TileArgs A)
 {
 	extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-	zero_ring<TC, NTHREADS>(smem, A.nbuf, A.S);
-	das_tile<STORAGE, CF, NTXMAX, TC, NTHREADS, MULTI>(A, xcd_tile(), smem);
+	const uint32_t item = xcd_item();
+	das_tile<STORAGE, NT, P, RC, H>(A, item % A.ntiles, item / A.ntiles, smem);
 }
 
-// A batch of frames in one launch, their tiles concatenated: the hardware
+// A batch of frames in one launch, their items concatenated: the hardware
 // dispatcher starts each workgroup as a CU frees up, so frames of uneven cost
 // balance by themselves.  (A separate kernel: a frame's arguments picked from
 // the table by a run-time index are reloaded from memory at their uses.)
-template<int STORAGE, int CF, int NTXMAX, int TC, int NTHREADS, bool MULTI>
-__global__ void __launch_bounds__(NTHREADS)
-__attribute__((amdgpu_waves_per_eu(tile_waves_per_eu<NTHREADS>(), tile_waves_per_eu<NTHREADS>())))
+template<int STORAGE, int NT, int P, int RC, int H>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 das_tile_batch_kernel(const TileBatch B)
 {
 	extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-	zero_ring<TC, NTHREADS>(smem, B.jobs[0].nbuf, B.jobs[0].S);
-	const uint32_t g = xcd_tile();
+	const uint32_t g = xcd_item();
 	uint32_t j = 0;
 	while (j + 1 < B.njobs && B.first[j + 1] <= g) ++j;
-	das_tile<STORAGE, CF, NTXMAX, TC, NTHREADS, MULTI>(B.jobs[j], g - B.first[j], smem);
+	const uint32_t item = g - B.first[j];
+	das_tile<STORAGE, NT, P, RC, H>(B.jobs[j], item % B.jobs[j].ntiles, item / B.jobs[j].ntiles, smem);
 }
 
-// LDS bytes of one chunk buffer: TC windows of S 1 KiB slots + the rx delays.
-inline size_t tile_buffer_bytes(uint32_t tc, uint32_t S, uint32_t nt)
+template<int STORAGE, int NT, int P, int RC, int H>
+void launch_tile_t(const TileBatch& B, hipStream_t s)
 {
-	return static_cast<size_t>(tc) * S * 1024u + nt * 4;
-}
-
-template<int STORAGE, int CF, int NTXMAX>
-void launch_tile_t(const TileBatch& B, uint32_t nt, uint32_t tc, hipStream_t s)
-{
-	const TileArgs& A = B.jobs[0];   // S, nbuf and the transmit padding are shared by the batch
-	const size_t lds = A.nbuf * tile_buffer_bytes(tc, A.S, nt) + tile_stats_bytes(CF, nt);
-	const uint32_t grid = B.total;   // a workgroup per tile
-	auto go1 = [&](auto kern, auto kern_batch, uint32_t threads) {
-		if (B.njobs == 1) {
-			HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-					static_cast<int>(lds)));
-			hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), lds, s, A);
-		} else {
-			HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern_batch),
-					hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-			hipLaunchKernelGGL(kern_batch, dim3(grid), dim3(threads), lds, s, B);
-		}
+	const TileArgs& A = B.jobs[0];   // the ring's size is shared by the batch
+	auto go = [&](auto kern, const auto& args) {
+		HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+				static_cast<int>(A.lds)));
+		hipLaunchKernelGGL(kern, dim3(B.total), dim3(NT), A.lds, s, args);
 	};
-#define MISTA_GO(tcv, ntv, multi) \
-	go1(das_tile_kernel<STORAGE, CF, NTXMAX, tcv, ntv, multi>, das_tile_batch_kernel<STORAGE, CF, NTXMAX, tcv, ntv, multi>, ntv)
-	if constexpr (NTXMAX == 128) {
-		if (A.ntx_pad > NTXMAX) {   // several transmit blocks: 512-lane tiles only
-			if (nt != 512) MISTA_THROW(MISTA_E_INVALID_STATE, "tile of " << nt << " lanes for " << A.ntx_pad << " transmits");
-			MISTA_GO(8, 512, true);
-			return;
-		}
-	}
-	if constexpr (NTXMAX == 128) {
-		if (nt == 512 && tc == 16) {
-			MISTA_GO(16, 512, false);
-			return;
-		}
-	}
-	if (nt == 512) MISTA_GO(8, 512, false);
-	else if (tc == 8) MISTA_GO(8, 256, false);
-	else MISTA_GO(4, 256, false);
-#undef MISTA_GO
-}
-
-template<int STORAGE, int CF>
-void launch_tile_n(const TileBatch& B, uint32_t nt, uint32_t tc, hipStream_t s)
-{
-	const uint32_t ntx_pad = B.jobs[0].ntx_pad;
-	if (ntx_pad == 32) launch_tile_t<STORAGE, CF, 32>(B, nt, tc, s);
-	else if (ntx_pad == 64) launch_tile_t<STORAGE, CF, 64>(B, nt, tc, s);
-	else launch_tile_t<STORAGE, CF, 128>(B, nt, tc, s);
+	if (B.njobs == 1) go(das_tile_kernel<STORAGE, NT, P, RC, H>, A);
+	else go(das_tile_batch_kernel<STORAGE, NT, P, RC, H>, B);
 }
 
 // Tiled launch for one storage kind (instantiated in das_tile_<storage>.hip).
 template<int STORAGE>
-void launch_tile_storage(int cf, const TileBatch& B, uint32_t nt, uint32_t tc, hipStream_t s)
+void launch_tile_storage(const TileBatch& B, uint32_t npts, uint32_t r, uint32_t nt, hipStream_t s)
 {
-	switch (cf) {
-	case MISTA_CF_NONE: launch_tile_n<STORAGE, MISTA_CF_NONE>(B, nt, tc, s); break;
-	case MISTA_CF_PCF: launch_tile_n<STORAGE, MISTA_CF_PCF>(B, nt, tc, s); break;
-	default: launch_tile_n<STORAGE, MISTA_CF_SCF>(B, nt, tc, s); break;
-	}
+	if (npts == 256) launch_tile_t<STORAGE, 256, 1, 4, 1>(B, s);
+	else if (npts == 512 && r == 16) launch_tile_t<STORAGE, 512, 1, 4, 4>(B, s);
+	else if (npts == 512 && r == 8) launch_tile_t<STORAGE, 256, 2, 4, 2>(B, s);
+	else if (npts == 512) launch_tile_t<STORAGE, 256, 2, 4, 1>(B, s);
+	else if (npts == 1024 && r == 8) launch_tile_t<STORAGE, 512, 2, 4, 2>(B, s);
+	else if (npts == 1024) launch_tile_t<STORAGE, 512, 2, 4, 1>(B, s);
+	else if (nt == 512) launch_tile_t<STORAGE, 512, 4, 2, 2>(B, s);
+	else if (r == 8) launch_tile_t<STORAGE, 1024, 2, 4, 2>(B, s);
+	else launch_tile_t<STORAGE, 1024, 2, 4, 1>(B, s);
 }
 
 }  // namespace das

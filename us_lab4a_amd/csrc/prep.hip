@@ -966,18 +966,18 @@ void launch_tensor_convert_out(const FrameGeom& g, const void* d_tensor, const f
 
 // ---------------------------------------------------------------- weights
 
-// w[r][t] = rxApod[r] * txApod[t] * scale[t][r], rx-major with the tx row
-// padded to ntx_pad zeros (the tx loop reads consecutive weights);
+// rxApod[r] * txApod[t] * scale[t][r] as w[r / 4][t][r % 4], the order in which
+// the tiled DAS reads weights (groups of four receive elements), padding zero;
 // txApod/scale optional.
-__global__ void __launch_bounds__(256) weights_kernel(uint32_t ntx, uint32_t ntx_pad, uint32_t nrx,
+__global__ void __launch_bounds__(256) weights_kernel(uint32_t ntx, uint32_t nrx, uint32_t n,
 		const float* __restrict__ rx_apod, const float* __restrict__ tx_apod, const float* __restrict__ scale,
 		float* __restrict__ w)
 {
 	const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= ntx_pad * nrx) return;
-	const uint32_t r = i / ntx_pad, t = i % ntx_pad;
+	if (i >= n) return;
+	const uint32_t r = i / (4 * ntx) * 4 + i % 4, t = i / 4 % ntx;
 	float v = 0.0f;
-	if (t < ntx) {
+	if (r < nrx) {
 		v = rx_apod[r];
 		if (tx_apod) v = v * tx_apod[t];
 		if (scale) v = v * scale[static_cast<uint64_t>(t) * nrx + r];
@@ -988,8 +988,8 @@ __global__ void __launch_bounds__(256) weights_kernel(uint32_t ntx, uint32_t ntx
 void launch_weights(const FrameGeom& g, const float* d_rx_apod, const float* d_tx_apod, const float* d_scale,
 		float* d_w, hipStream_t s)
 {
-	const uint32_t n = g.ntx_pad * g.nrx;
-	hipLaunchKernelGGL(weights_kernel, dim3((n + 255) / 256), dim3(256), 0, s, g.ntx, g.ntx_pad, g.nrx, d_rx_apod,
+	const uint32_t n = g.ntx * pad_nrx(g.nrx);
+	hipLaunchKernelGGL(weights_kernel, dim3((n + 255) / 256), dim3(256), 0, s, g.ntx, g.nrx, n, d_rx_apod,
 			d_tx_apod, storage_scaled(g.storage) ? d_scale : nullptr, d_w);
 	HIP_CHECK(hipGetLastError());
 }

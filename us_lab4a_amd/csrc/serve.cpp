@@ -114,7 +114,7 @@ size_t estimate_bytes(const mista_job& j)
 	const uint64_t npix = static_cast<uint64_t>(j.n1) * j.n2;
 	const uint64_t tensor = ntx * nrx * L * storage_bytes(c.storage);
 	const uint64_t delays = nrx * npix * 4 + npix * 8;
-	const uint64_t ntx_pad = pad_ntx(static_cast<uint32_t>(ntx));
+	const uint64_t ntx_pad = budget_pad_ntx(static_cast<uint32_t>(ntx));
 	const uint64_t tables = (npix / 256 + 1) * (nrx * ntx_pad * 8 + nrx * 8);
 	const uint64_t chunk = std::min<uint64_t>(ntx * nrx, 1024);
 	const uint64_t prep = chunk * nf * (4 + 8 + 16);
