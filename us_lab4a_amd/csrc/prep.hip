@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace mista {
 
@@ -285,11 +286,23 @@ __device__ inline uint32_t pack_f16x2(float re, float im)
 //             x, Y[k] = -i sgn(k) X[k] (sgn 0 at bins 0 and N/2), a real
 //             signal: y[2m] + i y[2m+1] = IDFT_M(C)[m] / M with C[0] = 0,
 //             C[k] = i sin(2 pi k/N) Z[k] + cos(2 pi k/N) conj(Z[M-k]);
-//   output:   (x_i - mean, y_i), x recomputed from the echo and the filter,
-//             which stay in LDS after the transform buffer.
+//   output:   (x_i - mean, y_i), x recomputed from the echo, which stays in
+//             LDS after the transform buffer.
 // The inverse runs as a forward transform of the conjugate.  FFTs are
-// Stockham passes of radix 8/4/2/3/5: every thread reads its butterflies'
+// Stockham passes of radix 8/9/6/4/2/3/5: every thread reads its butterflies'
 // inputs into registers, a barrier, then writes the outputs in place.
+//
+// Bounds, 128 x 128 channels of 4096 samples x 8 (M = 17 280; one workgroup a
+// CU, its 138 KB of transform): the ten passes 1.56 ms (LDS in and out, then
+// arithmetic, a barrier between: with one workgroup nothing fills the other's
+// phase), FIR, mean and output 1.2 ms at FP16, 1.45 at FP32, of which writing
+// the tensor is 0.5 / 0.95.  With both FIR evaluations as vector arithmetic
+// (27 fma an output, twice) and the spectrum rule and the scale as passes of
+// their own the kernel took 3.82 ms at FP32 and 3.29 at FP16; now 2.98 and
+// 2.77 (64 x 64 channels of 2048 x 8, two workgroups a CU: 0.54 -> 0.37).
+// Measured slower: twiddles loaded ahead of a pass's barrier (3.0 to 3.5 ms
+// at FP16), twiddles in [i][j] order (3.44), the FIR's echo operand straight
+// from memory (3.9).
 
 constexpr int kFftThreads = 1024;
 constexpr uint32_t kFirJ = 27;   // taps per phase of the Kaiser upsampling design (every U)
@@ -448,16 +461,31 @@ template<> __device__ __forceinline__ void dft<9>(float2* v)
 	}
 }
 
-template<int R>
-__device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uint32_t magic,
-		const float2* __restrict__ tw)
+// Transforms per lane count: a workgroup of NT lanes holds at most 18 NT
+// complex values (kFftMaxM at 1024 lanes).
+constexpr uint32_t kFftPerLane = 18;
+static_assert(kFftPerLane * kFftThreads == kFftMaxM, "1024 lanes hold the longest transform");
+
+// Table entry i: a 32-bit byte offset from the uniform base (one address
+// register a load; the tables are below 4 GiB).
+__device__ __forceinline__ float2 table_at(const float2* __restrict__ base, uint32_t i)
 {
-	constexpr int MAXB = static_cast<int>((kFftMaxM / R + kFftThreads - 1) / kFftThreads);
+	return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(base) + i * static_cast<uint32_t>(sizeof(float2)));
+}
+
+// One Stockham pass over D in place: every lane reads its butterflies' inputs,
+// a barrier, then the outputs.  MAX: also the largest |re|, |im| of the outputs
+// with index below npair (and |re| at npair when odd).
+template<int NT, int R, bool MAX>
+__device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uint32_t magic,
+		const float2* __restrict__ tw, uint32_t L, float& mx)
+{
+	constexpr int MAXB = static_cast<int>((kFftPerLane + R - 1) / R);
 	const uint32_t nb = M / R;
 	float2 v[MAXB][R];
 #pragma unroll
 	for (int t = 0; t < MAXB; ++t) {
-		const uint32_t b = threadIdx.x + static_cast<uint32_t>(t) * kFftThreads;
+		const uint32_t b = threadIdx.x + static_cast<uint32_t>(t) * NT;
 		if (b < nb) {
 #pragma unroll
 			for (int i = 0; i < R; ++i) v[t][i] = D[b + i * nb];
@@ -466,7 +494,7 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 	__syncthreads();
 #pragma unroll
 	for (int t = 0; t < MAXB; ++t) {
-		const uint32_t b = threadIdx.x + static_cast<uint32_t>(t) * kFftThreads;
+		const uint32_t b = threadIdx.x + static_cast<uint32_t>(t) * NT;
 		if (b < nb) {
 			// q = b / Ns by a multiply-high: with magic = ceil(2^32 / Ns) =
 			// (2^32 + e) / Ns, b * magic / 2^32 = b / Ns + b e / (Ns 2^32),
@@ -474,7 +502,9 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 			const uint32_t q = (Ns == 1) ? b : __umulhi(b, magic);
 			const uint32_t j = b - q * Ns;
 			if (Ns > 1) {   // (the first pass's twiddles are all 1)
-				const float2* w = tw + j * (R - 1);
+				// a lane's twiddles are consecutive: few wide loads (an [i][j]
+				// layout, coalesced but a load each, measured slower)
+				const float2* w = reinterpret_cast<const float2*>(reinterpret_cast<const char*>(tw) + j * static_cast<uint32_t>((R - 1) * sizeof(float2)));
 #pragma unroll
 				for (int i = 1; i < R; ++i) v[t][i] = cmul(v[t][i], w[i - 1]);
 			}
@@ -482,25 +512,147 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 			const uint32_t o = q * Ns * R + j;
 #pragma unroll
 			for (int i = 0; i < R; ++i) D[o + i * Ns] = v[t][i];
+			if constexpr (MAX) {
+#pragma unroll
+				for (int i = 0; i < R; ++i) {
+					const uint32_t k = 2 * (o + i * Ns);
+					if (k < L) mx = fmaxf(mx, fabsf(v[t][i].x));
+					if (k + 1 < L) mx = fmaxf(mx, fabsf(v[t][i].y));
+				}
+			}
 		}
 	}
 	__syncthreads();
 }
 
-__device__ void fft_forward(float2* D, const FftPlanArgs& P, const float2* __restrict__ tw)
+// Spectrum rule Z -> conj(C) (C[0] = 0, C[k] = i sin(2 pi k/N) Z[k] +
+// cos(2 pi k/N) conj(Z[M-k]), C[M/2] = i Z[M/2]) and the first inverse pass
+// (no twiddles) in one trip through the registers: the bins of butterfly u are
+// u + i nb, and the partner M - k of bin i is bin R - 1 - i of butterfly
+// nb - u, so a lane takes both butterflies.  u = 0 (bin i with bin R - i) and
+// u = nb/2 (i with R - 1 - i) are their own partners.
+// Butterfly pairs a lane holds: two of radix 5 (u <= M / 10 <= 1.8 NT), one of
+// radix 8 or 9, whose registers would spill (longer transforms run
+// hilbert_in_place and a plain pass).
+template<int R> constexpr int hilbert_slots() { return R == 5 ? 2 : 1; }
+template<int NT, int R>
+__device__ __forceinline__ void hilbert_pass(float2* D, uint32_t M, const float2* __restrict__ wpost)
 {
-	for (uint32_t p = 0; p < P.npass; ++p) {
-		const float2* t = tw + P.tw_off[p];
-		switch (P.radix[p]) {
-		case 8: fft_pass<8>(D, P.M, P.ns[p], P.ns_magic[p], t); break;
-		case 9: fft_pass<9>(D, P.M, P.ns[p], P.ns_magic[p], t); break;
-		case 6: fft_pass<6>(D, P.M, P.ns[p], P.ns_magic[p], t); break;
-		case 4: fft_pass<4>(D, P.M, P.ns[p], P.ns_magic[p], t); break;
-		case 2: fft_pass<2>(D, P.M, P.ns[p], P.ns_magic[p], t); break;
-		case 3: fft_pass<3>(D, P.M, P.ns[p], P.ns_magic[p], t); break;
-		default: fft_pass<5>(D, P.M, P.ns[p], P.ns_magic[p], t); break;
+	constexpr int MAXP = hilbert_slots<R>();
+	const uint32_t nb = M / R;
+	float2 v1[MAXP][R], v2[MAXP][R];
+#pragma unroll
+	for (int s = 0; s < MAXP; ++s) {
+		const uint32_t u = threadIdx.x + static_cast<uint32_t>(s) * NT;
+		if (2 * u <= nb) {
+#pragma unroll
+			for (int i = 0; i < R; ++i) {
+				v1[s][i] = D[u + i * nb];
+				// the partners of v1[i], i = R-1 .. 0: for u = 0 the next bin's
+				v2[s][i] = D[u == 0 ? (i + 1 < R ? i + 1 : 0) * nb : nb - u + i * nb];
+			}
 		}
 	}
+	__syncthreads();
+#pragma unroll
+	for (int s = 0; s < MAXP; ++s) {
+		uint32_t u = threadIdx.x + static_cast<uint32_t>(s) * NT;
+		// fence: this slot's table loads are not moved ahead of the barrier
+		asm volatile("" : "+v"(u));
+		if (2 * u <= nb) {
+#pragma unroll
+			for (int i = 0; i < R; ++i) {
+				// the pair (k, M - k) with the lower bin first: this bin is
+				// the lower one for 2 i < R (k = M/2, its own partner, only
+				// for i = R / 2 with u = 0 or u = nb/2)
+				float2& a = v1[s][i];
+				float2& b = v2[s][R - 1 - i];
+				const uint32_t k = u + i * nb;
+				const bool low = 2 * i < R;   // compile time: the loop is unrolled
+				const float2 w = table_at(wpost, low ? k : M - k);   // (cos, -sin)
+				const float2 p = low ? a : b, q = low ? b : a;
+				const float c = w.x, sn = -w.y;
+				float2 ck = make_float2(fmaf(c, q.x, -sn * p.y), fmaf(sn, p.x, -c * q.y));
+				float2 cm = make_float2(fmaf(-c, p.x, -sn * q.y), fmaf(sn, q.x, c * p.y));
+				if (i == R / 2 && 2 * k == M) ck = cm = make_float2(-p.y, p.x);   // i Z
+				if (s == 0 && i == 0 && u == 0) ck = make_float2(0.0f, 0.0f);
+				a = conjf2(low ? ck : cm);
+				b = conjf2(low ? cm : ck);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+			dft<R>(v1[s]);
+#pragma unroll
+			for (int i = 0; i < R; ++i) D[u * R + i] = v1[s][i];
+			if (u != 0 && 2 * u != nb) {
+				dft<R>(v2[s]);
+#pragma unroll
+				for (int i = 0; i < R; ++i) D[(nb - u) * R + i] = v2[s][i];
+			}
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	}
+	__syncthreads();
+}
+
+// The spectrum rule alone, a lane a bin pair.
+template<int NT>
+__device__ __forceinline__ void hilbert_in_place(float2* D, uint32_t M, const float2* __restrict__ wpost)
+{
+	for (uint32_t k = threadIdx.x; k <= M / 2; k += NT) {
+		if (k == 0) {
+			D[0] = make_float2(0.0f, 0.0f);
+		} else if (2 * k == M) {
+			const float2 a = D[k];
+			D[k] = make_float2(-a.y, -a.x);   // conj(i Z)
+		} else {
+			const float2 a = D[k], b = D[M - k];
+			const float2 w = table_at(wpost, k);
+			const float c = w.x, sn = -w.y;
+			D[k] = conjf2(make_float2(fmaf(c, b.x, -sn * a.y), fmaf(sn, a.x, -c * b.y)));
+			D[M - k] = conjf2(make_float2(fmaf(-c, a.x, -sn * b.y), fmaf(sn, b.x, c * a.y)));
+		}
+	}
+	__syncthreads();
+}
+
+#define MISTA_RADIX(r, call) \
+	switch (r) { \
+	case 8: call(8); break; \
+	case 9: call(9); break; \
+	case 6: call(6); break; \
+	case 4: call(4); break; \
+	case 2: call(2); break; \
+	case 3: call(3); break; \
+	default: call(5); break; \
+	}
+
+// D = DFT_M of the packed real signal in place -> F = DFT_M(conj C), the
+// Hilbert transform's samples; returns the lane's part of the largest |re|,
+// |im| of F over the first L samples.
+template<int NT>
+__device__ __forceinline__ float analytic_transforms(float2* D, const FftPlanArgs& P, const float2* __restrict__ tw,
+		const float2* __restrict__ wpost, uint32_t L)
+{
+	float mx = 0.0f;
+	const uint32_t np = P.npass;
+	// forward passes, spectrum and the first inverse pass, the other inverse
+	// passes.  Transforms this long start with radix 5, 8 or 9.
+	const bool pairs = P.radix[0] == 5;
+	for (uint32_t s = 0; s + 1 < 2 * np; ++s) {
+		const uint32_t p = s < np ? s : s - np;
+		if (s == np && pairs) {
+			hilbert_pass<NT, 5>(D, P.M, wpost);
+			continue;
+		}
+		if (s == np) hilbert_in_place<NT>(D, P.M, wpost);
+#define MISTA_CALL(r) fft_pass<NT, r, false>(D, P.M, P.ns[p], P.ns_magic[p], tw + P.tw_off[p], L, mx)
+		MISTA_RADIX(P.radix[p], MISTA_CALL)
+#undef MISTA_CALL
+	}
+#define MISTA_CALL(r) fft_pass<NT, r, true>(D, P.M, P.ns[np - 1], P.ns_magic[np - 1], tw + P.tw_off[np - 1], L, mx)
+	MISTA_RADIX(P.radix[np - 1], MISTA_CALL)
+#undef MISTA_CALL
+	return mx;
 }
 
 // FIR x U output i (no DC removal): the generic polyphase loop over the
@@ -518,172 +670,230 @@ __device__ __forceinline__ float fir_at(const AnalyticArgs& A, const float* xs, 
 	return acc;
 }
 
-__global__ void __launch_bounds__(kFftThreads) analytic_lds_kernel(const AnalyticArgs A)
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// FIR x UP on the matrix cores (UP divides 16; UP = 1: the samples themselves).
+// The outputs i = 256 tile + 16 c + m of 16 columns c are the product of a
+// constant 16 x K matrix of taps (row m = dq UP + p: phase p of the column's
+// dq-th input position) and a K x 16 matrix of echo samples, K = 27 taps +
+// 16/UP - 1 rounded up to 4: K/4 steps of v_mfma_f32_16x16x4_f32, which rounds
+// like the fma chain over the taps in order (measured: equal bits; the zero
+// taps at both ends add nothing).  Lane l gets the outputs
+// i = 256 tile + 16 (l % 16) + 4 (l / 16) + 0..3.
+template<int UP> struct MatFir {
+	static constexpr int Q = 16 / UP;   // input positions per column
+	static constexpr int STEPS = UP == 1 ? 1 : (static_cast<int>(kFirJ) + Q - 1 + 3) / 4;
+	// the echo in LDS: zeros before and after it, for the columns at both ends
+	static constexpr int PADL = 16, PADR = Q + 16;
+	static_assert(UP == 1 || 4 * STEPS - Q - 13 <= PADL, "the first column's oldest sample");
+	float a[STEPS];
+	int c0;   // echo index of this lane's first B entry at tile 0
+	__device__ explicit MatFir(const AnalyticArgs& A)
+	{
+		const int lane = static_cast<int>(threadIdx.x & 63), m = lane % 16, g = lane / 16;
+		if constexpr (UP > 1) {
+			// step entry s = 4 k + g holds tap j = s - (Q - 1) + dq and echo
+			// sample Q c + off/UP + Q - 1 - s
+			const int dq = m / UP, p = m % UP;
+#pragma unroll
+			for (int k = 0; k < STEPS; ++k) {
+				const int j = 4 * k + g - (Q - 1) + dq;
+				a[k] = (j >= 0 && j < static_cast<int>(kFirJ)) ? A.hpoly[p * static_cast<int>(kFirJ) + j] : 0.0f;
+			}
+			c0 = Q * m + static_cast<int>(A.off) / UP + Q - 1 - g;
+		} else {
+			a[0] = 0.0f;
+			c0 = 16 * m + 4 * g;
+		}
+	}
+	// x: the echo in LDS (UP > 1; sample q at x[PADL + q]) or in memory (UP = 1)
+	__device__ __forceinline__ f32x4 tile(const float* x, uint32_t ns, uint32_t t) const
+	{
+		// (columns past the record's last read its end: their outputs are dropped)
+		const int last = static_cast<int>(ns) + PADR - 1;
+		const int c = min(c0 + static_cast<int>(t) * (16 * Q), last);
+		f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+		if constexpr (UP > 1) {
+			float b[STEPS];
+			const float* xc = x + (PADL + c);
+#pragma unroll
+			for (int k = 0; k < STEPS; ++k) b[k] = xc[-4 * k];
+#pragma unroll
+			for (int k = 0; k < STEPS; ++k) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[k], b[k], acc, 0, 0, 0);
+		} else {
+#pragma unroll
+			for (int k = 0; k < 4; ++k) acc[k] = c + k < static_cast<int>(ns) ? x[c + k] : 0.0f;
+		}
+		return acc;
+	}
+};
+
+// UP: the matrix-core FIR's factor, 0 = any other factor or filter (taps and
+// echo in LDS, NT = 1024).
+template<int NT, int UP>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4))) analytic_lds_kernel(const AnalyticArgs A)
 {
 	extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-	__shared__ double red[kFftThreads / 64];
-	__shared__ float redm[kFftThreads / 64], redx[kFftThreads / 64], redn[kFftThreads / 64];
+	constexpr uint32_t NW = NT / 64;
+	constexpr uint32_t TILES = 2 * kFftPerLane * NT / 256 / NW;   // 256-output FIR tiles of a wave, at most
+	__shared__ double red[NW];
+	__shared__ float redm[NW], redx[NW], redn[NW];
 	const uint32_t tid = threadIdx.x, ch = blockIdx.x;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
 	const uint32_t M = A.plan.M, N = A.N, L = A.L, up = A.up, J = A.J;
 	float2* D = reinterpret_cast<float2*>(lds);
 	float* Df = reinterpret_cast<float*>(lds);
 	const uint32_t right = A.off / up + 2;
-	float* xs = reinterpret_cast<float*>(lds + static_cast<size_t>(M) * sizeof(float2));   // [J + ns + right]
-	float* hs = xs + J + A.ns + right;                                                    // [up][J]
+	float* xs = reinterpret_cast<float*>(lds + static_cast<size_t>(M) * sizeof(float2));   // the echo: UP = 0 [J + ns + right], UP > 1 [PADL + ns + PADR]
+	float* hs = xs + J + A.ns + right;                                                    // UP = 0: [up][J]
+	const float* src = A.raw + static_cast<uint64_t>(ch) * A.ns;
+	const uint32_t ntl = (L + 255) / 256;
+	const uint32_t in_tile = 16 * (lane % 16) + 4 * (lane / 16);
+	const float* echo = UP > 1 ? xs : src;
 
 	// FIR x U (Interpolator.h:64-138, polyphase) and DC removal
 	// (Util.h:1009-1018) into the packed real array Df[0, L); Df[L, N) = 0.
-	const float* src = A.raw + static_cast<uint64_t>(ch) * A.ns;
-	if (up > 1) {
-		for (uint32_t i = tid; i < J + A.ns + right; i += kFftThreads) {
-			const int q = static_cast<int>(i) - static_cast<int>(J);
-			xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
-		}
-		for (uint32_t i = tid; i < up * J; i += kFftThreads) hs[i] = A.hpoly[i];
-		__syncthreads();
-	}
 	double part = 0.0;
 	float xmax = -3.4e38f, xmin = 3.4e38f;   // extremes of the FIR output over [0, L) (storage scale)
-	if (up > 1 && J == kFirJ) {
-		// Lane per input position q: the window x[q-26..q] sits in registers
-		// and serves all U phases (outputs m = q*U + p, i = m - off); the
-		// taps, the same for every lane, come through the scalar cache.  Each
-		// output is the same fma chain over j = 0..J-1 as below.
-		const cf32_t hg = (cf32_t)A.hpoly;
-		const uint32_t q_lo = A.off / up, q_hi = (L - 1 + A.off) / up;
-		for (uint32_t q = q_lo + tid; q <= q_hi; q += kFftThreads) {
-			float xw[kFirJ];
-			const float* xrow = xs + J + q;
+	float mean = 0.0f;
+	auto reduce_mean = [&]() {
+		if (!(A.flags & kRemoveDc)) return;
+		for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
+		if (lane == 0) red[wave] = part;
+		__syncthreads();
+		double sum = red[0];
+		for (uint32_t w = 1; w < NW; ++w) sum += red[w];
+		mean = static_cast<float>(sum / static_cast<double>(L - A.dz));
+	};
+	if constexpr (UP > 0) {
+		// the wave's outputs wait in registers for the mean
+		const MatFir<UP> fir(A);
+		if constexpr (UP > 1) {
+			constexpr int PADL = MatFir<UP>::PADL;
+			for (uint32_t i = tid; i < A.ns + PADL + MatFir<UP>::PADR; i += NT) {
+				const int q = static_cast<int>(i) - PADL;
+				xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
+			}
+			__syncthreads();
+		}
+		f32x4 x[TILES];
 #pragma unroll
-			for (int j = 0; j < kFirJ; ++j) xw[j] = xrow[-j];
-			const int ibase = static_cast<int>(q * up) - static_cast<int>(A.off);
-			// U = 8 or 4 with the lane's outputs inside [dz, L) and 16-byte
-			// aligned: the U phases leave as float4 stores (one lane's
-			// outputs are contiguous; phase by phase the lanes would write
-			// 4U bytes apart, onto a few LDS banks)
-			if ((up == 8 || up == 4) && ibase >= static_cast<int>(A.dz) && ibase + static_cast<int>(up) <= static_cast<int>(L) &&
-					(ibase & 3) == 0) {
+		for (uint32_t k = 0; k < TILES; ++k) {
+			const uint32_t t = wave + k * NW;
+			if (t >= ntl) continue;
+			x[k] = fir.tile(echo, A.ns, t);
+			if (256 * t >= A.dz && 256 * (t + 1) <= L) {
 #pragma unroll
-				for (uint32_t h = 0; h < 8; h += 4) {
-					if (h >= up) break;
-					float o[4];
+				for (int q = 0; q < 4; ++q) {
+					part += static_cast<double>(x[k][q]);
+					xmax = fmaxf(xmax, x[k][q]);
+					xmin = fminf(xmin, x[k][q]);
+				}
+			} else {
 #pragma unroll
-					for (int k = 0; k < 4; ++k) {
-						const cf32_t hrow = hg + (h + k) * kFirJ;
-						float acc = 0.0f;
+				for (int q = 0; q < 4; ++q) {
+					const uint32_t i = 256 * t + in_tile + q;
+					if (i < L) {
+						if (i >= A.dz) part += static_cast<double>(x[k][q]);
+						xmax = fmaxf(xmax, x[k][q]);
+						xmin = fminf(xmin, x[k][q]);
+					}
+				}
+			}
+		}
+		reduce_mean();
 #pragma unroll
-						for (int j = 0; j < kFirJ; ++j) acc = fmaf(hrow[j], xw[j], acc);
-						o[k] = acc;
-						part += static_cast<double>(acc);
+		for (uint32_t k = 0; k < TILES; ++k) {
+			const uint32_t t = wave + k * NW;
+			if (t >= ntl) continue;
+			const uint32_t i = 256 * t + in_tile;
+#pragma unroll
+			for (int q = 0; q < 4; ++q) x[k][q] = i + q < L ? x[k][q] - mean : 0.0f;
+			*reinterpret_cast<f32x4*>(Df + i) = x[k];   // (256 ntl <= L + 255 < N)
+		}
+		for (uint32_t i = 256 * ntl + tid; i < N; i += NT) Df[i] = 0.0f;
+	} else {
+		if (up > 1) {
+			for (uint32_t i = tid; i < J + A.ns + right; i += NT) {
+				const int q = static_cast<int>(i) - static_cast<int>(J);
+				xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
+			}
+			for (uint32_t i = tid; i < up * J; i += NT) hs[i] = A.hpoly[i];
+			__syncthreads();
+		}
+		if (up > 1 && J == kFirJ) {
+			// Lane per input position q: the window x[q-26..q] sits in
+			// registers and serves all U phases (outputs m = q*U + p,
+			// i = m - off); the taps, the same for every lane, come through
+			// the scalar cache.
+			const cf32_t hg = (cf32_t)A.hpoly;
+			const uint32_t q_lo = A.off / up, q_hi = (L - 1 + A.off) / up;
+			for (uint32_t q = q_lo + tid; q <= q_hi; q += NT) {
+				float xw[kFirJ];
+				const float* xrow = xs + J + q;
+#pragma unroll
+				for (int j = 0; j < static_cast<int>(kFirJ); ++j) xw[j] = xrow[-j];
+				const int ibase = static_cast<int>(q * up) - static_cast<int>(A.off);
+				for (uint32_t ph = 0; ph < up; ++ph) {
+					const cf32_t hrow = hg + ph * kFirJ;
+					float acc = 0.0f;
+#pragma unroll
+					for (int j = 0; j < static_cast<int>(kFirJ); ++j) acc = fmaf(hrow[j], xw[j], acc);
+					const int i = ibase + static_cast<int>(ph);
+					if (i >= 0 && i < static_cast<int>(L)) {
+						if (static_cast<uint32_t>(i) >= A.dz) part += static_cast<double>(acc);
 						xmax = fmaxf(xmax, acc);
 						xmin = fminf(xmin, acc);
+						Df[i] = acc;
 					}
-					*reinterpret_cast<float4*>(Df + ibase + h) = make_float4(o[0], o[1], o[2], o[3]);
-				}
-				continue;
-			}
-			for (uint32_t ph = 0; ph < up; ++ph) {
-				const cf32_t hrow = hg + ph * kFirJ;
-				float acc = 0.0f;
-#pragma unroll
-				for (int j = 0; j < kFirJ; ++j) acc = fmaf(hrow[j], xw[j], acc);
-				const int i = ibase + static_cast<int>(ph);
-				if (i >= 0 && i < static_cast<int>(L)) {
-					if (static_cast<uint32_t>(i) >= A.dz) part += static_cast<double>(acc);
-					xmax = fmaxf(xmax, acc);
-					xmin = fminf(xmin, acc);
-					Df[i] = acc;
 				}
 			}
+		} else for (uint32_t i = tid; i < L; i += NT) {
+			const float acc = fir_at(A, xs, hs, src, i);
+			if (i >= A.dz) part += static_cast<double>(acc);
+			xmax = fmaxf(xmax, acc);
+			xmin = fminf(xmin, acc);
+			Df[i] = acc;
 		}
-	} else for (uint32_t i = tid; i < L; i += kFftThreads) {
-		const float acc = fir_at(A, xs, hs, src, i);
-		if (i >= A.dz) part += static_cast<double>(acc);
-		xmax = fmaxf(xmax, acc);
-		xmin = fminf(xmin, acc);
-		Df[i] = acc;
-	}
-	for (uint32_t i = L + tid; i < N; i += kFftThreads) Df[i] = 0.0f;
-	float mean = 0.0f;
-	if (A.flags & kRemoveDc) {
-		for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
-		if ((tid & 63) == 0) red[tid >> 6] = part;
-		__syncthreads();
-		if (tid == 0) {
-			double s = 0.0;
-			for (int w = 0; w < kFftThreads / 64; ++w) s += red[w];
-			red[0] = s;
-		}
-		__syncthreads();
-		mean = static_cast<float>(red[0] / static_cast<double>(L - A.dz));
-		for (uint32_t i = tid; i < L; i += kFftThreads) Df[i] = Df[i] - mean;
+		for (uint32_t i = L + tid; i < N; i += NT) Df[i] = 0.0f;
+		reduce_mean();
+		if (A.flags & kRemoveDc)
+			for (uint32_t i = tid; i < L; i += NT) Df[i] = Df[i] - mean;
 	}
 	__syncthreads();
 
-	fft_forward(D, A.plan, A.tw);
-
-	// Z = DFT_M(x[2m] + i x[2m+1]) -> conj(C), in place: C[0] = 0,
-	// C[k] = i sin(2 pi k/N) Z[k] + cos(2 pi k/N) conj(Z[M-k]), 0 < k < M
-	// (pairs k, M-k by one thread; C[M/2] = i Z[M/2]).
-	const uint32_t half = M / 2;
-	for (uint32_t k = tid; k <= half; k += kFftThreads) {
-		if (k == 0) {
-			D[0] = make_float2(0.0f, 0.0f);
-		} else if (2 * k == M) {
-			const float2 a = D[k];
-			D[k] = make_float2(-a.y, -a.x);   // conj(i Z)
-		} else {
-			const float2 a = D[k], b = D[M - k];
-			const float2 w = A.wpost[k];      // (cos, -sin)
-			const float c = w.x, sn = -w.y;
-			const float2 ck = make_float2(fmaf(c, b.x, -sn * a.y), fmaf(sn, a.x, -c * b.y));
-			const float2 cm = make_float2(fmaf(-c, a.x, -sn * b.y), fmaf(sn, b.x, c * a.y));
-			D[k] = conjf2(ck);
-			D[M - k] = conjf2(cm);
-		}
-	}
-	__syncthreads();
-	fft_forward(D, A.plan, A.tw);
+	float my = analytic_transforms<NT>(D, A.plan, A.tw, A.wpost, L);
 
 	// y[2m] + i y[2m+1] = conj(D[m]) / M: the Hilbert transform of x, the
 	// imaginary part of the analytic signal, whose real part is x itself
-	// (recomputed from the echo and filter kept in LDS).
+	// (recomputed from the echo and the filter).
 	const float coef = 2.0f / static_cast<float>(N);
-	auto hil = [&](uint32_t i) -> float {
-		const float2 v = D[i >> 1];
-		return (i & 1u) ? -v.y * coef : v.x * coef;
-	};
 	const bool mag = (A.flags & kOutMagnitude) != 0;
 	float inv = 1.0f;
 	if (A.out16) {
 		// FP16/BF16 storage over the channel scale s = max(|re|, |im|) (1 if
 		// zero), stored value z/s.  max |x_i - mean| is reached at the
-		// extremes of x (rounding is monotonic and odd): the workgroup's
-		// max x, max -x and max |y| are reduced first.
-		float my = 0.0f, nxmin = -xmin;
-		for (uint32_t m = tid; 2 * m < L; m += kFftThreads) {
-			const float2 v = D[m];
-			my = fmaxf(my, fabsf(v.x * coef));
-			if (2 * m + 1 < L) my = fmaxf(my, fabsf(-v.y * coef));
-		}
+		// extremes of x, max |y| at max |F| (rounding is monotonic and odd):
+		// the workgroup's max x, max -x and max |F| are reduced first.
+		float nxmin = -xmin;
 		for (int o = 32; o > 0; o >>= 1) {
 			my = fmaxf(my, __shfl_xor(my, o, 64));
 			xmax = fmaxf(xmax, __shfl_xor(xmax, o, 64));
 			nxmin = fmaxf(nxmin, __shfl_xor(nxmin, o, 64));
 		}
-		if ((tid & 63) == 0) {
-			redm[tid >> 6] = my;
-			redx[tid >> 6] = xmax;
-			redn[tid >> 6] = nxmin;
+		if (lane == 0) {
+			redm[wave] = my;
+			redx[wave] = xmax;
+			redn[wave] = nxmin;
 		}
 		__syncthreads();
 		float gy = redm[0], gx = redx[0], gn = redn[0];
-		for (int w = 1; w < kFftThreads / 64; ++w) {
+		for (uint32_t w = 1; w < NW; ++w) {
 			gy = fmaxf(gy, redm[w]);
 			gx = fmaxf(gx, redx[w]);
 			gn = fmaxf(gn, redn[w]);
 		}
-		const float gm = fmaxf(gy, fmaxf(fabsf(gx - mean), fabsf(-gn - mean)));
+		const float gm = fmaxf(gy * coef, fmaxf(fabsf(gx - mean), fabsf(-gn - mean)));
 		const float sc = (gm > 0.0f) ? gm : 1.0f;
 		inv = 1.0f / sc;
 		if (tid == 0) A.scale[ch] = sc;
@@ -698,67 +908,44 @@ __global__ void __launch_bounds__(kFftThreads) analytic_lds_kernel(const Analyti
 		else if (mag) dmag[i] = sqrtf(re * re + im * im);
 		else dst[i] = make_float2(re, im);
 	};
-	if (up > 1 && J == kFirJ && (up == 8 || up == 4) && A.off % up == 0 && !mag) {
-		// the FIR again, lane per input position: the lane's U outputs are
-		// contiguous and aligned (off is a multiple of U), written as 16-byte
-		// stores of (x, y) pairs
-		const cf32_t hg = (cf32_t)A.hpoly;
-		const uint32_t q_lo = A.off / up, q_hi = (L - 1 + A.off) / up;
-		for (uint32_t q = q_lo + tid; q <= q_hi; q += kFftThreads) {
-			float xw[kFirJ];
-			const float* xrow = xs + J + q;
-#pragma unroll
-			for (int j = 0; j < kFirJ; ++j) xw[j] = xrow[-j];
-			const uint32_t i0 = q * up - A.off;
-			if (i0 + up <= L) {
-#pragma unroll
-				for (uint32_t h = 0; h < 8; h += 4) {
-					if (h >= up) break;
-					float re[4], im[4];
-#pragma unroll
-					for (int k = 0; k < 4; ++k) {
-						const cf32_t hrow = hg + (h + k) * kFirJ;
-						float acc = 0.0f;
-#pragma unroll
-						for (int j = 0; j < kFirJ; ++j) acc = fmaf(hrow[j], xw[j], acc);
-						re[k] = acc - mean;
-					}
-					const float4 yv = *reinterpret_cast<const float4*>(D + ((i0 + h) >> 1));   // y pairs of 4 outputs
-					im[0] = yv.x * coef;
-					im[1] = -yv.y * coef;
-					im[2] = yv.z * coef;
-					im[3] = -yv.w * coef;
-					if (A.out16) {
-						uint4 pk;
-						if (bf) {
-							pk = make_uint4(pack_bf16x2(re[0] * inv, im[0] * inv), pack_bf16x2(re[1] * inv, im[1] * inv),
-									pack_bf16x2(re[2] * inv, im[2] * inv), pack_bf16x2(re[3] * inv, im[3] * inv));
-						} else {
-							pk = make_uint4(pack_f16x2(re[0] * inv, im[0] * inv), pack_f16x2(re[1] * inv, im[1] * inv),
-									pack_f16x2(re[2] * inv, im[2] * inv), pack_f16x2(re[3] * inv, im[3] * inv));
-						}
-						*reinterpret_cast<uint4*>(row16 + i0 + h) = pk;
+	if constexpr (UP > 0) {
+		// whole 16-byte stores where every row starts aligned
+		const bool vec = A.out16 ? (L & 3u) == 0 : (!mag && (L & 1u) == 0);
+		const MatFir<UP> fir(A);
+#pragma unroll 1
+		for (uint32_t t = wave; t < ntl; t += NW) {
+			const uint32_t i = 256 * t + in_tile;
+			const f32x4 x = fir.tile(echo, A.ns, t);
+			const float4 yv = *reinterpret_cast<const float4*>(Df + i);
+			const float re[4] = {x[0] - mean, x[1] - mean, x[2] - mean, x[3] - mean};
+			const float im[4] = {yv.x * coef, -yv.y * coef, yv.z * coef, -yv.w * coef};
+			if (vec && i + 4 <= L) {
+				if (A.out16) {
+					uint4 pk;
+					if (bf) {
+						pk = make_uint4(pack_bf16x2(re[0] * inv, im[0] * inv), pack_bf16x2(re[1] * inv, im[1] * inv),
+								pack_bf16x2(re[2] * inv, im[2] * inv), pack_bf16x2(re[3] * inv, im[3] * inv));
 					} else {
-						*reinterpret_cast<float4*>(dst + i0 + h) = make_float4(re[0], im[0], re[1], im[1]);
-						*reinterpret_cast<float4*>(dst + i0 + h + 2) = make_float4(re[2], im[2], re[3], im[3]);
+						pk = make_uint4(pack_f16x2(re[0] * inv, im[0] * inv), pack_f16x2(re[1] * inv, im[1] * inv),
+								pack_f16x2(re[2] * inv, im[2] * inv), pack_f16x2(re[3] * inv, im[3] * inv));
 					}
+					*reinterpret_cast<uint4*>(row16 + i) = pk;
+				} else {
+					*reinterpret_cast<float4*>(dst + i) = make_float4(re[0], im[0], re[1], im[1]);
+					*reinterpret_cast<float4*>(dst + i + 2) = make_float4(re[2], im[2], re[3], im[3]);
 				}
 			} else {
-				for (uint32_t ph = 0; ph < up; ++ph) {
-					const uint32_t i = i0 + ph;
-					if (i >= L) break;
-					const cf32_t hrow = hg + ph * kFirJ;
-					float acc = 0.0f;
 #pragma unroll
-					for (int j = 0; j < kFirJ; ++j) acc = fmaf(hrow[j], xw[j], acc);
-					put1(i, acc - mean, hil(i));
-				}
+				for (int q = 0; q < 4; ++q)
+					if (i + q < L) put1(i + q, re[q], im[q]);
 			}
 		}
-		return;
+	} else {
+		for (uint32_t i = tid; i < L; i += NT) {
+			const float2 v = D[i >> 1];
+			put1(i, fir_at(A, xs, hs, src, i) - mean, (i & 1u) ? -v.y * coef : v.x * coef);
+		}
 	}
-	// any other filter or rate: output by output
-	for (uint32_t i = tid; i < L; i += kFftThreads) put1(i, fir_at(A, xs, hs, src, i) - mean, hil(i));
 }
 
 // ---------------------------------------------------------------- long records
@@ -1054,7 +1241,17 @@ static void launch_fir(uint32_t nch, const FrameGeom& g, const float* raw, const
 			hpoly, J, off, out, xmax);
 }
 
-// LDS bytes of the fused kernel for this frame (0 if it cannot run).
+// Matrix-core FIR factor of the fused kernel for this filter, 0 where its taps
+// do not tile (the other factors run the generic FIR).
+static uint32_t fused_up(uint32_t up, uint32_t J, uint32_t off)
+{
+	if (up == 1) return 1;
+	const bool tiles = up == 2 || up == 4 || up == 8 || up == 16;
+	return tiles && J == kFirJ && off % up == 0 ? up : 0;
+}
+
+// LDS bytes of the fused kernel for this frame (0 if it cannot run): the
+// transform, the echo, and the taps where the generic FIR runs.
 static size_t fused_lds_bytes(const FrameGeom& g, uint32_t J, uint32_t off)
 {
 	if (g.nf % 2 != 0) return 0;
@@ -1063,6 +1260,34 @@ static size_t fused_lds_bytes(const FrameGeom& g, uint32_t J, uint32_t off)
 	size_t b = static_cast<size_t>(M) * sizeof(float2);
 	if (g.up > 1) b += (static_cast<size_t>(J) + g.ns + off / g.up + 2 + static_cast<size_t>(g.up) * J) * sizeof(float);
 	return b <= 160 * 1024 - 512 ? b : 0;
+}
+
+// The fused kernel over n channels.  Lanes by the transform's size (18 values
+// a lane at most), so that short ones leave room for two to four workgroups on
+// a CU, whose barriers and memory phases then overlap.
+static void launch_analytic(const AnalyticArgs& A, uint32_t n, size_t lds, hipStream_t s)
+{
+	auto go = [&](auto kern, uint32_t nt) {
+		HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+				static_cast<int>(lds)));
+		hipLaunchKernelGGL(kern, dim3(n), dim3(nt), lds, s, A);
+		HIP_CHECK(hipGetLastError());
+	};
+	const uint32_t M = A.plan.M;
+	auto by_size = [&](auto up) {
+		constexpr int UP = decltype(up)::value;
+		if (M <= kFftPerLane * 256 && lds <= 53 * 1024) go(analytic_lds_kernel<256, UP>, 256);
+		else if (M <= kFftPerLane * 512 && lds <= 80 * 1024) go(analytic_lds_kernel<512, UP>, 512);
+		else go(analytic_lds_kernel<1024, UP>, 1024);
+	};
+	switch (fused_up(A.up, A.J, A.off)) {
+	case 1: by_size(std::integral_constant<int, 1>{}); break;
+	case 2: by_size(std::integral_constant<int, 2>{}); break;
+	case 4: by_size(std::integral_constant<int, 4>{}); break;
+	case 8: by_size(std::integral_constant<int, 8>{}); break;
+	case 16: by_size(std::integral_constant<int, 16>{}); break;
+	default: go(analytic_lds_kernel<1024, 0>, 1024); break;
+	}
 }
 
 // Radix plan (5s, one 8, 9s, a 6 or 3, 8s, 4, 2 in that order) and twiddles of
@@ -1094,6 +1319,8 @@ static void build_fused_plan(PrepPlan& P, uint32_t nf, hipStream_t s)
 	while (m % 2 == 0) { rad.push_back(2); m /= 2; }
 	if (m != 1 || rad.size() > static_cast<size_t>(kFftMaxPasses))
 		MISTA_THROW(MISTA_E_INVALID_PARAM, "FFT size " << nf << " is not 2-3-5 smooth");
+	if (rad.size() < 2 || (rad[0] != 5 && rad[0] != 8 && rad[0] != 9))   // (never: FFT sizes are at least 2048)
+		MISTA_THROW(MISTA_E_INVALID_STATE, "FFT size " << nf << " has no on-chip plan");
 	std::vector<float2> tw;
 	uint32_t Ns = 1;
 	for (size_t p = 0; p < rad.size(); ++p) {
@@ -1137,8 +1364,6 @@ static void prepare_fused(PrepState& st, const FrameGeom& g, const float* d_raw,
 	PrepPlan& P = *st.plan;
 	if (P.fused_nf != g.nf) build_fused_plan(P, g.nf, s);
 	const bool scaled = g.storage != MISTA_STORAGE_F32;
-	HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(analytic_lds_kernel),
-			hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
 	AnalyticArgs A{};
 	A.hpoly = d_filter_poly;
 	A.tw = P.tw.as<const float2>();
@@ -1166,8 +1391,7 @@ static void prepare_fused(PrepState& st, const FrameGeom& g, const float* d_raw,
 			A.out16 = nullptr;
 			A.scale = nullptr;
 		}
-		hipLaunchKernelGGL(analytic_lds_kernel, dim3(n), dim3(kFftThreads), lds, s, A);
-		HIP_CHECK(hipGetLastError());
+		launch_analytic(A, n, lds, s);
 	}
 }
 
@@ -1522,8 +1746,6 @@ void envelope_rows(PrepState& st, float* d_data, uint32_t n1, uint32_t n2, hipSt
 	PrepPlan& P = *st.plan;
 	if (P.fused_nf != g.nf) build_fused_plan(P, g.nf, s);
 	const uint32_t chunk = std::min<uint32_t>(n1, 1024u);
-	HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(analytic_lds_kernel),
-			hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
 	AnalyticArgs A{};
 	A.tw = P.tw.as<const float2>();
 	A.wpost = P.wpost.as<const float2>();
@@ -1540,8 +1762,7 @@ void envelope_rows(PrepState& st, float* d_data, uint32_t n1, uint32_t n2, hipSt
 		// in place: each sample is read (for the transform and again for the
 		// output) by the thread that later writes its magnitude
 		A.out_mag = d_data + static_cast<uint64_t>(r0) * n2;
-		hipLaunchKernelGGL(analytic_lds_kernel, dim3(n), dim3(kFftThreads), lds, s, A);
-		HIP_CHECK(hipGetLastError());
+		launch_analytic(A, n, lds, s);
 	}
 }
 
