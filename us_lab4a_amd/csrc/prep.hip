@@ -481,11 +481,15 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 		const float2* __restrict__ tw, uint32_t L, float& mx)
 {
 	constexpr int MAXB = static_cast<int>((kFftPerLane + R - 1) / R);
+	// opaque, so that the addresses of every radix's butterflies are formed
+	// here and not kept in registers around the loop over the passes
+	uint32_t tid = threadIdx.x;
+	asm volatile("" : "+v"(tid), "+s"(M));
 	const uint32_t nb = M / R;
 	float2 v[MAXB][R];
 #pragma unroll
 	for (int t = 0; t < MAXB; ++t) {
-		const uint32_t b = threadIdx.x + static_cast<uint32_t>(t) * NT;
+		const uint32_t b = tid + static_cast<uint32_t>(t) * NT;
 		if (b < nb) {
 #pragma unroll
 			for (int i = 0; i < R; ++i) v[t][i] = D[b + i * nb];
@@ -494,7 +498,7 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 	__syncthreads();
 #pragma unroll
 	for (int t = 0; t < MAXB; ++t) {
-		const uint32_t b = threadIdx.x + static_cast<uint32_t>(t) * NT;
+		const uint32_t b = tid + static_cast<uint32_t>(t) * NT;
 		if (b < nb) {
 			// q = b / Ns by a multiply-high: with magic = ceil(2^32 / Ns) =
 			// (2^32 + e) / Ns, b * magic / 2^32 = b / Ns + b e / (Ns 2^32),
@@ -688,9 +692,9 @@ template<int UP> struct MatFir {
 	static_assert(UP == 1 || 4 * STEPS - Q - 13 <= PADL, "the first column's oldest sample");
 	float a[STEPS];
 	int c0;   // echo index of this lane's first B entry at tile 0
-	__device__ explicit MatFir(const AnalyticArgs& A)
+	__device__ MatFir(const AnalyticArgs& A, uint32_t tid)
 	{
-		const int lane = static_cast<int>(threadIdx.x & 63), m = lane % 16, g = lane / 16;
+		const int lane = static_cast<int>(tid & 63), m = lane % 16, g = lane / 16;
 		if constexpr (UP > 1) {
 			// step entry s = 4 k + g holds tap j = s - (Q - 1) + dq and echo
 			// sample Q c + off/UP + Q - 1 - s
@@ -767,7 +771,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 	};
 	if constexpr (UP > 0) {
 		// the wave's outputs wait in registers for the mean
-		const MatFir<UP> fir(A);
+		const MatFir<UP> fir(A, tid);
 		if constexpr (UP > 1) {
 			constexpr int PADL = MatFir<UP>::PADL;
 			for (uint32_t i = tid; i < A.ns + PADL + MatFir<UP>::PADR; i += NT) {
@@ -911,7 +915,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 	if constexpr (UP > 0) {
 		// whole 16-byte stores where every row starts aligned
 		const bool vec = A.out16 ? (L & 3u) == 0 : (!mag && (L & 1u) == 0);
-		const MatFir<UP> fir(A);
+		const MatFir<UP> fir(A, tid);
 #pragma unroll 1
 		for (uint32_t t = wave; t < ntl; t += NW) {
 			const uint32_t i = 256 * t + in_tile;
@@ -948,7 +952,250 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 	}
 }
 
-// ---------------------------------------------------------------- long records
+// ---------------------------------------------------------------- long records on chip
+
+// Records whose half-size transform (M = N/2 values) no longer fits the LDS but
+// half of it does (H = M/2 <= kFftMaxM): the transforms by one split in time
+// and one in frequency around H-point transforms in LDS.
+//   z[2a], z[2a+1]   E = DFT_H(even), O = DFT_H(odd):
+//                    Z[k] = E[k] + w^k O[k], Z[k+H] = E[k] - w^k O[k], w = exp(-2 pi i / M)
+//   spectrum rule    on the bins k, M-k and H-k, H+k, which one lane forms
+//                    from E and O at k and H-k
+//   F = DFT_M(conj C)  F[2j] = DFT_H(G0)[j], F[2j+1] = DFT_H(G1)[j] with
+//                    G0[k] = C'[k] + C'[k+H], G1[k] = (C'[k] - C'[k+H]) w^k
+// A workgroup a channel, one after the other; what waits (the odd samples, E,
+// then G1 and F's even half) lies in a scratch of 2 H values a workgroup.
+// Against the four-step path, which moves every channel through memory seven
+// times, 192 x 192 channels of 8192 samples x 8 take 20 ms instead of 48.4 at
+// FP16 (a channel of 96 x 96, in us a workgroup: 139, of which the transforms
+// 35, the output 22, the spectrum 17, the rest the FIR and the 1.1 MB that pass
+// through the scratch).  Keeping only H values of scratch by forming the odd
+// samples again measured slower (159 us).
+struct LongArgs {
+	AnalyticArgs a;        // a.plan, a.tw: the H-point transforms
+	const float2* wm;      // exp(-2 pi i k / M), k <= H / 2
+	float2* scratch;       // [workgroups][2][H rounded up to even]
+	uint32_t nch;
+};
+constexpr uint32_t kPieceTiles = 64;   // FIR tiles whose echo is staged at a time for the output
+
+// conj(C) of the bins (k, M - k) from p = Z[k], q = Z[M - k], w = exp(-2 pi i k / N).
+__device__ __forceinline__ void spectrum_pair(float2& p, float2& q, float2 w)
+{
+	const float c = w.x, sn = -w.y;
+	const float2 ck = make_float2(fmaf(c, q.x, -sn * p.y), fmaf(sn, p.x, -c * q.y));
+	const float2 cm = make_float2(fmaf(-c, p.x, -sn * q.y), fmaf(sn, q.x, c * p.y));
+	p = conjf2(ck);
+	q = conjf2(cm);
+}
+
+template<int UP>
+__global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) analytic_long_kernel(const LongArgs B)
+{
+	extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+	constexpr int NT = kFftThreads;
+	constexpr uint32_t NW = NT / 64;
+	constexpr uint32_t TILES = 4 * kFftPerLane * NT / 256 / NW;
+	__shared__ double red[NW];
+	__shared__ float redm[NW];
+	const AnalyticArgs& A = B.a;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const uint32_t H = A.plan.M, np = A.plan.npass, L = A.L, ntl = (L + 255) / 256;
+	float2* D = reinterpret_cast<float2*>(lds);                                          // [H]
+	float* piece = reinterpret_cast<float*>(lds + static_cast<size_t>(H) * sizeof(float2));   // a piece of the echo
+	const uint32_t He = H + (H & 1u);   // (the halves stay 16-byte aligned)
+	float2* sa = B.scratch + static_cast<uint64_t>(blockIdx.x) * 2 * He;   // odd samples, then F's even half
+	float2* sb = sa + He;                                                  // E, then G1
+	const float coef = 2.0f / static_cast<float>(A.N);
+
+	for (uint32_t ch = blockIdx.x; ch < B.nch; ch += gridDim.x) {
+		// opaque, so that no address is kept in registers around the channels
+		uint32_t tid = threadIdx.x;
+		asm volatile("" : "+v"(tid));
+		const uint32_t lane = tid & 63, in_tile = 16 * (lane % 16) + 4 * (lane / 16);
+		const float* src = A.raw + static_cast<uint64_t>(ch) * A.ns;
+		double part = 0.0;
+		float mx = 0.0f, mean = 0.0f;   // largest |x - mean|
+		__syncthreads();   // the channel before is written out
+		{
+			const MatFir<UP> fir(A, tid);
+			f32x4 x[TILES];
+			const float* echo = src;
+			if constexpr (UP > 1) {
+				float* xs = reinterpret_cast<float*>(lds);   // the whole echo, before the transform needs the space
+				constexpr int PADL = MatFir<UP>::PADL;
+				for (uint32_t i = tid; i < A.ns + PADL + MatFir<UP>::PADR; i += NT) {
+					const int q = static_cast<int>(i) - PADL;
+					xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
+				}
+				__syncthreads();
+				echo = xs;
+			}
+			// (every tile of the wave, those past the record too: a branch
+			// around each would cost registers)
+#pragma unroll
+			for (uint32_t k = 0; k < TILES; ++k) {
+				const uint32_t i = 256 * (wave + k * NW) + in_tile;
+				x[k] = fir.tile(echo, A.ns, wave + k * NW);
+				const uint32_t i0 = 256 * (wave + k * NW);
+				if (i0 >= A.dz && i0 + 256 <= L) {
+#pragma unroll
+					for (int q = 0; q < 4; ++q) part += static_cast<double>(x[k][q]);
+				} else {
+#pragma unroll
+					for (uint32_t q = 0; q < 4; ++q)
+						if (i + q >= A.dz && i + q < L) part += static_cast<double>(x[k][q]);
+				}
+				__builtin_amdgcn_sched_barrier(0);   // one tile's operands at a time
+			}
+			for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
+			if (lane == 0) red[wave] = part;
+			__syncthreads();   // (also: the echo is read)
+			double sum = red[0];
+			for (uint32_t w = 1; w < NW; ++w) sum += red[w];
+			mean = static_cast<float>(sum / static_cast<double>(L - A.dz));
+#pragma unroll
+			for (uint32_t k = 0; k < TILES; ++k) {
+				const uint32_t t = wave + k * NW;
+				if (t >= ntl) continue;
+				const uint32_t i = 256 * t + in_tile;
+#pragma unroll
+				for (int q = 0; q < 4; ++q) {
+					x[k][q] = i + q < L ? x[k][q] - mean : 0.0f;
+					mx = fmaxf(mx, fabsf(x[k][q]));
+				}
+				D[i / 4] = make_float2(x[k][0], x[k][1]);
+				sa[i / 4] = make_float2(x[k][2], x[k][3]);
+			}
+			for (uint32_t c = 64 * ntl + tid; c < H; c += NT) D[c] = make_float2(0.0f, 0.0f);
+			__syncthreads();
+		}
+		float my = 0.0f;   // largest |re|, |im| of F over the first L samples (this lane's part)
+#pragma unroll 1
+		for (uint32_t stage = 0; stage < 4; ++stage) {
+			// D: the even samples, the odd samples, G0, G1
+			if (stage == 1) {
+				for (uint32_t c = tid; c < H; c += NT) D[c] = c < 64 * ntl ? sa[c] : make_float2(0.0f, 0.0f);
+			} else if (stage == 3) {
+				for (uint32_t c = tid; c < H; c += NT) D[c] = sb[c];
+			} else if (stage == 2) {
+				my = 0.0f;
+				for (uint32_t k = tid; k <= H / 2; k += NT) {
+					const uint32_t k2 = k == 0 ? 0u : H - k;
+					const float2 e1 = sb[k], e2 = sb[k2];
+					const float2 w1 = table_at(B.wm, k), w2 = make_float2(-w1.x, w1.y);   // w^k, w^(H-k)
+					const float2 t1 = cmul(w1, D[k]), t2 = cmul(w2, D[k2]);
+					float2 a = cadd(e1, t1), b = csub(e1, t1);     // Z[k], Z[k + H]
+					float2 c = cadd(e2, t2), d = csub(e2, t2);     // Z[H - k], Z[M - k]
+					if (k == 0) {
+						a = make_float2(0.0f, 0.0f);
+						b = make_float2(-b.y, -b.x);   // bin M/2: conj(i Z)
+						c = a;
+						d = b;
+					} else {
+						spectrum_pair(a, d, table_at(A.wpost, k));
+						spectrum_pair(c, b, table_at(A.wpost, H - k));
+						if (2 * k == H) c = a, d = b;   // its own partner: bins k and k + H alone
+					}
+					if (2 * k == H) b = d;
+					D[k] = cadd(a, b);
+					sb[k] = cmul(csub(a, b), w1);
+					if (k != 0 && 2 * k != H) {
+						D[k2] = cadd(c, d);
+						sb[k2] = cmul(csub(c, d), w2);
+					}
+				}
+			}
+			__syncthreads();
+			for (uint32_t p = 0; p + 1 < np; ++p) {
+#define MISTA_CALL(r) fft_pass<NT, r, false>(D, H, A.plan.ns[p], A.plan.ns_magic[p], A.tw + A.plan.tw_off[p], L, my)
+				MISTA_RADIX(A.plan.radix[p], MISTA_CALL)
+#undef MISTA_CALL
+			}
+			// (L / 2: half of the samples are in either half of F)
+#define MISTA_CALL(r) fft_pass<NT, r, true>(D, H, A.plan.ns[np - 1], A.plan.ns_magic[np - 1], A.tw + A.plan.tw_off[np - 1], L / 2, my)
+			MISTA_RADIX(A.plan.radix[np - 1], MISTA_CALL)
+#undef MISTA_CALL
+			if (stage == 0 || stage == 2) {
+				float2* out = stage == 0 ? sb : sa;
+				for (uint32_t c = tid; c < H; c += NT) out[c] = D[c];
+				__syncthreads();
+			}
+		}
+		float inv = 1.0f;
+		if (A.out16) {
+			float gm = fmaxf(my * coef, mx);
+			for (int o = 32; o > 0; o >>= 1) gm = fmaxf(gm, __shfl_xor(gm, o, 64));
+			if (lane == 0) redm[wave] = gm;
+			__syncthreads();
+			gm = redm[0];
+			for (uint32_t w = 1; w < NW; ++w) gm = fmaxf(gm, redm[w]);
+			const float sc = (gm > 0.0f) ? gm : 1.0f;
+			inv = 1.0f / sc;
+			if (tid == 0) A.scale[ch] = sc;
+		}
+		const bool bf = (A.flags & kOutBf16) != 0;
+		float2* dst = A.out + static_cast<uint64_t>(ch) * L;
+		uint32_t* row16 = A.out16 + static_cast<uint64_t>(ch) * L;
+		// x again, the echo a piece at a time beside the transform
+		const MatFir<UP> fir(A, tid);
+		constexpr int SPAN = static_cast<int>(kPieceTiles) * 256 / UP;   // a piece's input positions
+		constexpr uint32_t PER = kPieceTiles / NW;   // a wave's tiles of a piece
+		for (uint32_t t0 = 0; t0 < ntl; t0 += kPieceTiles) {
+			const float* echo = src;
+			// F's even half of the wave's tiles, in flight while the echo is staged
+			float2 f0[PER];
+#pragma unroll
+			for (uint32_t k = 0; k < PER; ++k) {
+				const uint32_t i = 256 * (t0 + wave + k * NW) + in_tile;
+				if (i < L) f0[k] = sa[i / 4];
+			}
+			if constexpr (UP > 1) {
+				constexpr int PADL = MatFir<UP>::PADL, COUNT = SPAN + PADL + MatFir<UP>::PADR;
+				const int shift = static_cast<int>(t0 / kPieceTiles) * SPAN;   // the piece's first input position
+				float e[(COUNT + NT - 1) / NT];
+#pragma unroll
+				for (int k = 0; k < (COUNT + NT - 1) / NT; ++k) {
+					const int q = shift + static_cast<int>(tid) + k * NT - PADL;
+					e[k] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
+				}
+				__syncthreads();   // the piece before is read
+#pragma unroll
+				for (int k = 0; k < (COUNT + NT - 1) / NT; ++k)
+					if (static_cast<int>(tid) + k * NT < COUNT) piece[tid + k * NT] = e[k];
+				__syncthreads();
+				echo = piece;
+			}
+#pragma unroll
+			for (uint32_t k = 0; k < PER; ++k) {
+				const uint32_t t = t0 + wave + k * NW;
+				if (t >= ntl) continue;
+				const uint32_t i = 256 * t + in_tile;
+				const f32x4 x = fir.tile(echo, UP > 1 ? static_cast<uint32_t>(SPAN) : A.ns, UP > 1 ? t - t0 : t);
+				if (i >= L) continue;   // (L is a multiple of 4)
+				const float2 f1 = D[i / 4];
+				const float re[4] = {x[0] - mean, x[1] - mean, x[2] - mean, x[3] - mean};
+				const float im[4] = {f0[k].x * coef, -f0[k].y * coef, f1.x * coef, -f1.y * coef};
+				if (A.out16) {
+					uint4 pk;
+					if (bf) {
+						pk = make_uint4(pack_bf16x2(re[0] * inv, im[0] * inv), pack_bf16x2(re[1] * inv, im[1] * inv),
+								pack_bf16x2(re[2] * inv, im[2] * inv), pack_bf16x2(re[3] * inv, im[3] * inv));
+					} else {
+						pk = make_uint4(pack_f16x2(re[0] * inv, im[0] * inv), pack_f16x2(re[1] * inv, im[1] * inv),
+								pack_f16x2(re[2] * inv, im[2] * inv), pack_f16x2(re[3] * inv, im[3] * inv));
+					}
+					*reinterpret_cast<uint4*>(row16 + i) = pk;
+				} else {
+					*reinterpret_cast<float4*>(dst + i) = make_float4(re[0], im[0], re[1], im[1]);
+					*reinterpret_cast<float4*>(dst + i + 2) = make_float4(re[2], im[2], re[3], im[3]);
+				}
+			}
+		}
+	}
+}
+
+// ---------------------------------------------------------------- long records through memory
 
 // Z = DFT_M(x[2m] + i x[2m+1]) -> conj(C) in place, the Hilbert spectrum of
 // the fused kernel (C[0] = 0, C[k] = i sin(2 pi k/N) Z[k] + cos(2 pi k/N)
@@ -1192,7 +1439,11 @@ struct PrepPlan {
 	uint32_t fused_nf = 0;
 	FftPlanArgs fplan{};
 	DeviceBuffer tw, wpost;
-	// four-step path (records too long for the fused kernel)
+	// long records on chip: the H-point plan and its tables, the waiting halves
+	uint32_t long_nf = 0;
+	FftPlanArgs lplan{};
+	DeviceBuffer ltw, lwm, lscratch;
+	// four-step path (records too long for the on-chip kernels)
 	Fft4Plan* f4 = nullptr;     // size Nf / 2
 	DeviceBuffer t4, wpost4;    // transpose buffer; exp(-2 pi i k / Nf), k <= Nf / 4
 	DeviceBuffer chmax;         // per channel of a round: max |x| (float), max |F| (float bits)
@@ -1215,7 +1466,8 @@ size_t prep_device_bytes(const PrepState& st)
 	const PrepPlan& P = *st.plan;
 	// the C2C plan's work area is taken as one more complex chunk
 	return P.real.capacity() + P.spec.capacity() + 2 * P.z.capacity() + P.tw.capacity() + P.wpost.capacity() +
-			P.t4.capacity() + P.wpost4.capacity() + P.chmax.capacity() + fft4_device_bytes(P.f4);
+			P.t4.capacity() + P.wpost4.capacity() + P.chmax.capacity() + P.ltw.capacity() + P.lwm.capacity() +
+			P.lscratch.capacity() + fft4_device_bytes(P.f4);
 }
 
 static void make_plans(hipfftHandle* r2c, hipfftHandle* c2c, uint32_t nf, uint32_t batch, hipStream_t s)
@@ -1292,9 +1544,8 @@ static void launch_analytic(const AnalyticArgs& A, uint32_t n, size_t lds, hipSt
 
 // Radix plan (5s, one 8, 9s, a 6 or 3, 8s, 4, 2 in that order) and twiddles of
 // the size-M transforms, computed in double and rounded once.
-static void build_fused_plan(PrepPlan& P, uint32_t nf, hipStream_t s)
+static FftPlanArgs lds_plan(uint32_t M, std::vector<float2>& tw)
 {
-	const uint32_t M = nf / 2;
 	FftPlanArgs F{};
 	F.M = M;
 	uint32_t m = M;
@@ -1318,10 +1569,9 @@ static void build_fused_plan(PrepPlan& P, uint32_t nf, hipStream_t s)
 	while (m % 4 == 0) { rad.push_back(4); m /= 4; }
 	while (m % 2 == 0) { rad.push_back(2); m /= 2; }
 	if (m != 1 || rad.size() > static_cast<size_t>(kFftMaxPasses))
-		MISTA_THROW(MISTA_E_INVALID_PARAM, "FFT size " << nf << " is not 2-3-5 smooth");
+		MISTA_THROW(MISTA_E_INVALID_PARAM, "FFT size " << M << " is not 2-3-5 smooth");
 	if (rad.size() < 2 || (rad[0] != 5 && rad[0] != 8 && rad[0] != 9))   // (never: FFT sizes are at least 2048)
-		MISTA_THROW(MISTA_E_INVALID_STATE, "FFT size " << nf << " has no on-chip plan");
-	std::vector<float2> tw;
+		MISTA_THROW(MISTA_E_INVALID_STATE, "FFT size " << M << " has no on-chip plan");
 	uint32_t Ns = 1;
 	for (size_t p = 0; p < rad.size(); ++p) {
 		const uint32_t R = rad[p];
@@ -1339,16 +1589,35 @@ static void build_fused_plan(PrepPlan& P, uint32_t nf, hipStream_t s)
 	}
 	F.npass = static_cast<uint32_t>(rad.size());
 	tw.push_back(make_float2(0.0f, 0.0f));   // keep the table non-empty
-	std::vector<float2> wp(M / 2 + 1);
-	for (uint32_t k = 0; k <= M / 2; ++k) {
-		const double a = -2.0 * M_PI * static_cast<double>(k) / static_cast<double>(nf);
-		wp[k] = make_float2(static_cast<float>(std::cos(a)), static_cast<float>(std::sin(a)));
+	return F;
+}
+
+// exp(-2 pi i k / n), k < count.
+static std::vector<float2> roots(uint32_t n, uint32_t count)
+{
+	std::vector<float2> w(count);
+	for (uint32_t k = 0; k < count; ++k) {
+		const double a = -2.0 * M_PI * static_cast<double>(k) / static_cast<double>(n);
+		w[k] = make_float2(static_cast<float>(std::cos(a)), static_cast<float>(std::sin(a)));
 	}
-	void* dt = P.tw.reserve(tw.size() * sizeof(float2));
-	void* dw = P.wpost.reserve(wp.size() * sizeof(float2));
-	HIP_CHECK(hipMemcpyAsync(dt, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice, s));
-	HIP_CHECK(hipMemcpyAsync(dw, wp.data(), wp.size() * sizeof(float2), hipMemcpyHostToDevice, s));
+	return w;
+}
+
+static void upload_table(DeviceBuffer& d, const std::vector<float2>& t, hipStream_t s)
+{
+	void* p = d.reserve(t.size() * sizeof(float2));
+	HIP_CHECK(hipMemcpyAsync(p, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice, s));
 	HIP_CHECK(hipStreamSynchronize(s));
+}
+
+static void build_fused_plan(PrepPlan& P, uint32_t nf, hipStream_t s)
+{
+	const uint32_t M = nf / 2;
+	std::vector<float2> tw;
+	const FftPlanArgs F = lds_plan(M, tw);
+	P.fused_nf = 0;
+	upload_table(P.tw, tw, s);
+	upload_table(P.wpost, roots(nf, M / 2 + 1), s);
 	P.fplan = F;
 	P.fused_nf = nf;
 }
@@ -1557,6 +1826,79 @@ static void launch_store(const FrameGeom& g, uint32_t n, const float2* z, void* 
 	HIP_CHECK(hipGetLastError());
 }
 
+// LDS bytes of the long-record kernel for this frame (0 if it cannot run): half
+// of the transform and a piece of the echo.
+static size_t long_lds_bytes(const FrameGeom& g, uint32_t J, uint32_t off)
+{
+	const uint32_t up = fused_up(g.up, J, off);
+	if (up == 0 || g.nf % 4 != 0 || g.nf / 4 > kFftMaxM || g.L % 4 != 0) return 0;
+	size_t b = static_cast<size_t>(g.nf / 4) * sizeof(float2);
+	if (up > 1) b += (static_cast<size_t>(kPieceTiles) * 256 / up + 64) * sizeof(float);
+	return b <= 160 * 1024 - 512 ? b : 0;
+}
+
+static void prepare_long(PrepState& st, const FrameGeom& g, const float* d_raw, const float* d_filter_poly, uint32_t J,
+		uint32_t off, void* d_tensor, float* d_scale, size_t lds, hipStream_t s)
+{
+	const uint32_t nch = g.ntx * g.nrx, M = g.nf / 2, H = M / 2;
+	if (!st.plan) st.plan = new PrepPlan();
+	PrepPlan& P = *st.plan;
+	if (P.long_nf != g.nf) {
+		std::vector<float2> tw;
+		const FftPlanArgs F = lds_plan(H, tw);
+		P.long_nf = 0;
+		upload_table(P.ltw, tw, s);
+		upload_table(P.lwm, roots(M, H / 2 + 1), s);
+		P.wpost4_nf = 0;
+		upload_table(P.wpost4, roots(g.nf, H + 1), s);
+		P.wpost4_nf = g.nf;
+		P.lplan = F;
+		P.long_nf = g.nf;
+	}
+	// a workgroup a CU, each with its own scratch
+	const uint32_t groups = std::min(nch, 256u);
+	LongArgs B{};
+	B.scratch = static_cast<float2*>(P.lscratch.reserve(static_cast<size_t>(groups) * 2 * (H + (H & 1u)) * sizeof(float2)));
+	B.wm = P.lwm.as<const float2>();
+	AnalyticArgs& A = B.a;
+	A.hpoly = d_filter_poly;
+	A.tw = P.ltw.as<const float2>();
+	A.wpost = P.wpost4.as<const float2>();
+	A.ns = g.ns;
+	A.up = g.up;
+	A.J = J;
+	A.off = off;
+	A.L = g.L;
+	A.N = g.nf;
+	A.dz = g.dz_up;
+	A.flags = kRemoveDc | (g.storage == MISTA_STORAGE_BF16 ? kOutBf16 : 0u);
+	A.plan = P.lplan;
+	const bool scaled = g.storage != MISTA_STORAGE_F32;
+	// 1024-channel chunks when the host uploads each chunk just in time
+	const uint32_t chunk = st.before_chunk ? std::min<uint32_t>(nch, 1024u) : nch;
+	for (uint32_t c0 = 0; c0 < nch; c0 += chunk) {
+		B.nch = std::min(chunk, nch - c0);
+		if (st.before_chunk) st.before_chunk(c0, B.nch);
+		A.raw = d_raw + static_cast<uint64_t>(c0) * g.ns;
+		A.out = scaled ? nullptr : static_cast<float2*>(d_tensor) + static_cast<uint64_t>(c0) * g.L;
+		A.out16 = scaled ? static_cast<uint32_t*>(d_tensor) + static_cast<uint64_t>(c0) * g.L : nullptr;
+		A.scale = scaled ? d_scale + c0 : nullptr;
+		auto go = [&](auto kern) {
+			HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+					static_cast<int>(lds)));
+			hipLaunchKernelGGL(kern, dim3(std::min(groups, B.nch)), dim3(kFftThreads), lds, s, B);
+			HIP_CHECK(hipGetLastError());
+		};
+		switch (fused_up(g.up, J, off)) {
+		case 1: go(analytic_long_kernel<1>); break;
+		case 2: go(analytic_long_kernel<2>); break;
+		case 4: go(analytic_long_kernel<4>); break;
+		case 8: go(analytic_long_kernel<8>); break;
+		default: go(analytic_long_kernel<16>); break;
+		}
+	}
+}
+
 // Records too long for the fused kernel: the fused kernel's algorithm with
 // its transforms of size M = Nf/2 as four-step FFTs through HBM (fft4.hip):
 // FIR x U + DC removal into x, Z = DFT_M(x as M complex pairs), the Hilbert
@@ -1628,13 +1970,8 @@ void prepare_signals(PrepState& st, const FrameGeom& g, const float* d_raw, cons
 		uint32_t J, uint32_t off, void* d_tensor, float* d_scale, hipStream_t s)
 {
 	const uint32_t nch = g.ntx * g.nrx;
-	if (st.method == 3) {
-		st.last_fused = false;
-		prepare_four_step(st, g, d_raw, d_filter_poly, J, off, d_tensor, d_scale, s);
-		return;
-	}
 	if (st.method != 1) {
-		const size_t lds = fused_lds_bytes(g, J, off);
+		const size_t lds = st.method == 3 ? 0 : fused_lds_bytes(g, J, off);
 		if (lds) {
 			prepare_fused(st, g, d_raw, d_filter_poly, J, off, d_tensor, d_scale, lds, s);
 			st.last_fused = true;
@@ -1642,7 +1979,11 @@ void prepare_signals(PrepState& st, const FrameGeom& g, const float* d_raw, cons
 		}
 		if (st.method == 2) MISTA_THROW(MISTA_E_INVALID_PARAM, "the fused preparation does not fit this frame (FFT size " << g.nf << ")");
 		st.last_fused = false;
-		prepare_four_step(st, g, d_raw, d_filter_poly, J, off, d_tensor, d_scale, s);
+		// long records: on chip by halves, beyond that (and for shorter ones
+		// that the fused kernel does not hold or was not asked for) through memory
+		const size_t long_lds = g.nf / 2 > kFftMaxM ? long_lds_bytes(g, J, off) : 0;
+		if (long_lds) prepare_long(st, g, d_raw, d_filter_poly, J, off, d_tensor, d_scale, long_lds, s);
+		else prepare_four_step(st, g, d_raw, d_filter_poly, J, off, d_tensor, d_scale, s);
 		return;
 	}
 	st.last_fused = false;
