@@ -140,30 +140,207 @@ __global__ void __launch_bounds__(256) das_rx_sums_kernel(const DasArgs a)
 	a.partial[static_cast<uint64_t>(r) * a.npix + p] = make_float2(ar, ai);
 }
 
+// The same sums with every record passing through LDS: a workgroup takes one
+// receive element and up to 1024 P pixels (lane: pixels pb 1024 P + k 1024 +
+// tid), and copies the receive element's records HBM -> LDS transmit after
+// transmit, each once, in `pieces` of at most half the LDS, so that one piece
+// is copied while the one before is used.  A position lies in exactly one piece
+// (consecutive pieces overlap by four entries), so the sums are the same fma
+// chains as above.
+struct RecordArgs {
+	uint32_t pieces, slots;   // pieces of a record, 1 KiB slots of a piece
+	uint32_t step;            // entries from one piece to the next
+	uint32_t npb;             // pixel blocks
+};
+constexpr uint32_t kRecordLanes = 1024;
+constexpr uint32_t kRecordLds = 160u * 1024u;
+
+template<int STORAGE, int P>
+__global__ void __launch_bounds__(kRecordLanes) das_record_sums_kernel(const DasArgs a, const RecordArgs R)
+{
+	using E = typename Entry<STORAGE>::T;
+	constexpr uint32_t ESZ = sizeof(E), NW = kRecordLanes / 64;
+	extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+	const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64);
+	// the pixel blocks of a receive element follow each other on one XCD and
+	// share its records through the L2
+	const uint32_t item = xcd_item(), r = item / R.npb, pb = item % R.npb;
+	const uint32_t buf_bytes = R.slots * 1024u;
+	const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) void*)smem));
+	const uint32_t voff = tid % 64 * 16;
+	const uint64_t chan_bytes = static_cast<uint64_t>(a.L) * ESZ;
+	const uint64_t p0 = static_cast<uint64_t>(pb) * (kRecordLanes * P) + tid;
+
+	float drx[P], dt[P], dnext[P], ar[P], ai[P];
+	uint64_t px[P];
+#pragma unroll
+	for (int k = 0; k < P; ++k) {
+		// lanes past the last pixel shadow it
+		const uint64_t p = p0 + static_cast<uint64_t>(k) * kRecordLanes;
+		px[k] = p < a.npix ? p : a.npix - 1;
+		drx[k] = a.delay[static_cast<uint64_t>(r) * a.npix + px[k]];
+		ar[k] = ai[k] = 0.0f;
+	}
+	auto load_delays = [&](uint32_t t) {
+		const float* row = a.delay + static_cast<uint64_t>(a.first_tx + t) * a.npix;
+#pragma unroll
+		for (int k = 0; k < P; ++k) dnext[k] = row[px[k]];
+	};
+	load_delays(0);
+
+	// Copy cursor: piece is_j of transmit is_t into buffer is_b.  Only the slots
+	// with entries up to index L; the last slot may reach past them (into the
+	// next channel, or the padding after the tensor).
+	uint32_t is_t = 0, is_j = 0, is_b = 0;
+	const unsigned char* chan = static_cast<const unsigned char*>(a.tensor) + r * chan_bytes;
+	auto issue = [&]() {
+		const uint32_t first = is_j * R.step;
+		const uint32_t need = ((a.L + 1u - first) * ESZ + 1023u) / 1024u, n = need < R.slots ? need : R.slots;
+		const uint32_t h = (n + NW - 1) / NW, s0 = wave * h;
+		uint32_t left = s0 < n ? (h < n - s0 ? h : n - s0) : 0u;
+		const unsigned char* src = chan + static_cast<uint64_t>(first) * ESZ + s0 * 1024u;
+		uint32_t dst = lds0 + is_b * buf_bytes + s0 * 1024u;
+		for (; left > 4; left -= 4, src += 4096, dst += 4096) lds_dma16_slots(src, voff, dst, 4);
+		lds_dma16_slots(src, voff, dst, left);
+		is_b ^= 1u;
+		if (++is_j == R.pieces) {
+			is_j = 0;
+			++is_t;
+			chan += chan_bytes * a.nrx;
+		}
+	};
+	issue();
+	uint32_t buf = 0;
+	for (uint32_t t = 0; t < a.ntx; ++t) {
+		const float w = a.weight(r, t);
+		for (uint32_t j = 0; j < R.pieces; ++j) {
+			// this piece and, with a transmit's first, its delays have arrived;
+			// every wave is done with the other buffer
+			MISTA_VMCNT(0);
+			if (j == 0) {
+#pragma unroll
+				for (int k = 0; k < P; ++k) {
+					asm volatile("" : "+v"(dnext[k]));
+					dt[k] = a.offset + dnext[k];
+				}
+			}
+			__syncthreads();
+			if (is_t < a.ntx) issue();
+			if (j == 0 && t + 1 < a.ntx) load_delays(t + 1);
+			const uint32_t first = j * R.step, end = j + 1 == R.pieces ? a.L - 1u : first + R.step;
+			const uint32_t lo = __float_as_uint(static_cast<float>(first)), span = __float_as_uint(static_cast<float>(end)) - lo;
+			const uint32_t base = lds0 + buf * buf_bytes;
+			constexpr int G = P < 4 ? P : 4;   // pixels whose LDS reads are in flight together
+#pragma unroll
+			for (int k0 = 0; k0 < P; k0 += G) {
+				uint32_t addr[G];
+				float kf[G];
+				bool ok[G];
+#pragma unroll
+				for (int q = 0; q < G; ++q) {
+					const float pos = dt[k0 + q] + drx[k0 + q];
+					// first <= pos < end by the bit patterns, in order for
+					// floats >= 0; negative values and NaN are above them
+					ok[q] = __float_as_uint(pos) - lo < span;
+					kf[q] = __builtin_amdgcn_fractf(pos);
+					addr[q] = ok[q] ? (static_cast<uint32_t>(pos) - first) * ESZ + base : base;
+				}
+				typename LdsPair<ESZ>::T v[G];
+				lds_read_pairs<ESZ, G>(addr, v);
+#pragma unroll
+				for (int q = 0; q < G; ++q) {
+					const float2 s = Entry<STORAGE>::lerp2(v[q], kf[q]);
+					const float nr = fmaf(s.x, w, ar[k0 + q]);
+					ar[k0 + q] = ok[q] ? nr : ar[k0 + q];
+					if constexpr (STORAGE != kStorageReal) {
+						const float ni = fmaf(s.y, w, ai[k0 + q]);
+						ai[k0 + q] = ok[q] ? ni : ai[k0 + q];
+					}
+				}
+			}
+			buf ^= 1u;
+		}
+	}
+#pragma unroll
+	for (int k = 0; k < P; ++k) {
+		const uint64_t p = p0 + static_cast<uint64_t>(k) * kRecordLanes;
+		if (p < a.npix) a.partial[static_cast<uint64_t>(r) * a.npix + p] = make_float2(ar[k], ai[k]);
+	}
+}
+
 // A lane per pixel: the per-rx sums in rx order through the same statistics
 // as both other kernels (so the images equal the tiled kernel's).
 template<int CF>
-__global__ void __launch_bounds__(256) das_rx_stats_kernel(const DasArgs a)
+__global__ void __launch_bounds__(64) das_rx_stats_kernel(const DasArgs a)
 {
 	const uint64_t p = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
 	if (p >= a.npix) return;
 	PixelStats<CF> st;
-	for (uint32_t r = 0; r < a.nrx; ++r) {
-		const float2 v = a.partial[static_cast<uint64_t>(r) * a.npix + p];
+	const float2* src = a.partial + p;
+	uint32_t r = 0;
+	for (; r + 16 <= a.nrx; r += 16) {   // loads in flight: few lanes share the chip
+		float2 v[16];
+#pragma unroll
+		for (uint32_t k = 0; k < 16; ++k) v[k] = src[(r + k) * a.npix];
+#pragma unroll
+		for (uint32_t k = 0; k < 16; ++k) st.add_rx(v[k].x, v[k].y, r + k == 0);
+	}
+	for (; r < a.nrx; ++r) {
+		const float2 v = src[r * a.npix];
 		st.add_rx(v.x, v.y, r == 0);
 	}
 	st.write(a, p);
 }
 
+// Record form: pixels a lane (P) and pixel blocks, pieces of a record.  Not
+// where a pixel's own cache lines are less than the record (few pixels), nor
+// where a record takes more than 8 pieces, which every pixel passes.
+bool record_plan(const FrameGeom& g, RecordArgs& R, uint32_t& p)
+{
+	constexpr uint32_t kMaxP = 12;
+	const uint64_t bytes = (static_cast<uint64_t>(g.L) + 1u) * storage_bytes(g.storage);
+	const uint64_t blocks = (g.npix + kRecordLanes - 1) / kRecordLanes;
+	const uint64_t npb = std::max<uint64_t>((blocks + kMaxP - 1) / kMaxP, std::min<uint64_t>(blocks, 256u / std::min(g.nrx, 256u)));
+	const uint32_t cap = kRecordLds / 2048u - 1u;   // slots of the largest piece
+	const uint64_t pieces = (bytes + cap * 1024u - 33u) / (cap * 1024u - 32u);
+	if (pieces > 8 || npb * bytes > g.npix * 64u || npb * g.nrx >= (1ull << 31)) return false;
+	R.npb = static_cast<uint32_t>(npb);
+	R.pieces = static_cast<uint32_t>(pieces);
+	R.slots = static_cast<uint32_t>((bytes + pieces - 1) / pieces + 32u + 1023u) / 1024u;
+	R.step = R.slots * 1024u / static_cast<uint32_t>(storage_bytes(g.storage)) - 4u;
+	p = static_cast<uint32_t>((blocks + npb - 1) / npb);
+	return true;
+}
+
+template<int STORAGE>
+void launch_record(const FrameGeom& g, const DasArgs& a, const RecordArgs& R, uint32_t p, hipStream_t s)
+{
+	const uint32_t lds = 2u * R.slots * 1024u;
+	auto go = [&](auto kern) {
+		HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+				static_cast<int>(lds)));
+		hipLaunchKernelGGL(kern, dim3(g.nrx * R.npb), dim3(kRecordLanes), lds, s, a, R);
+	};
+	if (p <= 1) go(das_record_sums_kernel<STORAGE, 1>);
+	else if (p <= 2) go(das_record_sums_kernel<STORAGE, 2>);
+	else if (p <= 4) go(das_record_sums_kernel<STORAGE, 4>);
+	else if (p <= 8) go(das_record_sums_kernel<STORAGE, 8>);
+	else go(das_record_sums_kernel<STORAGE, 12>);
+}
+
 template<int STORAGE>
 void launch_rx_parallel(const FrameGeom& g, const DasArgs& a, hipStream_t s)
 {
-	const uint32_t nb = static_cast<uint32_t>((g.npix + 255) / 256);
-	hipLaunchKernelGGL(das_rx_sums_kernel<STORAGE>, dim3(nb, g.nrx), dim3(256), 0, s, a);
+	const uint32_t nb = static_cast<uint32_t>((g.npix + 255) / 256), ns = static_cast<uint32_t>((g.npix + 63) / 64);
+	RecordArgs R;
+	uint32_t p = 0;
+	if (record_plan(g, R, p)) launch_record<STORAGE>(g, a, R, p, s);
+	else hipLaunchKernelGGL(das_rx_sums_kernel<STORAGE>, dim3(nb, g.nrx), dim3(256), 0, s, a);
+	HIP_CHECK(hipGetLastError());
 	switch (g.cf_kind) {
-	case MISTA_CF_NONE: hipLaunchKernelGGL(das_rx_stats_kernel<MISTA_CF_NONE>, dim3(nb), dim3(256), 0, s, a); break;
-	case MISTA_CF_PCF: hipLaunchKernelGGL(das_rx_stats_kernel<MISTA_CF_PCF>, dim3(nb), dim3(256), 0, s, a); break;
-	default: hipLaunchKernelGGL(das_rx_stats_kernel<MISTA_CF_SCF>, dim3(nb), dim3(256), 0, s, a); break;
+	case MISTA_CF_NONE: hipLaunchKernelGGL(das_rx_stats_kernel<MISTA_CF_NONE>, dim3(ns), dim3(64), 0, s, a); break;
+	case MISTA_CF_PCF: hipLaunchKernelGGL(das_rx_stats_kernel<MISTA_CF_PCF>, dim3(ns), dim3(64), 0, s, a); break;
+	default: hipLaunchKernelGGL(das_rx_stats_kernel<MISTA_CF_SCF>, dim3(ns), dim3(64), 0, s, a); break;
 	}
 }
 
