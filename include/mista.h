@@ -233,7 +233,8 @@ int mista_query(const mista_handle* h, uint32_t* signal_length, uint32_t* fft_si
  * one-pixel-per-lane gather, 2 = LDS-tiled).  Tile parameters 0 = default;
  * tile_param1 = pairs per transmit step (the receive elements of a
  * workgroup: 4, 8, or 16 on 512-point tiles) | ring buffers << 8 | LDS budget
- * in KiB << 16.  Where the
+ * in KiB << 16 | on 2048-point tiles 1 << 24 (1024 lanes) or 2 << 24 (1024
+ * lanes, chunks of two receive elements).  Where the
  * variant's tiles do not fit, the rx-parallel form runs instead. */
 int mista_set_kernel(mista_handle* h, int variant, int tile_param0, int tile_param1);
 
@@ -257,7 +258,7 @@ int mista_tuned_kernel(const mista_handle* h, int* tile_param0, int* tile_param1
 
 /* The configuration of the last DAS launch: tile shape (-1 when the gather
  * kernel ran, -2 the rx-parallel form that runs where no tile fits: per-rx
- * sums a lane per (pixel, rx), then the statistics a lane per pixel) and
+ * sums by record or a lane per (pixel, rx), then the statistics a lane per pixel) and
  * pairs per transmit step | ring buffers << 8 | LDS budget in KiB << 16.  No
  * counterpart in the reference. */
 int mista_last_kernel(const mista_handle* h, int* tile_param0, int* tile_param1);

@@ -12,9 +12,11 @@
 // Kernels:
 //  das_gather_kernel  one pixel per lane, global gathers (reference shape;
 //                     the explicit gather variant).
-//  das_rx_sums_kernel + das_rx_stats_kernel  the fallback where no tile
-//                     fits: a lane per (pixel, rx) sums over the transmits,
-//                     then a lane per pixel folds the per-rx sums in rx order.
+//  das_record_sums_kernel / das_rx_sums_kernel + das_rx_stats_kernel  the
+//                     fallback where no tile fits: per (pixel, rx) the sum over
+//                     the transmits, from whole records passing through LDS or,
+//                     for few pixels, by gathers; then a lane per pixel folds
+//                     the per-rx sums in rx order.
 //  das_tile_kernel + das_tile_stats_kernel  the tiled form: a workgroup forms
 //                     the per-rx sums of a tile of pixels for a few receive
 //                     elements; for every (rx, tx) pair the tile's signal
@@ -35,10 +37,10 @@
 namespace mista {
 
 namespace das {
-extern template void launch_tile_storage<MISTA_STORAGE_F32>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
-extern template void launch_tile_storage<MISTA_STORAGE_F16>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
-extern template void launch_tile_storage<MISTA_STORAGE_BF16>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
-extern template void launch_tile_storage<kStorageReal>(const TileBatch&, uint32_t, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<MISTA_STORAGE_F32>(const TileBatch&, uint32_t, uint32_t, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<MISTA_STORAGE_F16>(const TileBatch&, uint32_t, uint32_t, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<MISTA_STORAGE_BF16>(const TileBatch&, uint32_t, uint32_t, uint32_t, uint32_t, hipStream_t);
+extern template void launch_tile_storage<kStorageReal>(const TileBatch&, uint32_t, uint32_t, uint32_t, uint32_t, hipStream_t);
 }  // namespace das
 
 using namespace das;
@@ -146,7 +148,9 @@ __global__ void __launch_bounds__(256) das_rx_sums_kernel(const DasArgs a)
 // transmit, each once, in `pieces` of at most half the LDS, so that one piece
 // is copied while the one before is used.  A position lies in exactly one piece
 // (consecutive pieces overlap by four entries), so the sums are the same fma
-// chains as above.
+// chains as above.  Bound by reading the tensor once per pixel block: the gather
+// form moves a 128-byte line for the 8 or 16 bytes of a pair (192 elements, 96 x
+// 96 points, 32 768 FP16 samples: 4.81 ms; this 0.94, 5.1 TB/s).
 struct RecordArgs {
 	uint32_t pieces, slots;   // pieces of a record, 1 KiB slots of a piece
 	uint32_t step;            // entries from one piece to the next
@@ -292,18 +296,21 @@ __global__ void __launch_bounds__(64) das_rx_stats_kernel(const DasArgs a)
 	st.write(a, p);
 }
 
-// Record form: pixels a lane (P) and pixel blocks, pieces of a record.  Not
-// where a pixel's own cache lines are less than the record (few pixels), nor
-// where a record takes more than 8 pieces, which every pixel passes.
+// Record form: pixels a lane (p) and pixel blocks, pieces of a record.  Up to 256
+// workgroups, a CU each, as long as the records' bytes (each block copies all of
+// them) stay below 64 for each pixel, half a cache line of the gather form, and 12
+// pixels a lane.  Not where one block passes that (few pixels), nor where a record
+// takes more than 8 pieces, which every pixel passes.
 bool record_plan(const FrameGeom& g, RecordArgs& R, uint32_t& p)
 {
 	constexpr uint32_t kMaxP = 12;
 	const uint64_t bytes = (static_cast<uint64_t>(g.L) + 1u) * storage_bytes(g.storage);
-	const uint64_t blocks = (g.npix + kRecordLanes - 1) / kRecordLanes;
-	const uint64_t npb = std::max<uint64_t>((blocks + kMaxP - 1) / kMaxP, std::min<uint64_t>(blocks, 256u / std::min(g.nrx, 256u)));
+	const uint64_t blocks = (g.npix + kRecordLanes - 1) / kRecordLanes, few = (blocks + kMaxP - 1) / kMaxP;
+	const uint64_t most = g.npix * 64u / bytes;   // blocks whose records are that many bytes
+	const uint64_t npb = std::max(few, std::min({blocks, static_cast<uint64_t>(256u / std::min(g.nrx, 256u)), most}));
 	const uint32_t cap = kRecordLds / 2048u - 1u;   // slots of the largest piece
 	const uint64_t pieces = (bytes + cap * 1024u - 33u) / (cap * 1024u - 32u);
-	if (pieces > 8 || npb * bytes > g.npix * 64u || npb * g.nrx >= (1ull << 31)) return false;
+	if (pieces > 8 || npb > most || npb * g.nrx >= (1ull << 31)) return false;
 	R.npb = static_cast<uint32_t>(npb);
 	R.pieces = static_cast<uint32_t>(pieces);
 	R.slots = static_cast<uint32_t>((bytes + pieces - 1) / pieces + 32u + 1023u) / 1024u;
@@ -595,6 +602,7 @@ uint32_t read_u32(const uint32_t* d, hipStream_t s)
 struct Chunking {
 	uint32_t r = 0;       // receive elements per workgroup: pairs per transmit step
 	uint32_t nt = 0;      // lanes
+	uint32_t rc = 0;      // receive elements per chunk
 	uint32_t nbmax = 0;   // most chunk buffers
 	uint32_t lds = 0;     // LDS bytes
 	uint32_t nbuf = 0;    // chunk buffers of the tile with the longest window
@@ -605,32 +613,39 @@ struct Chunking {
 // pairs per transmit step (4, 8, or 16 on 512-point tiles), byte 1 most chunk
 // buffers, byte 2 LDS budget in KiB (default: the smallest in which two
 // buffers of the longest window fit, of those that put 4, 3, 2 or 1
-// workgroups on a CU).  Returns false when nothing fits.
+// workgroups on a CU; LDS is handed out in 1280-byte blocks, of which 52 KiB
+// take a third and 53 KiB more), byte 3 for 2048-point tiles: 1 = 1024 lanes in
+// any budget, 2 = the same with chunks of two receive elements.  Returns false
+// when nothing fits.
 bool choose_chunking(uint32_t npts, int p1, uint32_t S, Chunking& c)
 {
 	if (S > kMaxSlots) return false;
 	const uint32_t want_r = static_cast<uint32_t>(p1) & 0xFF, want_nb = (static_cast<uint32_t>(p1) >> 8) & 0xFF;
 	const uint32_t want_kb = (static_cast<uint32_t>(p1) >> 16) & 0xFF;
+	const uint32_t wide = npts == 2048u ? static_cast<uint32_t>(p1) >> 24 & 3u : 0u;
 	c.nbmax = want_nb ? std::max(2u, std::min(want_nb, 4u)) : 4u;
-	for (uint32_t kb : {40u, 53u, 80u, 160u}) {
+	for (uint32_t kb : {40u, 52u, 80u, 160u}) {
 		if (want_kb) {
 			if (kb != 40u) break;
 			kb = std::min(want_kb, 160u);
 		}
-		// lanes per workgroup; no more workgroups than the CU's registers hold
-		c.nt = npts <= 512 ? 256u : npts == 1024 ? 512u : kb <= 80u ? 512u : 1024u;
-		if (!want_kb && c.nt == 512u && kb < 80u) continue;
+		c.nt = npts <= 512 ? 256u : npts == 1024 ? 512u : kb <= 80u && !wide ? 512u : 1024u;
+		// (2048 points: two workgroups a CU at most)
+		if (!want_kb && npts == 2048u && kb < 80u) continue;
 		c.lds = kb * 1024u;
 		for (uint32_t r : {4u, 8u, 16u}) {
 			if (want_r ? r != want_r : r == 16u) continue;
-			if ((r == 16u && npts != 512u) || (r == 8u && (npts == 256u || (npts == 2048u && c.nt == 512u)))) continue;
-			const uint32_t rc = npts == 2048u && c.nt == 512u ? 2u : 4u;
+			if ((r == 16u && npts != 512u) || (r == 8u && (npts == 256u || (npts == 2048u && (c.nt == 512u || wide == 2u))))) continue;
+			const uint32_t rc = npts == 2048u && (c.nt == 512u || wide == 2u) ? 2u : 4u;
 			c.r = r;
+			c.rc = rc;
 			if (r == 16u) c.nt = 512u;
 			c.nbuf = tile_buffers(c.nbmax, c.lds, S, rc, r / rc, npts);
 			if (c.nbuf) return true;
 		}
 	}
+	// long windows on 2048 points: chunks of two receive elements in the whole LDS
+	if (npts == 2048u && p1 == 0) return choose_chunking(npts, 4 | (160 << 16) | (2 << 24), S, c);
 	return false;
 }
 
@@ -658,10 +673,10 @@ TileArgs tile_args(const FrameGeom& g, const DasArgs& a, uint32_t ntiles, const 
 void launch_batch(int storage, const TileBatch& B, uint32_t npts, const Chunking& c, hipStream_t s)
 {
 	switch (storage) {
-	case MISTA_STORAGE_F32: launch_tile_storage<MISTA_STORAGE_F32>(B, npts, c.r, c.nt, s); break;
-	case MISTA_STORAGE_F16: launch_tile_storage<MISTA_STORAGE_F16>(B, npts, c.r, c.nt, s); break;
-	case kStorageReal: launch_tile_storage<kStorageReal>(B, npts, c.r, c.nt, s); break;
-	default: launch_tile_storage<MISTA_STORAGE_BF16>(B, npts, c.r, c.nt, s); break;
+	case MISTA_STORAGE_F32: launch_tile_storage<MISTA_STORAGE_F32>(B, npts, c.r, c.rc, c.nt, s); break;
+	case MISTA_STORAGE_F16: launch_tile_storage<MISTA_STORAGE_F16>(B, npts, c.r, c.rc, c.nt, s); break;
+	case kStorageReal: launch_tile_storage<kStorageReal>(B, npts, c.r, c.rc, c.nt, s); break;
+	default: launch_tile_storage<MISTA_STORAGE_BF16>(B, npts, c.r, c.rc, c.nt, s); break;
 	}
 	HIP_CHECK(hipGetLastError());
 }
@@ -1081,10 +1096,23 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 					// a try, then the smallest budget that fits; a long frame
 					// takes that alone
 					std::vector<int> cands;
-					if (!long_frame && npts == 2048) cands = {4 | (80 << 16), 8 | (160 << 16)};
-					else if (!long_frame && npts == 512) cands = {4 | (52 << 16), 8 | (52 << 16)};
-					if (npts != 2048 || long_frame) cands.push_back(0);
+					// 2048 points: 512 lanes with two workgroups a CU,
+					// 1024 lanes with two (4-byte entries: short windows,
+					// 100-element BF16 frame 0.66 -> 0.55 ms; 8-byte ones in
+					// chunks of two receive elements: 128-element frame 5.76
+					// -> 5.54 ms) or one; where none of them fits, the chunks
+					// of two in the whole LDS (192 elements of 65 536 samples
+					// 4.14 ms against 5.05 at 32x32).  1024 points: three
+					// workgroups a CU where they fit (128-element F16 frame
+					// 3.96 -> 3.55 ms, RF 1.03 -> 0.86), else two.
+					const int wide = g.storage == MISTA_STORAGE_F32 ? 2 << 24 : 1 << 24;
+					if (!long_frame && npts == 2048) cands = {4 | (80 << 16), 4 | (80 << 16) | wide, 8 | (160 << 16)};
+					else if (!long_frame && npts == 1024) cands = {4 | (80 << 16)};
+					else if (!long_frame && npts == 512) cands = {8 | (52 << 16)};
+					cands.push_back(0);
+					bool any = false;
 					for (const int p1 : cands) {
+						if (p1 == 0 && npts == 2048 && any) break;
 						// the better of two runs (the first may find cold caches)
 						float ms = 0.0f;
 						bool run = false;
@@ -1094,6 +1122,7 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 							ms = rep == 0 ? t : std::min(ms, t);
 							if (!run || t > kTuneLimitMs) break;
 						}
+						any = any || run;
 						if (run && (bp0 < 0 || ms < best)) {
 							best = ms;
 							bp0 = p0;

@@ -195,11 +195,14 @@ struct PixelStats {
 
 // Tile geometry: a tw1 (x) by tw2 (y) by tzh (z) block of grid points, one
 // point per lane.  A plane has ny = tw2 = 1; a volume is laid out as
-// n1 = nx * ny columns (y fastest) by n2 = nz rows.  In a plane tile each wave
-// takes an 8 x 8 block of points (x fastest within the block): the lanes of
-// one LDS read pass then sit close together in both directions, which spreads
-// their window entries over more banks than a 16 x 4 strip.  Volume tiles
-// keep x fastest, then y, then z.  Tiles are numbered depth-band major (all
+// n1 = nx * ny columns (y fastest) by n2 = nz rows.  Each wave takes a compact
+// block of points, x fastest: 8 x 8 of a plane tile, 4 x 4 x 4 of a volume tile
+// (every tile is whole blocks).  An LDS read of two 8-byte entries takes 16
+// lanes a clock over 32 banks (4-byte entries: 32 lanes), and of the blocks
+// measured these collide least: a plane's 16 lanes 8 x 2 wait 10.4 clocks a
+// read, 4 x 4 11.3, 16 x 1 12.5, 1 x 16 14.4; a volume's 4 x 4 x 1 3.9, 8 x 2
+// 5.9, 16 x 1 5.9 to 9.4 (1024 x 64 volume, DAS 17.6 -> 15.6 ms against
+// lanes of 16 x 4 x 1, with 1024-point tiles).  Tiles are numbered depth-band major (all
 // tiles of a band of tzh rows are consecutive), so the workgroups resident
 // at one time cover a depth band and share signal windows through L2/MALL.
 struct TileGeom {
@@ -212,15 +215,17 @@ struct TileGeom {
 		const uint32_t tz = tile / per_band, rem = tile % per_band;
 		const uint32_t tx = rem / tiles_y, ty = rem % tiles_y;
 		uint32_t lx, ly, lz;
-		if (tw2 == 1 && tw1 % 8 == 0 && tzh % 8 == 0) {
-			const uint32_t blk = lane_id / 64, l = lane_id % 64, bx = tw1 / 8;
+		const uint32_t blk = lane_id / 64, l = lane_id % 64;
+		if (tw2 == 1) {
+			const uint32_t bx = tw1 / 8;
 			lx = (blk % bx) * 8 + l % 8;
 			lz = (blk / bx) * 8 + l / 8;
 			ly = 0;
 		} else {
-			lx = lane_id % tw1;
-			ly = (lane_id / tw1) % tw2;
-			lz = lane_id / (tw1 * tw2);
+			const uint32_t bx = tw1 / 4, by = tw2 / 4;
+			lx = (blk % bx) * 4 + l % 4;
+			ly = (blk / bx % by) * 4 + l / 4 % 4;
+			lz = (blk / (bx * by)) * 4 + l / 16;
 		}
 		const uint32_t ix = tx * tw1 + lx, iy = ty * tw2 + ly, iz = tz * tzh + lz;
 		valid = ix < nx && iy < ny && iz < n2;
@@ -247,8 +252,6 @@ constexpr uint32_t kWsMask = (1u << 24) - 1u;
 constexpr uint32_t kSlotShift = 24;
 constexpr uint32_t kMaxWindowL = 1u << 21;   // records up to here: every ws * ESZ fits the word
 
-typedef __attribute__((address_space(1))) const void* gptr_t;
-typedef __attribute__((address_space(3))) void* lptr_t;
 // Read-only tables (window words, weights) through the constant address
 // space: uniform indices then become scalar loads.
 typedef __attribute__((address_space(4))) const uint32_t* cu32_t;
@@ -655,7 +658,7 @@ __device__ __forceinline__ uint32_t xcd_item()
 // One frame: its arguments arrive as the kernel's own, which the compiler
 // keeps in scalar registers.
 template<int STORAGE, int NT, int P, int RC, int H>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8)))
 das_tile_kernel(const TileArgs A)
 {
 	extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -668,7 +671,7 @@ das_tile_kernel(const TileArgs A)
 // balance by themselves.  (A separate kernel: a frame's arguments picked from
 // the table by a run-time index are reloaded from memory at their uses.)
 template<int STORAGE, int NT, int P, int RC, int H>
-__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 8)))
 das_tile_batch_kernel(const TileBatch B)
 {
 	extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -694,7 +697,7 @@ void launch_tile_t(const TileBatch& B, hipStream_t s)
 
 // Tiled launch for one storage kind (instantiated in das_tile_<storage>.hip).
 template<int STORAGE>
-void launch_tile_storage(const TileBatch& B, uint32_t npts, uint32_t r, uint32_t nt, hipStream_t s)
+void launch_tile_storage(const TileBatch& B, uint32_t npts, uint32_t r, uint32_t rc, uint32_t nt, hipStream_t s)
 {
 	if (npts == 256) launch_tile_t<STORAGE, 256, 1, 4, 1>(B, s);
 	else if (npts == 512 && r == 16) launch_tile_t<STORAGE, 512, 1, 4, 4>(B, s);
@@ -703,6 +706,7 @@ void launch_tile_storage(const TileBatch& B, uint32_t npts, uint32_t r, uint32_t
 	else if (npts == 1024 && r == 8) launch_tile_t<STORAGE, 512, 2, 4, 2>(B, s);
 	else if (npts == 1024) launch_tile_t<STORAGE, 512, 2, 4, 1>(B, s);
 	else if (nt == 512) launch_tile_t<STORAGE, 512, 4, 2, 2>(B, s);
+	else if (rc == 2) launch_tile_t<STORAGE, 1024, 2, 2, 2>(B, s);
 	else if (r == 8) launch_tile_t<STORAGE, 1024, 2, 4, 2>(B, s);
 	else launch_tile_t<STORAGE, 1024, 2, 4, 1>(B, s);
 }
