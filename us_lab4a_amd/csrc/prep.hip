@@ -293,16 +293,20 @@ __device__ inline uint32_t pack_f16x2(float re, float im)
 // inputs into registers, a barrier, then writes the outputs in place.
 //
 // Bounds, 128 x 128 channels of 4096 samples x 8 (M = 17 280; one workgroup a
-// CU, its 138 KB of transform): the ten passes 1.56 ms (LDS in and out, then
-// arithmetic, a barrier between: with one workgroup nothing fills the other's
-// phase), FIR, mean and output 1.2 ms at FP16, 1.45 at FP32, of which writing
-// the tensor is 0.5 / 0.95.  With both FIR evaluations as vector arithmetic
+// CU, its 138 KB of transform): of a channel's 98 600 cycles (F16) the ten
+// passes take 55 800, echo load, FIR and mean 26 000, the output with its second
+// FIR 13 700 (F32 23 400).  The passes are paced by LDS traffic, latency and
+// barriers: without their arithmetic the kernel takes 2.31 of 2.63 ms, without
+// their twiddle loads 2.54.  With both FIR evaluations as vector arithmetic
 // (27 fma an output, twice) and the spectrum rule and the scale as passes of
-// their own the kernel took 3.82 ms at FP32 and 3.29 at FP16; now 2.98 and
-// 2.77 (64 x 64 channels of 2048 x 8, two workgroups a CU: 0.54 -> 0.37).
+// their own the kernel took 3.82 ms at FP32 and 3.29 at FP16; now 2.86 and
+// 2.66 (64 x 64 channels of 2048 x 8, two workgroups a CU: 0.54 -> 0.35; 64 x
+// 1024 of 2048 x 4: 5.5 -> 2.34).  Taking the largest |F| from the outputs'
+// registers instead of inside the last pass gave the last 2 to 4 %.
 // Measured slower: twiddles loaded ahead of a pass's barrier (3.0 to 3.5 ms
 // at FP16), twiddles in [i][j] order (3.44), the FIR's echo operand straight
-// from memory (3.9).
+// from memory (3.9), the FIR's outputs kept in registers through the
+// transforms (12 registers spill: F32 2.98 -> 3.1).
 
 constexpr int kFftThreads = 1024;
 constexpr uint32_t kFirJ = 27;   // taps per phase of the Kaiser upsampling design (every U)
@@ -473,12 +477,20 @@ __device__ __forceinline__ float2 table_at(const float2* __restrict__ base, uint
 	return *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(base) + i * static_cast<uint32_t>(sizeof(float2)));
 }
 
+// mx = max(mx, |v.x|, |v.y|), a NaN ignored (fmaxf's canonicalising forms take
+// four instructions).
+__device__ __forceinline__ void max_abs(float& mx, float2 v)
+{
+	asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(mx) : "v"(v.x), "v"(v.y));
+}
+
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) f32x2* lds_c64_t;
+
 // One Stockham pass over D in place: every lane reads its butterflies' inputs,
-// a barrier, then the outputs.  MAX: also the largest |re|, |im| of the outputs
-// with index below npair (and |re| at npair when odd).
-template<int NT, int R, bool MAX>
-__device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uint32_t magic,
-		const float2* __restrict__ tw, uint32_t L, float& mx)
+// a barrier, then the outputs.
+template<int NT, int R>
+__device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uint32_t magic, const float2* __restrict__ tw)
 {
 	constexpr int MAXB = static_cast<int>((kFftPerLane + R - 1) / R);
 	// opaque, so that the addresses of every radix's butterflies are formed
@@ -486,13 +498,19 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 	uint32_t tid = threadIdx.x;
 	asm volatile("" : "+v"(tid), "+s"(M));
 	const uint32_t nb = M / R;
-	float2 v[MAXB][R];
+	// LDS addresses formed once, from a base the compiler does not see through:
+	// the butterflies of a lane then differ by immediate offsets
+	const uint32_t d0 = static_cast<uint32_t>(reinterpret_cast<size_t>((__attribute__((address_space(3))) float2*)D));
+	uint32_t base = d0 + tid * static_cast<uint32_t>(sizeof(float2));
+	asm volatile("" : "+v"(base));
+	f32x2 v[MAXB][R];
 #pragma unroll
 	for (int t = 0; t < MAXB; ++t) {
 		const uint32_t b = tid + static_cast<uint32_t>(t) * NT;
 		if (b < nb) {
 #pragma unroll
-			for (int i = 0; i < R; ++i) v[t][i] = D[b + i * nb];
+			for (int i = 0; i < R; ++i)
+				v[t][i] = *(lds_c64_t)(size_t)(base + i * nb * static_cast<uint32_t>(sizeof(float2)) + t * NT * static_cast<uint32_t>(sizeof(float2)));
 		}
 	}
 	__syncthreads();
@@ -505,25 +523,20 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 			// and b e < 2^32 (b, e < 2^15) keeps the floor exact
 			const uint32_t q = (Ns == 1) ? b : __umulhi(b, magic);
 			const uint32_t j = b - q * Ns;
+			float2 u[R];
+#pragma unroll
+			for (int i = 0; i < R; ++i) u[i] = make_float2(v[t][i].x, v[t][i].y);
 			if (Ns > 1) {   // (the first pass's twiddles are all 1)
 				// a lane's twiddles are consecutive: few wide loads (an [i][j]
 				// layout, coalesced but a load each, measured slower)
 				const float2* w = reinterpret_cast<const float2*>(reinterpret_cast<const char*>(tw) + j * static_cast<uint32_t>((R - 1) * sizeof(float2)));
 #pragma unroll
-				for (int i = 1; i < R; ++i) v[t][i] = cmul(v[t][i], w[i - 1]);
+				for (int i = 1; i < R; ++i) u[i] = cmul(u[i], w[i - 1]);
 			}
-			dft<R>(v[t]);
-			const uint32_t o = q * Ns * R + j;
+			dft<R>(u);
+			const uint32_t o = d0 + (q * Ns * R + j) * static_cast<uint32_t>(sizeof(float2));
 #pragma unroll
-			for (int i = 0; i < R; ++i) D[o + i * Ns] = v[t][i];
-			if constexpr (MAX) {
-#pragma unroll
-				for (int i = 0; i < R; ++i) {
-					const uint32_t k = 2 * (o + i * Ns);
-					if (k < L) mx = fmaxf(mx, fabsf(v[t][i].x));
-					if (k + 1 < L) mx = fmaxf(mx, fabsf(v[t][i].y));
-				}
-			}
+			for (int i = 0; i < R; ++i) *(lds_c64_t)(size_t)(o + i * Ns * static_cast<uint32_t>(sizeof(float2))) = f32x2{u[i].x, u[i].y};
 		}
 	}
 	__syncthreads();
@@ -631,32 +644,26 @@ __device__ __forceinline__ void hilbert_in_place(float2* D, uint32_t M, const fl
 	}
 
 // D = DFT_M of the packed real signal in place -> F = DFT_M(conj C), the
-// Hilbert transform's samples; returns the lane's part of the largest |re|,
-// |im| of F over the first L samples.
+// Hilbert transform's samples.
 template<int NT>
-__device__ __forceinline__ float analytic_transforms(float2* D, const FftPlanArgs& P, const float2* __restrict__ tw,
-		const float2* __restrict__ wpost, uint32_t L)
+__device__ __forceinline__ void analytic_transforms(float2* D, const FftPlanArgs& P, const float2* __restrict__ tw,
+		const float2* __restrict__ wpost)
 {
-	float mx = 0.0f;
 	const uint32_t np = P.npass;
 	// forward passes, spectrum and the first inverse pass, the other inverse
 	// passes.  Transforms this long start with radix 5, 8 or 9.
 	const bool pairs = P.radix[0] == 5;
-	for (uint32_t s = 0; s + 1 < 2 * np; ++s) {
+	for (uint32_t s = 0; s < 2 * np; ++s) {
 		const uint32_t p = s < np ? s : s - np;
 		if (s == np && pairs) {
 			hilbert_pass<NT, 5>(D, P.M, wpost);
 			continue;
 		}
 		if (s == np) hilbert_in_place<NT>(D, P.M, wpost);
-#define MISTA_CALL(r) fft_pass<NT, r, false>(D, P.M, P.ns[p], P.ns_magic[p], tw + P.tw_off[p], L, mx)
+#define MISTA_CALL(r) fft_pass<NT, r>(D, P.M, P.ns[p], P.ns_magic[p], tw + P.tw_off[p])
 		MISTA_RADIX(P.radix[p], MISTA_CALL)
 #undef MISTA_CALL
 	}
-#define MISTA_CALL(r) fft_pass<NT, r, true>(D, P.M, P.ns[np - 1], P.ns_magic[np - 1], tw + P.tw_off[np - 1], L, mx)
-	MISTA_RADIX(P.radix[np - 1], MISTA_CALL)
-#undef MISTA_CALL
-	return mx;
 }
 
 // FIR x U output i (no DC removal): the generic polyphase loop over the
@@ -674,25 +681,43 @@ __device__ __forceinline__ float fir_at(const AnalyticArgs& A, const float* xs, 
 	return acc;
 }
 
+// put(c, get(c)) for c = tid, tid + NT, ... below n, B loads in flight (one at a
+// time each waits out the memory's latency: the 2048-sample echo of a 256-lane
+// workgroup took 11 500 of a channel's 80 000 cycles; 64 x 1024 channels of
+// 2048 x 4 samples 2.93 -> 2.61 ms).
+template<int NT, int B, typename GET, typename PUT>
+__device__ __forceinline__ void copy_batched(uint32_t tid, uint32_t n, GET get, PUT put)
+{
+	for (uint32_t c0 = tid; c0 < n; c0 += NT * B) {
+		decltype(get(0u)) v[B];
+#pragma unroll
+		for (uint32_t k = 0; k < B; ++k) v[k] = get(min(c0 + k * NT, n - 1));
+#pragma unroll
+		for (uint32_t k = 0; k < B; ++k)
+			if (c0 + k * NT < n) put(c0 + k * NT, v[k]);
+	}
+}
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 // FIR x UP on the matrix cores (UP divides 16; UP = 1: the samples themselves).
 // The outputs i = 256 tile + 16 c + m of 16 columns c are the product of a
 // constant 16 x K matrix of taps (row m = dq UP + p: phase p of the column's
-// dq-th input position) and a K x 16 matrix of echo samples, K = 27 taps +
+// dq-th input position) and a K x 16 matrix of echo samples, K = J taps +
 // 16/UP - 1 rounded up to 4: K/4 steps of v_mfma_f32_16x16x4_f32, which rounds
 // like the fma chain over the taps in order (measured: equal bits; the zero
 // taps at both ends add nothing).  Lane l gets the outputs
 // i = 256 tile + 16 (l % 16) + 4 (l / 16) + 0..3.
-template<int UP> struct MatFir {
+template<int UP, int J = static_cast<int>(kFirJ)> struct MatFir {
 	static constexpr int Q = 16 / UP;   // input positions per column
-	static constexpr int STEPS = UP == 1 ? 1 : (static_cast<int>(kFirJ) + Q - 1 + 3) / 4;
+	static constexpr int STEPS = UP == 1 ? 1 : (J + Q - 1 + 3) / 4;
 	// the echo in LDS: zeros before and after it, for the columns at both ends
 	static constexpr int PADL = 16, PADR = Q + 16;
 	static_assert(UP == 1 || 4 * STEPS - Q - 13 <= PADL, "the first column's oldest sample");
 	float a[STEPS];
 	int c0;   // echo index of this lane's first B entry at tile 0
-	__device__ MatFir(const AnalyticArgs& A, uint32_t tid)
+	__device__ MatFir(const AnalyticArgs& A, uint32_t tid) : MatFir(A.hpoly, A.off, tid) {}
+	__device__ MatFir(const float* __restrict__ hpoly, uint32_t off, uint32_t tid)
 	{
 		const int lane = static_cast<int>(tid & 63), m = lane % 16, g = lane / 16;
 		if constexpr (UP > 1) {
@@ -702,9 +727,9 @@ template<int UP> struct MatFir {
 #pragma unroll
 			for (int k = 0; k < STEPS; ++k) {
 				const int j = 4 * k + g - (Q - 1) + dq;
-				a[k] = (j >= 0 && j < static_cast<int>(kFirJ)) ? A.hpoly[p * static_cast<int>(kFirJ) + j] : 0.0f;
+				a[k] = (j >= 0 && j < J) ? hpoly[p * J + j] : 0.0f;
 			}
-			c0 = Q * m + static_cast<int>(A.off) / UP + Q - 1 - g;
+			c0 = Q * m + static_cast<int>(off) / UP + Q - 1 - g;
 		} else {
 			a[0] = 0.0f;
 			c0 = 16 * m + 4 * g;
@@ -748,12 +773,35 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 	float2* D = reinterpret_cast<float2*>(lds);
 	float* Df = reinterpret_cast<float*>(lds);
 	const uint32_t right = A.off / up + 2;
-	float* xs = reinterpret_cast<float*>(lds + static_cast<size_t>(M) * sizeof(float2));   // the echo: UP = 0 [J + ns + right], UP > 1 [PADL + ns + PADR]
-	float* hs = xs + J + A.ns + right;                                                    // UP = 0: [up][J]
+	// The echo: UP = 0 [J + ns + right] and the taps [up][J] after the transform,
+	// UP > 1 [PADL + ns + PADR] after it, too, or (SHARE) in its space, staged
+	// again for the output: 256-lane workgroups, of which four instead of three
+	// then share a CU (64 x 1024 channels of 2048 x 4 samples 2.61 -> 2.34 ms).
+	constexpr bool SHARE = NT == 256 && UP > 1;
+	float* xs = SHARE ? Df : reinterpret_cast<float*>(lds + static_cast<size_t>(M) * sizeof(float2));
+	float* hs = xs + J + A.ns + right;
 	const float* src = A.raw + static_cast<uint64_t>(ch) * A.ns;
 	const uint32_t ntl = (L + 255) / 256;
 	const uint32_t in_tile = 16 * (lane % 16) + 4 * (lane / 16);
 	const float* echo = UP > 1 ? xs : src;
+
+	auto stage_echo = [&]() {
+		if constexpr (UP > 1) {
+			constexpr int PADL = MatFir<UP>::PADL;
+			if constexpr (NT == 1024) {
+				// (four or five samples a lane: batches of 2, 5 and 8 measured
+				// 1 to 2 % slower)
+				for (uint32_t i = tid; i < A.ns + PADL + MatFir<UP>::PADR; i += NT) {
+					const int q = static_cast<int>(i) - PADL;
+					xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
+				}
+			} else {
+				if (tid < PADL) xs[tid] = 0.0f;
+				if (tid < MatFir<UP>::PADR) xs[PADL + A.ns + tid] = 0.0f;
+				copy_batched<NT, 8>(tid, A.ns, [&](uint32_t q) { return src[q]; }, [&](uint32_t q, float v) { xs[PADL + q] = v; });
+			}
+		}
+	};
 
 	// FIR x U (Interpolator.h:64-138, polyphase) and DC removal
 	// (Util.h:1009-1018) into the packed real array Df[0, L); Df[L, N) = 0.
@@ -773,11 +821,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 		// the wave's outputs wait in registers for the mean
 		const MatFir<UP> fir(A, tid);
 		if constexpr (UP > 1) {
-			constexpr int PADL = MatFir<UP>::PADL;
-			for (uint32_t i = tid; i < A.ns + PADL + MatFir<UP>::PADR; i += NT) {
-				const int q = static_cast<int>(i) - PADL;
-				xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
-			}
+			stage_echo();
 			__syncthreads();
 		}
 		f32x4 x[TILES];
@@ -806,6 +850,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 			}
 		}
 		reduce_mean();
+		if (SHARE) __syncthreads();   // the echo is read
 #pragma unroll
 		for (uint32_t k = 0; k < TILES; ++k) {
 			const uint32_t t = wave + k * NW;
@@ -866,8 +911,20 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 	}
 	__syncthreads();
 
-	float my = analytic_transforms<NT>(D, A.plan, A.tw, A.wpost, L);
+	analytic_transforms<NT>(D, A.plan, A.tw, A.wpost);
 
+	// UP > 0: the wave's part of F in registers
+	f32x4 y[UP > 0 ? TILES : 1];
+	if constexpr (UP > 0) {
+#pragma unroll
+		for (uint32_t k = 0; k < TILES; ++k)
+			if (wave + k * NW < ntl) y[k] = *reinterpret_cast<const f32x4*>(Df + 256 * (wave + k * NW) + in_tile);
+		if constexpr (SHARE) {
+			__syncthreads();
+			stage_echo();
+			__syncthreads();
+		}
+	}
 	// y[2m] + i y[2m+1] = conj(D[m]) / M: the Hilbert transform of x, the
 	// imaginary part of the analytic signal, whose real part is x itself
 	// (recomputed from the echo and the filter).
@@ -879,7 +936,23 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 		// zero), stored value z/s.  max |x_i - mean| is reached at the
 		// extremes of x, max |y| at max |F| (rounding is monotonic and odd):
 		// the workgroup's max x, max -x and max |F| are reduced first.
-		float nxmin = -xmin;
+		float nxmin = -xmin, my = 0.0f;   // largest |F| over the first L samples
+		if constexpr (UP > 0) {
+#pragma unroll
+			for (uint32_t k = 0; k < TILES; ++k) {
+				const uint32_t t = wave + k * NW;
+				if (256 * (t + 1) <= L) {
+					max_abs(my, make_float2(y[k][0], y[k][1]));
+					max_abs(my, make_float2(y[k][2], y[k][3]));
+				} else {
+#pragma unroll
+					for (uint32_t q = 0; q < 4; ++q)
+						if (256 * t + in_tile + q < L) my = fmaxf(my, fabsf(y[k][q]));
+				}
+			}
+		} else {
+			for (uint32_t i = tid; i < L; i += NT) my = fmaxf(my, fabsf(Df[i]));
+		}
 		for (int o = 32; o > 0; o >>= 1) {
 			my = fmaxf(my, __shfl_xor(my, o, 64));
 			xmax = fmaxf(xmax, __shfl_xor(xmax, o, 64));
@@ -916,13 +989,14 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 		// whole 16-byte stores where every row starts aligned
 		const bool vec = A.out16 ? (L & 3u) == 0 : (!mag && (L & 1u) == 0);
 		const MatFir<UP> fir(A, tid);
-#pragma unroll 1
-		for (uint32_t t = wave; t < ntl; t += NW) {
+#pragma unroll
+		for (uint32_t k = 0; k < TILES; ++k) {
+			const uint32_t t = wave + k * NW;
+			if (t >= ntl) continue;
 			const uint32_t i = 256 * t + in_tile;
-			const f32x4 x = fir.tile(echo, A.ns, t);
-			const float4 yv = *reinterpret_cast<const float4*>(Df + i);
+			const f32x4 x = fir.tile(echo, A.ns, t), yv = y[k];
 			const float re[4] = {x[0] - mean, x[1] - mean, x[2] - mean, x[3] - mean};
-			const float im[4] = {yv.x * coef, -yv.y * coef, yv.z * coef, -yv.w * coef};
+			const float im[4] = {yv[0] * coef, -yv[1] * coef, yv[2] * coef, -yv[3] * coef};
 			if (vec && i + 4 <= L) {
 				if (A.out16) {
 					uint4 pk;
@@ -966,10 +1040,10 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 // A workgroup a channel, one after the other; what waits (the odd samples, E,
 // then G1 and F's even half) lies in a scratch of 2 H values a workgroup.
 // Against the four-step path, which moves every channel through memory seven
-// times, 192 x 192 channels of 8192 samples x 8 take 20 ms instead of 48.4 at
-// FP16 (a channel of 96 x 96, in us a workgroup: 139, of which the transforms
-// 35, the output 22, the spectrum 17, the rest the FIR and the 1.1 MB that pass
-// through the scratch).  Keeping only H values of scratch by forming the odd
+// times, 192 x 192 channels of 8192 samples x 8 take 17.4 ms instead of 48.4 at
+// FP16 (20 with one load of scratch or echo in flight at a time; a workgroup then
+// spent 139 us on a channel, 35 of them on the transforms, 22 on the output, 17
+// on the spectrum, the rest on the FIR and the 1.1 MB through the scratch).  Keeping only H values of scratch by forming the odd
 // samples again measured slower (159 us).
 struct LongArgs {
 	AnalyticArgs a;        // a.plan, a.tw: the H-point transforms
@@ -1024,10 +1098,9 @@ __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_e
 			if constexpr (UP > 1) {
 				float* xs = reinterpret_cast<float*>(lds);   // the whole echo, before the transform needs the space
 				constexpr int PADL = MatFir<UP>::PADL;
-				for (uint32_t i = tid; i < A.ns + PADL + MatFir<UP>::PADR; i += NT) {
-					const int q = static_cast<int>(i) - PADL;
-					xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
-				}
+				if (tid < PADL) xs[tid] = 0.0f;
+				if (tid < MatFir<UP>::PADR) xs[PADL + A.ns + tid] = 0.0f;
+				copy_batched<NT, 8>(tid, A.ns, [&](uint32_t q) { return src[q]; }, [&](uint32_t q, float v) { xs[PADL + q] = v; });
 				__syncthreads();
 				echo = xs;
 			}
@@ -1075,55 +1148,72 @@ __global__ void __launch_bounds__(kFftThreads) __attribute__((amdgpu_waves_per_e
 		for (uint32_t stage = 0; stage < 4; ++stage) {
 			// D: the even samples, the odd samples, G0, G1
 			if (stage == 1) {
-				for (uint32_t c = tid; c < H; c += NT) D[c] = c < 64 * ntl ? sa[c] : make_float2(0.0f, 0.0f);
+				const uint32_t n = 64 * ntl;   // (at most H)
+				copy_batched<NT, 9>(tid, n, [&](uint32_t c) { return sa[c]; }, [&](uint32_t c, float2 v) { D[c] = v; });
+				for (uint32_t c = n + tid; c < H; c += NT) D[c] = make_float2(0.0f, 0.0f);
 			} else if (stage == 3) {
-				for (uint32_t c = tid; c < H; c += NT) D[c] = sb[c];
+				copy_batched<NT, 9>(tid, H, [&](uint32_t c) { return sb[c]; }, [&](uint32_t c, float2 v) { D[c] = v; });
 			} else if (stage == 2) {
-				my = 0.0f;
-				for (uint32_t k = tid; k <= H / 2; k += NT) {
-					const uint32_t k2 = k == 0 ? 0u : H - k;
-					const float2 e1 = sb[k], e2 = sb[k2];
-					const float2 w1 = table_at(B.wm, k), w2 = make_float2(-w1.x, w1.y);   // w^k, w^(H-k)
-					const float2 t1 = cmul(w1, D[k]), t2 = cmul(w2, D[k2]);
-					float2 a = cadd(e1, t1), b = csub(e1, t1);     // Z[k], Z[k + H]
-					float2 c = cadd(e2, t2), d = csub(e2, t2);     // Z[H - k], Z[M - k]
-					if (k == 0) {
-						a = make_float2(0.0f, 0.0f);
-						b = make_float2(-b.y, -b.x);   // bin M/2: conj(i Z)
-						c = a;
-						d = b;
-					} else {
-						spectrum_pair(a, d, table_at(A.wpost, k));
-						spectrum_pair(c, b, table_at(A.wpost, H - k));
-						if (2 * k == H) c = a, d = b;   // its own partner: bins k and k + H alone
+				constexpr uint32_t PB = 3;   // pairs whose loads are in flight together
+				for (uint32_t k0 = tid; k0 <= H / 2; k0 += NT * PB) {
+					float2 e1s[PB], e2s[PB], w1s[PB], p1s[PB], p2s[PB];
+#pragma unroll
+					for (uint32_t u = 0; u < PB; ++u) {
+						const uint32_t k = min(k0 + u * NT, H / 2), k2 = k == 0 ? 0u : H - k;
+						e1s[u] = sb[k];
+						e2s[u] = sb[k2];
+						w1s[u] = table_at(B.wm, k);
+						p1s[u] = table_at(A.wpost, k);
+						p2s[u] = table_at(A.wpost, H - k);
 					}
-					if (2 * k == H) b = d;
-					D[k] = cadd(a, b);
-					sb[k] = cmul(csub(a, b), w1);
-					if (k != 0 && 2 * k != H) {
-						D[k2] = cadd(c, d);
-						sb[k2] = cmul(csub(c, d), w2);
+#pragma unroll
+					for (uint32_t u = 0; u < PB; ++u) {
+						const uint32_t k = k0 + u * NT, k2 = k == 0 ? 0u : H - k;
+						if (k > H / 2) break;
+						const float2 e1 = e1s[u], e2 = e2s[u];
+						const float2 w1 = w1s[u], w2 = make_float2(-w1.x, w1.y);   // w^k, w^(H-k)
+						const float2 t1 = cmul(w1, D[k]), t2 = cmul(w2, D[k2]);
+						float2 a = cadd(e1, t1), b = csub(e1, t1);     // Z[k], Z[k + H]
+						float2 c = cadd(e2, t2), d = csub(e2, t2);     // Z[H - k], Z[M - k]
+						if (k == 0) {
+							a = make_float2(0.0f, 0.0f);
+							b = make_float2(-b.y, -b.x);   // bin M/2: conj(i Z)
+							c = a;
+							d = b;
+						} else {
+							spectrum_pair(a, d, p1s[u]);
+							spectrum_pair(c, b, p2s[u]);
+							if (2 * k == H) c = a, d = b;   // its own partner: bins k and k + H alone
+						}
+						if (2 * k == H) b = d;
+						D[k] = cadd(a, b);
+						sb[k] = cmul(csub(a, b), w1);
+						if (k != 0 && 2 * k != H) {
+							D[k2] = cadd(c, d);
+							sb[k2] = cmul(csub(c, d), w2);
+						}
 					}
 				}
 			}
 			__syncthreads();
-			for (uint32_t p = 0; p + 1 < np; ++p) {
-#define MISTA_CALL(r) fft_pass<NT, r, false>(D, H, A.plan.ns[p], A.plan.ns_magic[p], A.tw + A.plan.tw_off[p], L, my)
+			for (uint32_t p = 0; p < np; ++p) {
+#define MISTA_CALL(r) fft_pass<NT, r>(D, H, A.plan.ns[p], A.plan.ns_magic[p], A.tw + A.plan.tw_off[p])
 				MISTA_RADIX(A.plan.radix[p], MISTA_CALL)
 #undef MISTA_CALL
 			}
-			// (L / 2: half of the samples are in either half of F)
-#define MISTA_CALL(r) fft_pass<NT, r, true>(D, H, A.plan.ns[np - 1], A.plan.ns_magic[np - 1], A.tw + A.plan.tw_off[np - 1], L / 2, my)
-			MISTA_RADIX(A.plan.radix[np - 1], MISTA_CALL)
-#undef MISTA_CALL
 			if (stage == 0 || stage == 2) {
 				float2* out = stage == 0 ? sb : sa;
-				for (uint32_t c = tid; c < H; c += NT) out[c] = D[c];
+				for (uint32_t c = tid; c < H; c += NT) {
+					const float2 f = D[c];
+					if (stage == 2 && 4 * c < L) max_abs(my, f);   // (L is a multiple of 4)
+					out[c] = f;
+				}
 				__syncthreads();
 			}
 		}
 		float inv = 1.0f;
 		if (A.out16) {
+			for (uint32_t c = tid; 4 * c < L; c += NT) max_abs(my, D[c]);
 			float gm = fmaxf(my * coef, mx);
 			for (int o = 32; o > 0; o >>= 1) gm = fmaxf(gm, __shfl_xor(gm, o, 64));
 			if (lane == 0) redm[wave] = gm;
@@ -1528,7 +1618,10 @@ static void launch_analytic(const AnalyticArgs& A, uint32_t n, size_t lds, hipSt
 	const uint32_t M = A.plan.M;
 	auto by_size = [&](auto up) {
 		constexpr int UP = decltype(up)::value;
-		if (M <= kFftPerLane * 256 && lds <= 53 * 1024) go(analytic_lds_kernel<256, UP>, 256);
+		if (M <= kFftPerLane * 256) {
+			if (UP > 1) lds = static_cast<size_t>(M) * sizeof(float2);
+			go(analytic_lds_kernel<256, UP>, 256);
+		}
 		else if (M <= kFftPerLane * 512 && lds <= 80 * 1024) go(analytic_lds_kernel<512, UP>, 512);
 		else go(analytic_lds_kernel<1024, UP>, 1024);
 	};
@@ -1832,6 +1925,7 @@ static size_t long_lds_bytes(const FrameGeom& g, uint32_t J, uint32_t off)
 {
 	const uint32_t up = fused_up(g.up, J, off);
 	if (up == 0 || g.nf % 4 != 0 || g.nf / 4 > kFftMaxM || g.L % 4 != 0) return 0;
+	if (up > 1 && g.L > 65536) return 0;   // refused, as by every FIR
 	size_t b = static_cast<size_t>(g.nf / 4) * sizeof(float2);
 	if (up > 1) b += (static_cast<size_t>(kPieceTiles) * 256 / up + 64) * sizeof(float);
 	return b <= 160 * 1024 - 512 ? b : 0;
