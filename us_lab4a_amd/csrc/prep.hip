@@ -2143,28 +2143,76 @@ std::vector<double> rf4x_filter()
 	return h;
 }
 
+constexpr int kRfUp = 4, kRfJ = 21;   // rf4x_filter's factor and taps per phase
+
+// FIR x 4 + DC removal of a channel a workgroup on the matrix cores, the outputs
+// waiting in registers for the mean (a wave: TILES tiles of 256, every NT / 64-th).
+// Bound by writing the tensor.  fir_dc_kernel, whose every tap reads both
+// operands from LDS, took 0.49 ms for 128 x 128 channels of 2048 samples in 16
+// launches (537 MB out); this takes 0.113 ms.
+template<int NT, int TILES>
+__global__ void __launch_bounds__(NT) rf_fir_kernel(const float* __restrict__ raw, uint32_t ns, uint32_t dz,
+		const float* __restrict__ hpoly, uint32_t off, float* __restrict__ out)
+{
+	using Fir = MatFir<kRfUp, kRfJ>;
+	extern __shared__ float xs[];   // the echo: [PADL + ns + PADR]
+	constexpr uint32_t NW = NT / 64;
+	__shared__ double red[NW];
+	const uint32_t tid = threadIdx.x, lane = tid & 63, L = ns * kRfUp, ntl = (L + 255) / 256;
+	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const uint32_t in_tile = 16 * (lane % 16) + 4 * (lane / 16);
+	const float* src = raw + static_cast<uint64_t>(blockIdx.x) * ns;
+	const Fir fir(hpoly, off, tid);
+	if (tid < Fir::PADL) xs[tid] = 0.0f;
+	if (tid < Fir::PADR) xs[Fir::PADL + ns + tid] = 0.0f;
+	copy_batched<NT, 8>(tid, ns, [&](uint32_t q) { return src[q]; }, [&](uint32_t q, float v) { xs[Fir::PADL + q] = v; });
+	__syncthreads();
+	f32x4 x[TILES];
+	double part = 0.0;
+#pragma unroll
+	for (uint32_t k = 0; k < TILES; ++k) {
+		const uint32_t t = wave + k * NW, i = 256 * t + in_tile;
+		if (t >= ntl) continue;
+		x[k] = fir.tile(xs, ns, t);
+#pragma unroll
+		for (uint32_t q = 0; q < 4; ++q)
+			if (i + q >= dz && i + q < L) part += static_cast<double>(x[k][q]);
+	}
+	for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
+	if (lane == 0) red[wave] = part;
+	__syncthreads();
+	double sum = red[0];
+	for (uint32_t w = 1; w < NW; ++w) sum += red[w];
+	const float mean = static_cast<float>(sum / static_cast<double>(L - dz));
+	float* dst = out + static_cast<uint64_t>(blockIdx.x) * L;
+#pragma unroll
+	for (uint32_t k = 0; k < TILES; ++k) {
+		const uint32_t i = 256 * (wave + k * NW) + in_tile;
+		if (i >= L) continue;   // (L is a multiple of 4)
+		*reinterpret_cast<f32x4*>(dst + i) = f32x4{x[k][0] - mean, x[k][1] - mean, x[k][2] - mean, x[k][3] - mean};
+	}
+}
+
 void prepare_signals_rf(const FrameGeom& g, const float* d_raw, const float* d_filter_poly, uint32_t J, uint32_t off,
 		float* d_tensor, hipStream_t s)
 {
+	if (g.up != kRfUp || J != kRfJ || off % kRfUp != 0) MISTA_THROW(MISTA_E_INVALID_STATE, "RF filter of " << J << " x " << g.up << " taps");
 	const uint32_t nch = g.ntx * g.nrx;
-	const uint32_t chunk = std::min<uint32_t>(nch, 1024u);
-	const size_t lds = (static_cast<size_t>(J) + g.ns + off / g.up + 2 + static_cast<size_t>(g.up) * J) * sizeof(float);
-	if (lds > 150 * 1024) MISTA_THROW(MISTA_E_INVALID_PARAM, "channel too long for the LDS FIR: " << g.ns << " samples");
-	const uint32_t vpt = (g.L + kFirThreads - 1) / kFirThreads;
-	if (vpt > 64) MISTA_THROW(MISTA_E_INVALID_PARAM, "signal length " << g.L << " exceeds 65536");
-	FrameGeom gr = g;
-	gr.nf = g.L;   // rows written back to back, no FFT padding
-	for (uint32_t c0 = 0; c0 < nch; c0 += chunk) {
-		const uint32_t n = std::min(chunk, nch - c0);
-		const float* raw = d_raw + static_cast<uint64_t>(c0) * g.ns;
-		float* out = d_tensor + static_cast<uint64_t>(c0) * g.L;
-		if (vpt <= 4) launch_fir<4>(n, gr, raw, d_filter_poly, J, off, out, s);
-		else if (vpt <= 8) launch_fir<8>(n, gr, raw, d_filter_poly, J, off, out, s);
-		else if (vpt <= 16) launch_fir<16>(n, gr, raw, d_filter_poly, J, off, out, s);
-		else if (vpt <= 32) launch_fir<32>(n, gr, raw, d_filter_poly, J, off, out, s);
-		else launch_fir<64>(n, gr, raw, d_filter_poly, J, off, out, s);
-		HIP_CHECK(hipGetLastError());
+	if (g.L > 65536) {
+		if ((static_cast<size_t>(g.ns) + 117u) * sizeof(float) > 150 * 1024) MISTA_THROW(MISTA_E_INVALID_PARAM, "channel too long for the LDS FIR: " << g.ns << " samples");
+		MISTA_THROW(MISTA_E_INVALID_PARAM, "signal length " << g.L << " exceeds 65536");
 	}
+	const size_t lds = (static_cast<size_t>(g.ns) + MatFir<kRfUp, kRfJ>::PADL + MatFir<kRfUp, kRfJ>::PADR) * sizeof(float);
+	auto go = [&](auto kern, uint32_t nt) {
+		HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+				static_cast<int>(lds)));
+		hipLaunchKernelGGL(kern, dim3(nch), dim3(nt), lds, s, d_raw, g.ns, g.dz_up, d_filter_poly, off, d_tensor);
+		HIP_CHECK(hipGetLastError());
+	};
+	if (g.L <= 8192) go(rf_fir_kernel<256, 8>, 256);
+	else if (g.L <= 16384) go(rf_fir_kernel<512, 8>, 512);
+	else if (g.L <= 32768) go(rf_fir_kernel<1024, 8>, 1024);
+	else go(rf_fir_kernel<1024, 16>, 1024);
 }
 
 void envelope_rows(PrepState& st, float* d_data, uint32_t n1, uint32_t n2, hipStream_t s)
