@@ -1113,10 +1113,10 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 					bool any = false;
 					for (const int p1 : cands) {
 						if (p1 == 0 && npts == 2048 && any) break;
-						// the better of two runs (the first may find cold caches)
+						// the best of three runs (the first may find cold caches)
 						float ms = 0.0f;
 						bool run = false;
-						for (int rep = 0; rep < 2; ++rep) {
+						for (int rep = 0; rep < 3; ++rep) {
 							float t = 0.0f;
 							run = timed(p0, p1, t);
 							ms = rep == 0 ? t : std::min(ms, t);

@@ -321,6 +321,11 @@ __device__ __forceinline__ void lds_dma16_slots(const void* base, uint32_t voff,
 			".Ldma_%=:"
 			:: "s"(lds), "v"(voff), "s"(base), "s"(n) : "memory", "m0", "scc");
 }
+// One slot.
+__device__ __forceinline__ void lds_dma16_slot(const void* base, uint32_t voff, uint32_t lds)
+{
+	asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // Wait until at most n (wave-uniform) vector memory operations of this wave
@@ -479,16 +484,19 @@ __device__ __forceinline__ void das_tile(const TileArgs& A, const uint32_t tile,
 	const uint32_t wj = wave / WPW, sub = wave % WPW;
 	uint32_t is_t = 0, is_h = 0, is_buf = 0, is_d = 0;
 	const unsigned char* is_base = static_cast<const unsigned char*>(A.tensor) + (static_cast<uint64_t>(grp) * R + wj) * chan_bytes;
+	const unsigned char* is_src = is_base;   // its channel of chunk is_h
 	uint32_t iw = 0;
-	auto load_issue_word = [&]() { iw = wtab[is_t * kRxGroup + is_h * hstride + wj]; };
+	// (32-bit byte offsets: scalar loads take them as they are)
+	typedef __attribute__((address_space(4))) const char* cbyte_t;
+	auto load_issue_word = [&]() { iw = *(cu32_t)((cbyte_t)wtab + (is_t * kRxGroup + is_h * hstride + wj) * 4u); };
 	auto issue_delays = [&](uint32_t t) -> uint32_t {   // transmit t's, a slot a wave
 		uint32_t count = 0;
 #pragma unroll
 		for (uint32_t d0 = 0; d0 < DSLOTS; d0 += NW) {
 			const uint32_t d = d0 + (NW - 1 - wave);
 			if (d0 + NW <= DSLOTS || d < DSLOTS) {
-				lds_dma16_slots(td + static_cast<uint64_t>(nrx + t) * NPTS + d * 256u, voff,
-						lds_ring + ring + (is_d * DSLOTS + d) * 1024u, 1);
+				lds_dma16_slot(td + static_cast<uint64_t>(nrx + t) * NPTS + d * 256u, voff,
+						lds_ring + ring + (is_d * DSLOTS + d) * 1024u);
 				++count;
 			}
 		}
@@ -498,19 +506,23 @@ __device__ __forceinline__ void das_tile(const TileArgs& A, const uint32_t tile,
 	// copies of the cursor's chunk; returns how many copy instructions this wave issued
 	auto issue = [&]() -> uint32_t {
 		const uint32_t n = (iw >> kSlotShift) & 127u;
-		const uint32_t h = (n + WPW - 1) / WPW, s0 = sub * h;
-		uint32_t left = s0 < n ? min(h, n - s0) : 0u;
-		uint32_t count = left;
-		const unsigned char* src = is_base + is_h * RC * chan_bytes + static_cast<uint64_t>((iw & kWsMask) + s0 * 1024u);
-		uint32_t dst = lds_ring + is_buf + wj * win + s0 * 1024u;
-		for (; left > 4; left -= 4, src += 4096, dst += 4096) lds_dma16_slots(src, voff, dst, 4);
-		lds_dma16_slots(src, voff, dst, left);
+		uint32_t count = 0;
+		if (sub * 4 < n) {
+			const unsigned char* src = is_src + ((iw & kWsMask) + sub * 4096u);
+			uint32_t dst = lds_ring + is_buf + wj * win + sub * 4096u;
+			for (uint32_t s0 = sub * 4; s0 < n; s0 += 4 * WPW, src += 4096 * WPW, dst += 4096 * WPW) {
+				lds_dma16_slots(src, voff, dst, n - s0);
+				count += min(n - s0, 4u);
+			}
+		}
 		is_buf += buf_bytes;
 		if (is_buf == ring) is_buf = 0;
+		is_src += RC * chan_bytes;
 		if (++is_h == H) {
 			is_h = 0;
 			++is_t;
 			is_base += tx_bytes;
+			is_src = is_base;
 			if (is_t < ntx) count += issue_delays(is_t);
 		}
 		return count;
@@ -529,8 +541,8 @@ __device__ __forceinline__ void das_tile(const TileArgs& A, const uint32_t tile,
 	auto load_chunk = [&](uint32_t off) {
 #pragma unroll
 		for (uint32_t j = 0; j < RC; ++j) {
-			cw[j] = wtab[off + j];
-			cwt[j] = weights[off + j];
+			cw[j] = ((cu32_t)((cbyte_t)wtab + off * 4u))[j];
+			cwt[j] = ((cf32_t)((cbyte_t)weights + off * 4u))[j];
 		}
 	};
 	load_chunk(0);
