@@ -158,11 +158,12 @@ def fp16_batched(wl, d_echoes, steps, warmup, inflight):
     from us_lab4a_amd.sta import CoherenceFactor
     npix = wl.n_x * wl.n_z
     outs = [(torch.empty(npix, device="cuda"), torch.empty(npix, device="cuda")) for _ in range(inflight)]
+    grid = wl.grid()   # one for the stream of frames, as a client keeps it
 
     def job(k):
         v, f = outs[k % len(outs)]
         return Job2D(config=wl.sta_config(), upsampling=wl.upsampling, coherence=CoherenceFactor(wl.cf, wl.cf_param),
-                     grid=wl.grid(), rx_apod=wl.rx_apodization(), tx_apod=wl.tx_apodization(), echoes=d_echoes,
+                     grid=grid, rx_apod=wl.rx_apodization(), tx_apod=wl.tx_apodization(), echoes=d_echoes,
                      value=v, factor=f, storage="f16", peak_offset=wl.peak_offset)
     with Engine(max_inflight=inflight, max_queued=4 * steps + 8) as eng:
         for t in [eng.submit(job(k)) for k in range(max(warmup, inflight))]:
@@ -553,7 +554,8 @@ def tile_name(ran):
     p0, p1 = ran
     if p0 < 0:
         return "gather kernel" if p0 == -1 else "rx-parallel (per-rx sums, then statistics; no tile fits)"
-    shape = {2: "8x32", 3: "32x8", 4: "8x8x4", 5: "16x32", 6: "32x16", 7: "8x8x8"}.get(p0, "16x16")
+    shape = {2: "8x32", 3: "32x8", 4: "8x8x4", 5: "16x32", 6: "32x16", 7: "8x8x8", 8: "32x32",
+             9: "64x32", 10: "16x8x8", 11: "16x16x8"}.get(p0, "16x16")
     tc, nb, kb = p1 & 0xFF, (p1 >> 8) & 0xFF, (p1 >> 16) & 0xFF
     budget = f"{kb} KiB budget" if kb else "smallest fitting budget"
     return f"{shape} tile, {tc} pairs per chunk, {nb} ring buffers ({budget})"

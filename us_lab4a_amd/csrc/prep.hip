@@ -3,7 +3,9 @@
 // Util.h:1009-1018, HilbertEnvelope.h:142-251), plus the FP64 element-to-pixel
 // delay table (replaces calculateDelaysSTAKernel, VectorialSTACUDAProcessor.cu:30-53).
 //
-// Per chunk of channels (one channel = one (tx, rx) echo):
+// One kernel a channel on chip (analytic_lds_kernel, analytic_long_kernel for long
+// records), four-step FFTs through memory beyond (fft4.hip), or, when selected,
+// the library's FFTs, per chunk of channels (one channel = one (tx, rx) echo):
 //   fir_dc_kernel     raw [ch][ns] -> real [ch][Nf]: polyphase FIR from LDS,
 //                     mean of [dz, L) removed, zero padding [L, Nf)
 //   hipfft R2C        real [ch][Nf] -> spec [ch][Nf/2+1]
