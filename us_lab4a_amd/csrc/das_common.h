@@ -321,10 +321,13 @@ __device__ __forceinline__ void lds_dma16_slots(const void* base, uint32_t voff,
 			".Ldma_%=:"
 			:: "s"(lds), "v"(voff), "s"(base), "s"(n) : "memory", "m0", "scc");
 }
-// One slot.
+// One slot.  The s_nop is the wait state that a load with LDS destination needs
+// after a scalar write of M0: the compiler puts it in for its own instructions,
+// but does not look inside asm (above, the compare and the branch are it).
 __device__ __forceinline__ void lds_dma16_slot(const void* base, uint32_t voff, uint32_t lds)
 {
-	asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+			:: "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
 #pragma clang diagnostic pop
 
