@@ -1,0 +1,63 @@
+"""The tiled DAS where its tables do not fit beside what else is on the device."""
+import numpy as np
+import pytest
+
+from us_lab4a_amd import workloads
+from us_lab4a_amd.sta import CoherenceFactor, HipSTAProcessor
+
+from parity import say
+
+pytestmark = pytest.mark.gpu
+
+MM = 1e-3
+GIB = 1 << 30
+
+
+def wide_frame():
+    """64 channels a side over 1000 x 2000 points: delay table 0.5 GB; kept whole,
+    the tiles' tables and sums take 2 GB."""
+    return workloads.Workload2D(name="wide", num_elements=64, num_samples=512, upsampling=4, cf="sign_coherence_factor",
+                                tx_apod="hanning", grid_x=(-8 * MM, 8 * MM), grid_z=(1 * MM, 10.8 * MM), n_x=1000, n_z=2000,
+                                points=6, point_x=(-7 * MM, 7 * MM), point_z=(2 * MM, 9 * MM), seed_points=41, seed_noise=42)
+
+
+def processor(wl, storage="f32"):
+    p = HipSTAProcessor(wl.sta_config(), None, wl.upsampling, CoherenceFactor(wl.cf, wl.cf_param), 0.0, wl.rx_apodization(),
+                        tx_apod=wl.tx_apodization(), storage=storage)
+    p.set_grid(wl.grid())
+    return p
+
+
+def das(p, v, f):
+    import torch
+    p.das_device(v, f)
+    torch.cuda.synchronize()
+    return v.cpu().numpy(), f.cpu().numpy()
+
+
+def test_frame_runs_where_its_tables_do_not_fit():
+    import torch
+    wl = wide_frame()
+    n = wl.n_x * wl.n_z
+    v, f = (torch.empty(n, dtype=torch.float32, device="cuda") for _ in range(2))
+    p = processor(wl)
+    p.set_kernel(1)
+    p.process_device(torch.from_numpy(wl.echoes_cpu()).cuda(), wl.num_samples, v, f)
+    torch.cuda.synchronize()
+    gv, gf = v.cpu().numpy(), f.cpu().numpy()
+    p.set_kernel(0)
+    held = []
+    while (free := torch.cuda.mem_get_info()[0]) > 3 * GIB // 2:
+        held.append(torch.empty(min(free - 5 * GIB // 4, 32 * GIB), dtype=torch.uint8, device="cuda"))
+    say("free bytes left", torch.cuda.mem_get_info()[0])
+    try:
+        for _ in range(2):   # the tuned frame, then one with the tables' slabs built again
+            tv, tf = das(p, v.fill_(-1.0), f.fill_(-1.0))
+            assert p.last_kernel()[0] >= 0, "the tiled DAS ran"
+            assert np.array_equal(tv, gv) and np.array_equal(tf, gf)
+    finally:
+        del held
+        torch.cuda.empty_cache()
+    tv, tf = das(p, v.fill_(-1.0), f.fill_(-1.0))
+    assert np.array_equal(tv, gv) and np.array_equal(tf, gf)
+    p.close()

@@ -435,6 +435,7 @@ int mista_create(const mista_sta_config* config, mista_handle** out)
 		h->rows = config->num_elements;
 		h->tx_row0 = config->first_tx_elem;
 		HIP_CHECK(hipStreamCreate(&h->stream));  // default priority
+		h->das_scratch.table_limit = das_table_limit(h->cfg.device);
 		h->rx_apod.assign(config->num_elements, 1.0f);
 		*out = h.release();
 	});
@@ -475,6 +476,7 @@ int mista_create_3d(const mista_sta3d_config* config, const float* tx_xy, const 
 		h->tx_row0 = config->num_rx;
 		set_elements_3d(h.get(), tx_xy, rx_xy);
 		HIP_CHECK(hipStreamCreate(&h->stream));  // default priority
+		h->das_scratch.table_limit = das_table_limit(h->cfg.device);
 		h->rx_apod.assign(config->num_rx, 1.0f);
 		*out = h.release();
 	});
@@ -508,6 +510,7 @@ int mista_create_rf(const mista_sta_config* config, mista_handle** out)
 		h->rows = c.num_elements;
 		h->tx_row0 = c.first_tx_elem;
 		HIP_CHECK(hipStreamCreate(&h->stream));  // default priority
+		h->das_scratch.table_limit = das_table_limit(h->cfg.device);
 		h->rx_apod.assign(c.num_elements, 1.0f);
 		*out = h.release();
 	});

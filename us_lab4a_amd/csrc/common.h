@@ -51,19 +51,13 @@ public:
 	DeviceBuffer& operator=(const DeviceBuffer&) = delete;
 	void* reserve(size_t bytes)
 	{
-		if (bytes > cap_) {
-			release();
-			if (bytes == 0) return nullptr;
-			hipError_t e = hipMalloc(&ptr_, bytes);
-			if (e != hipSuccess) {
-				ptr_ = nullptr;
-				MISTA_THROW(MISTA_E_NO_MEMORY, "hipMalloc(" << bytes << " bytes) failed: " << hipGetErrorString(e));
-			}
-			cap_ = bytes;
-			++alloc_epoch();
-		}
+		const hipError_t e = grow(bytes);
+		if (e != hipSuccess)
+			MISTA_THROW(MISTA_E_NO_MEMORY, "hipMalloc(" << bytes << " bytes) failed: " << hipGetErrorString(e));
 		return ptr_;
 	}
+	// The same, false where the memory is not there (the buffer is then empty).
+	bool try_reserve(size_t bytes) { return grow(bytes) == hipSuccess; }
 	void release()
 	{
 		if (ptr_) (void)hipFree(ptr_);
@@ -74,6 +68,20 @@ public:
 	size_t capacity() const { return cap_; }
 	template<typename T> T* as() const { return static_cast<T*>(ptr_); }
 private:
+	hipError_t grow(size_t bytes)
+	{
+		if (bytes <= cap_) return hipSuccess;
+		release();
+		const hipError_t e = hipMalloc(&ptr_, bytes);
+		if (e != hipSuccess) {
+			ptr_ = nullptr;
+			(void)hipGetLastError();   // not to be taken for a later launch's error
+			return e;
+		}
+		cap_ = bytes;
+		++alloc_epoch();
+		return hipSuccess;
+	}
 	void* ptr_ = nullptr;
 	size_t cap_ = 0;
 };
@@ -190,12 +198,16 @@ struct DasTuning {
 };
 struct DasScratch {
 	DeviceBuffer partial;           // small device scalars (max window slots)
-	DeviceBuffer delays;            // the tiles' delays in lane order
-	DeviceBuffer bounds;            // their bounds per tile and row
-	DeviceBuffer params;            // per (tile, rx, tx) window words
-	DeviceBuffer slots;             // per tile: slots of its longest window
+	// The tiles' delays in lane order, their bounds per tile and row, the window
+	// words per (tile, rx, tx) and per tile the slots of its longest window: of
+	// every tile (whole), or of a slab of tiles at a time, built as it runs.
+	DeviceBuffer delays, bounds, params, slots;
 	DeviceBuffer partials;          // per-rx sums (tiled: of a slab of tiles; rx-parallel form: of the frame)
-	uint64_t bounds_version = ~0ull;
+	size_t table_limit = 0;         // most bytes of those five for the tiled form (or one tile's)
+	size_t table_cap = 0;           // less where the device had no more for this grid (cap_version)
+	uint64_t cap_version = ~0ull;
+	bool whole = false;
+	uint64_t bounds_version = ~0ull;   // what max_slots and, if whole, the tables are of
 	uint64_t params_key = 0;
 	float params_offset = 0.0f;
 	uint32_t max_slots = 0;         // 1 KiB load slots per staged window
@@ -214,6 +226,10 @@ constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(256) << 20;
 // scratch: no device allocation; the tuned tile shape when there is one.
 void launch_das_noalloc(const FrameGeom& g, int tuned_p0, int tuned_p1, DasScratch& last, const void* d_tensor,
 		const float* d_delay, const float* d_w, float* d_value, float* d_factor, hipStream_t s);
+// Default DasScratch::table_limit on a device, and the most bytes that the tables
+// and sums of a frame take within a limit, over the shapes that the tuner tries.
+size_t das_table_limit(int device);
+size_t das_table_bytes(const FrameGeom& g, size_t limit);
 // One frame of a DAS batch.
 struct DasBatchItem {
 	const FrameGeom* g;

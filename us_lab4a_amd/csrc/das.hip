@@ -590,6 +590,14 @@ void build_window_tables(const FrameGeom& g, const TilePlan& tp, uint32_t tile0,
 	HIP_CHECK(hipGetLastError());
 }
 
+// The same into the first places of a handle's tables.
+void build_tables(const FrameGeom& g, const TilePlan& tp, uint32_t tile0, uint32_t n, const float* d_delay, DasScratch& scratch,
+		hipStream_t s)
+{
+	build_window_tables(g, tp, tile0, n, d_delay, scratch.delays.as<float>(), scratch.bounds.as<float2>(),
+			scratch.params.as<uint32_t>(), scratch.slots.as<uint32_t>(), scratch.partial.as<uint32_t>(), s);
+}
+
 uint32_t read_u32(const uint32_t* d, hipStream_t s)
 {
 	uint32_t v = 0;
@@ -723,52 +731,159 @@ void run_tiles(const FrameGeom& g, const TilePlan& tp, const TileArgs& first, co
 // The shape that is reported for p0 (0: the default).
 int reported_shape(const TilePlan& tp, int p0) { return p0 == 0 ? (tp.tg.ny > 1 ? 4 : 1) : p0; }
 
-// Tables of tile shape p0 in the handle's scratch (built when the grid, shape
-// or offset changed: synchronises s); false when the shape does not apply.
-bool ensure_tables(const FrameGeom& g, const TilePlan& tp, DasScratch& scratch, const float* d_delay, hipStream_t s)
+// Bytes of the tables of n tiles.
+size_t table_bytes(const FrameGeom& g, const TilePlan& tp, uint32_t n)
+{
+	return delays_bytes(g, tp, n) + bounds_bytes(g, tp, n) + words_bytes(g, tp, n) + n * sizeof(uint32_t);
+}
+
+// Tables and sums of a slab of a frame whose tables are not kept whole.
+constexpr size_t kSlabBytes = static_cast<size_t>(1) << 30;
+
+// How many tiles' tables and sums a frame holds at a time within a limit: whole,
+// the tables of all tiles and the sums of a slab of them, else both of a slab.
+struct TileRun {
+	bool whole = false;
+	uint32_t slab = 0;
+	uint32_t tables(const TilePlan& tp) const { return whole ? tp.ntiles : slab; }
+};
+
+TileRun tile_run(const FrameGeom& g, const TilePlan& tp, size_t limit)
+{
+	TileRun r;
+	r.slab = slab_tiles(g, tp);
+	r.whole = table_bytes(g, tp, tp.ntiles) + r.slab * sums_bytes(g, tp) <= limit;
+	if (!r.whole) {
+		const size_t per = table_bytes(g, tp, 1) + sums_bytes(g, tp);
+		r.slab = static_cast<uint32_t>(std::max<size_t>(1, std::min<size_t>(r.slab, std::min(limit, kSlabBytes) / per)));
+	}
+	return r;
+}
+
+// Tables of tile shape p0 (see tile_run), built when the grid, shape or offset
+// changed, which synchronises s; a slab's are built again as it runs.  Where the
+// device has no room for them, a smaller slab; false when the shape does not apply
+// or not even a tile's fit.
+bool ensure_tables(const FrameGeom& g, const TilePlan& tp, DasScratch& scratch, const float* d_delay, hipStream_t s, TileRun& run)
 {
 	if (!tp.ok) return false;
-	if (scratch.bounds_version != g.grid_version || scratch.params_key != tp.key || scratch.params_offset != g.offset) {
-		float* td = static_cast<float*>(scratch.delays.reserve(delays_bytes(g, tp, tp.ntiles)));
-		float2* b = static_cast<float2*>(scratch.bounds.reserve(bounds_bytes(g, tp, tp.ntiles)));
-		uint32_t* words = static_cast<uint32_t*>(scratch.params.reserve(words_bytes(g, tp, tp.ntiles)));
-		uint32_t* slots = static_cast<uint32_t*>(scratch.slots.reserve(static_cast<size_t>(tp.ntiles) * sizeof(uint32_t)));
-		uint32_t* d_max = static_cast<uint32_t*>(scratch.partial.reserve(256));
+	if (scratch.cap_version != g.grid_version) {
+		scratch.table_cap = scratch.table_limit;
+		scratch.cap_version = g.grid_version;
+	}
+	uint32_t* d_max = static_cast<uint32_t*>(scratch.partial.reserve(256));
+	for (;;) {
+		run = tile_run(g, tp, scratch.table_cap);
+		const uint32_t n = run.tables(tp);
+		DeviceBuffer* const buf[5] = {&scratch.delays, &scratch.bounds, &scratch.params, &scratch.slots, &scratch.partials};
+		const size_t bytes[5] = {delays_bytes(g, tp, n), bounds_bytes(g, tp, n), words_bytes(g, tp, n), n * sizeof(uint32_t),
+				run.slab * sums_bytes(g, tp)};
+		// a buffer that grows loses what it held, and so do all where another
+		// shape's larger ones would pass the limit together with this one's
+		bool grows = false, fits = true;
+		size_t need = 0, held = 0;
+		for (int k = 0; k < 5; ++k) {
+			grows = grows || (k < 4 && bytes[k] > buf[k]->capacity());
+			need += bytes[k];
+			held += std::max(bytes[k], buf[k]->capacity());
+		}
+		const bool drop = held > std::max(need, scratch.table_cap);
+		if (grows || drop) scratch.bounds_version = ~0ull;
+		if (drop)
+			for (DeviceBuffer* b : buf) b->release();
+		for (int k = 0; k < 5; ++k) fits = fits && buf[k]->try_reserve(bytes[k]);
+		if (fits) break;
+		scratch.bounds_version = ~0ull;
+		for (DeviceBuffer* b : buf) b->release();
+		if (n == 1) return false;
+		scratch.table_cap = std::min(run.whole ? kSlabBytes : need / 2, need - 1);
+	}
+	const bool same = scratch.bounds_version == g.grid_version && scratch.params_key == tp.key && scratch.params_offset == g.offset;
+	if (!same || (run.whole && !scratch.whole)) {
 		scratch.bounds_version = ~0ull;   // nothing half-built is kept
 		hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, d_max);
 		HIP_CHECK(hipGetLastError());
-		build_window_tables(g, tp, 0, tp.ntiles, d_delay, td, b, words, slots, d_max, s);
+		const uint32_t n = run.tables(tp);
+		for (uint32_t t0 = 0; t0 < tp.ntiles; t0 += n) build_tables(g, tp, t0, std::min(n, tp.ntiles - t0), d_delay, scratch, s);
 		scratch.max_slots = read_u32(d_max, s);
 		scratch.bounds_version = g.grid_version;
 		scratch.params_key = tp.key;
 		scratch.params_offset = g.offset;
 	}
+	scratch.whole = run.whole;
 	return true;
+}
+
+// Tile shapes that the tuner tries, in order.  The larger tiles copy fewer bytes
+// per pixel and pair (64x32 points: 0.67 window entries per point and pair against
+// 1.63 at 16x32, 128-element frame; DAS 5.8 ms at 64x32, 8.3 at 32x32, 9.1 at
+// 32x16).  The large ones go first, where they give every CU several workgroups.
+std::vector<int> tuner_shapes(const FrameGeom& g)
+{
+	std::vector<int> shapes;
+	for (int p0 : (g.ny > 1 ? std::vector<int>{11, 10} : std::vector<int>{9, 8})) {
+		const TilePlan tp = tile_plan(g, p0);
+		if (tp.ok && static_cast<uint64_t>(tp.ntiles) * (pad_nrx(g.nrx) / kRxGroup) >= 1024u) shapes.push_back(p0);
+	}
+	for (int p0 : (g.ny > 1 ? std::vector<int>{7, 4} : std::vector<int>{6, 5, 1, 3, 2})) shapes.push_back(p0);
+	return shapes;
 }
 
 }  // namespace
 
-// Builds (or reuses) the tables for tile shape p0 and runs the tiled kernel
-// with the chunking p1 (see choose_chunking).  p0: 0/1 = 16x16 (planes) or
-// 8x8x4 (volumes), 2 = 8x32, 3 = 32x8, 4 = 8x8x4; 512 points: 5 = 16x32,
+// A sixteenth of the device's memory.  Tables kept whole save building them in every
+// frame (1024 x 64 elements over 128 x 128 x 96 points, 7 GB of tables: DAS 46.6 ms
+// whole, 71.0 a slab at a time); past the limit the copy of the delays would stand
+// in the way of other handles' delay tables and tensors.
+size_t das_table_limit(int device)
+{
+	size_t total = 0;
+	HIP_CHECK(hipDeviceTotalMem(&total, device));
+	return total / 16;
+}
+
+size_t das_table_bytes(const FrameGeom& g, size_t limit)
+{
+	size_t most[5] = {0, 0, 0, 0, 0}, one = 0;
+	for (int p0 : tuner_shapes(g)) {
+		const TilePlan tp = tile_plan(g, p0);
+		if (!tp.ok) continue;
+		const TileRun run = tile_run(g, tp, limit);
+		const uint32_t n = run.tables(tp);
+		const size_t bytes[5] = {delays_bytes(g, tp, n), bounds_bytes(g, tp, n), words_bytes(g, tp, n), n * sizeof(uint32_t),
+				run.slab * sums_bytes(g, tp)};
+		size_t sum = 0;
+		for (int k = 0; k < 5; ++k) {
+			most[k] = std::max(most[k], bytes[k]);
+			sum += bytes[k];
+		}
+		one = std::max(one, sum);
+	}
+	return std::min(std::max(one, limit), most[0] + most[1] + most[2] + most[3] + most[4]);
+}
+
+// Builds (or reuses) the tables for tile shape p0 and runs the tiled kernel with
+// the chunking p1 (see choose_chunking).  p0: 0/1 = 16x16 (planes) or 8x8x4
+// (volumes), 2 = 8x32, 3 = 32x8, 4 = 8x8x4; 512 points: 5 = 16x32,
 // 6 = 32x16, 7 = 8x8x8; 1024 points: 8 = 32x32, 10 = 16x8x8; 2048 points:
 // 9 = 64x32, 11 = 16x16x8.  Returns false when the windows do not fit.
 bool launch_tiled(const FrameGeom& g, int p0, int p1, DasScratch& scratch, const DasArgs& args, const float* d_delay,
 		hipStream_t s)
 {
 	const TilePlan tp = tile_plan(g, p0);
-	if (!ensure_tables(g, tp, scratch, d_delay, s)) return false;
+	TileRun run;
+	if (!ensure_tables(g, tp, scratch, d_delay, s, run)) return false;
 	Chunking c;
 	if (!choose_chunking(tp.npts, p1, scratch.max_slots, c)) return false;
-	const uint32_t slab = slab_tiles(g, tp);
 	DasArgs a = args;
-	a.partial = static_cast<float2*>(scratch.partials.reserve(slab * sums_bytes(g, tp)));
-	for (uint32_t t0 = 0; t0 < tp.ntiles; t0 += slab) {
-		const uint32_t n = std::min(slab, tp.ntiles - t0);
+	a.partial = scratch.partials.as<float2>();
+	for (uint32_t t0 = 0; t0 < tp.ntiles; t0 += run.slab) {
+		const uint32_t n = std::min(run.slab, tp.ntiles - t0), first = run.whole ? t0 : 0u;
+		if (!run.whole) build_tables(g, tp, t0, n, d_delay, scratch, s);
 		TileArgs A = tile_args(g, a, n, c);
-		A.td = scratch.delays.as<const float>() + delays_bytes(g, tp, t0) / sizeof(float);
-		A.words = scratch.params.as<const uint32_t>() + words_bytes(g, tp, t0) / sizeof(uint32_t);
-		A.slots = scratch.slots.as<const uint32_t>() + t0;
+		A.td = scratch.delays.as<const float>() + delays_bytes(g, tp, first) / sizeof(float);
+		A.words = scratch.params.as<const uint32_t>() + words_bytes(g, tp, first) / sizeof(uint32_t);
+		A.slots = scratch.slots.as<const uint32_t>() + first;
 		run_tiles(g, tp, A, a, t0, n, c, s);
 	}
 	scratch.last_p0 = reported_shape(tp, p0);
@@ -945,10 +1060,11 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 			p1 = it.scratch->tuned_p1;
 		}
 		TilePlan tp;
+		TileRun run;
 		if (p0 >= 0) tp = tile_plan(g, p0);
-		if (p0 < 0 || !ensure_tables(g, tp, *it.scratch, it.delay, s) || it.scratch->max_slots > kMaxSlots ||
-				slab_tiles(g, tp) < tp.ntiles) {
-			alone.push_back(i);   // untuned geometry (it tunes alone), gather kernel, no tiled form, or more than one slab of sums
+		if (p0 < 0 || !ensure_tables(g, tp, *it.scratch, it.delay, s, run) || it.scratch->max_slots > kMaxSlots ||
+				!run.whole || run.slab < tp.ntiles) {
+			alone.push_back(i);   // untuned geometry (it tunes alone), gather kernel, no tiled form, or a slab at a time
 			continue;
 		}
 		const uint64_t cls = static_cast<uint64_t>(g.storage) | (static_cast<uint64_t>(tp.npts) << 32);
@@ -991,7 +1107,7 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 			const Ready& r = ready[grp[k]];
 			const DasBatchItem& it = items[r.i];
 			DasArgs a = das_args(*it.g, it.tensor, it.delay, it.w, it.value, it.factor);
-			a.partial = static_cast<float2*>(it.scratch->partials.reserve(r.tp.ntiles * sums_bytes(*it.g, r.tp)));
+			a.partial = it.scratch->partials.as<float2>();
 			TileArgs& A = B.jobs[k];
 			A = tile_args(*it.g, a, r.tp.ntiles, c);
 			A.td = it.scratch->delays.as<const float>();
@@ -1043,23 +1159,9 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 					(static_cast<uint64_t>(g.nrx) << 50) ^ (static_cast<uint64_t>(g.storage) << 60) ^
 					(static_cast<uint64_t>(g.cf_kind) << 62) ^ static_cast<uint64_t>(g.offset * 1024.0f);
 			if (scratch.tuned_key != key) {
-				// The larger tiles copy fewer bytes per pixel and pair (64x32
-				// points: 0.67 window entries per point and pair against 1.63
-				// at 16x32, 128-element frame; DAS 5.8 ms at 64x32, 8.3 at
-				// 32x32, 9.1 at 32x16).  The large ones go first, where they
-				// give every CU several workgroups; smaller planes are tried
-				// only where no large one fits, 256-point tiles only where
-				// nothing larger than 512 points won.
-				auto work = [&](int p0) {
-					const TilePlan tp = tile_plan(g, p0);
-					return static_cast<uint64_t>(tp.ntiles) * (pad_nrx(g.nrx) / kRxGroup);
-				};
-				std::vector<int> shapes;
-				const std::vector<int> large = g.ny > 1 ? std::vector<int>{11, 10} : std::vector<int>{9, 8};
-				for (int p0 : large)
-					if (tile_plan(g, p0).ok && work(p0) >= 1024u) shapes.push_back(p0);
-				for (int p0 : (g.ny > 1 ? std::vector<int>{7} : std::vector<int>{6, 5})) shapes.push_back(p0);
-				for (int p0 : (g.ny > 1 ? std::vector<int>{4} : std::vector<int>{1, 3, 2})) shapes.push_back(p0);
+				// Smaller planes are tried only where no large shape fits,
+				// 256-point tiles only where nothing larger than 512 points won.
+				const std::vector<int> shapes = tuner_shapes(g);
 				hipEvent_t e0 = nullptr, e1 = nullptr;
 				HIP_CHECK(hipEventCreate(&e0));
 				HIP_CHECK(hipEventCreate(&e1));
