@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 from us_lab4a_amd import workloads
+from us_lab4a_amd.serve import Engine, Job2D
 from us_lab4a_amd.sta import CoherenceFactor, HipSTAProcessor
 
 from parity import say
@@ -61,3 +62,45 @@ def test_frame_runs_where_its_tables_do_not_fit():
     tv, tf = das(p, v.fill_(-1.0), f.fill_(-1.0))
     assert np.array_equal(tv, gv) and np.array_equal(tf, gf)
     p.close()
+
+
+def job(wl, storage="f32"):
+    n = wl.n_x * wl.n_z
+    return Job2D(config=wl.sta_config(), upsampling=wl.upsampling, coherence=CoherenceFactor(wl.cf, wl.cf_param), grid=wl.grid(),
+                 rx_apod=wl.rx_apodization(), tx_apod=wl.tx_apodization(), echoes=wl.echoes_cpu(),
+                 value=np.zeros(n, np.float32), factor=np.zeros(n, np.float32), storage=storage)
+
+
+def run_jobs(jobs, budget=0):
+    """The jobs one after the other through one handle each; the largest number of
+    bytes that the engine counted as resident."""
+    most = 0
+    with Engine(max_inflight=2, hbm_budget=budget, handles_per_shape=1) as eng:
+        tickets = [eng.submit(j) for j in jobs]
+        while not all(eng.done(t) for t in tickets):
+            most = max(most, eng.stats()["resident_bytes"])
+        out = [eng.wait(t) for t in tickets]
+        most = max(most, eng.stats()["resident_bytes"])
+    return out, most
+
+
+def test_engine_keeps_to_its_budget():
+    """Short records over a large grid, where the tiles' tables and sums are most of a
+    handle: two jobs that do not fit together wait for each other; one that does not
+    fit with whole tables runs in slabs, to the same images."""
+    a, b = wide_frame(), wide_frame()
+    b.n_z = 1900
+    jobs = [job(a), job(b)]
+    (sa, sb), _ = run_jobs(jobs)
+    assert sa["ok"] and sb["ok"], (sa, sb)
+    ref = [(j.value.copy(), j.factor.copy()) for j in jobs]
+    fa, fb = sa["footprint"], sb["footprint"]
+    say("footprints", fa, fb)
+    for budget in (fa + fb - 1, fa - 1):
+        again = [job(a), job(b)]
+        stats, most = run_jobs(again, budget)
+        say("budget", budget, "resident", most, "footprints", [s["footprint"] for s in stats])
+        assert all(s["ok"] for s in stats), stats
+        assert most <= budget and max(s["footprint"] for s in stats) <= budget
+        for j, (v, f) in zip(again, ref):
+            assert np.array_equal(j.value, v) and np.array_equal(j.factor, f)

@@ -396,6 +396,7 @@ void set_elements_3d(mista_handle* h, const float* tx_xy, const float* rx_xy)
 namespace mista {
 // Library-internal accessors used by the serving engine (serve.cpp).
 hipStream_t handle_stream(mista_handle* h) { return h->stream; }
+void handle_limit_tables(mista_handle* h, size_t bytes) { h->das_scratch.table_limit = bytes; }
 size_t handle_device_bytes(const mista_handle* h)
 {
 	return h->d_rx_apod.capacity() + h->d_tx_apod.capacity() + h->d_w.capacity() + h->d_elem.capacity() +

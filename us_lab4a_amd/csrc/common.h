@@ -186,8 +186,10 @@ std::vector<double> rf4x_filter();
 void envelope_rows(PrepState& st, float* d_data, uint32_t n1, uint32_t n2, hipStream_t s);
 
 // Device bytes held by the signal-preparation state (plans' buffers and an
-// estimate of the FFT library's work area).
+// estimate of the FFT library's work area), and the most that it holds after
+// frames of this geometry in the automatic form, with the Kaiser filter.
 size_t prep_device_bytes(const PrepState& st);
+size_t prep_estimate(const FrameGeom& g);
 
 void launch_weights(const FrameGeom& g, const float* d_rx_apod, const float* d_tx_apod, const float* d_scale,
 		float* d_w, hipStream_t s);
@@ -254,5 +256,6 @@ void launch_tensor_convert_out(const FrameGeom& g, const void* d_tensor, const f
 // Serving-engine access to a processor handle (defined in api.cpp).
 hipStream_t handle_stream(mista_handle* h);
 size_t handle_device_bytes(const mista_handle* h);
+void handle_limit_tables(mista_handle* h, size_t bytes);
 
 }  // namespace mista

@@ -2062,6 +2062,20 @@ static void prepare_four_step(PrepState& st, const FrameGeom& g, const float* d_
 	}
 }
 
+size_t prep_estimate(const FrameGeom& g)
+{
+	const size_t nch = static_cast<size_t>(g.ntx) * g.nrx, M = g.nf / 2, c64 = sizeof(float2);
+	const uint32_t off = (kFirJ - 1) / 2 * g.up;
+	size_t b = static_cast<size_t>(g.up) * kFirJ * sizeof(float);   // taps
+	if (fused_lds_bytes(g, kFirJ, off)) return b + (M + 1 + M / 2 + 1) * c64;
+	if (M > kFftMaxM && long_lds_bytes(g, kFirJ, off)) {
+		const size_t H = M / 2;
+		return b + (H + 1 + H / 2 + 1 + H + 1) * c64 + std::min<size_t>(nch, 256) * 2 * (H + 1) * c64;
+	}
+	// four-step: a round's rows, its transforms twice, the channels' maxima; tables
+	return b + std::min<size_t>(nch, 256) * (g.nf * sizeof(float) + 2 * M * c64 + 2 * sizeof(float)) + 2 * (M + 1) * c64;
+}
+
 void prepare_signals(PrepState& st, const FrameGeom& g, const float* d_raw, const float* d_filter_poly,
 		uint32_t J, uint32_t off, void* d_tensor, float* d_scale, hipStream_t s)
 {

@@ -69,7 +69,7 @@ struct Job {
 	mista_job spec{};
 	std::vector<float> grid, rx_apod, tx_apod;   // owned copies of the small inputs
 	uint64_t key = 0;
-	size_t estimate = 0;
+	size_t estimate = 0, table_limit = 0;
 	Clock::time_point t_submit, t_admit, t_done;
 	hipEvent_t ev_start = nullptr, ev_end = nullptr, ev_prep = nullptr;
 	int slot = -1;
@@ -101,25 +101,41 @@ struct BuildTask {
 	int slot = -1;
 	mista_job spec{};
 	std::vector<float> grid, rx_apod, tx_apod;
+	size_t table_limit = 0;
 };
 
-// Device bytes of a 2-D processor for this job (tensor, delay table, window
-// tables, signal-preparation buffers, outputs), as the library allocates them.
-size_t estimate_bytes(const mista_job& j)
+// Device bytes of a 2-D processor for this job (tensor, delay table, signal
+// preparation, staged inputs and outputs, tile tables and sums), as the library
+// allocates them.  Where that passes the budget, the tables get what the rest leaves
+// of it (table_limit, else `most`): the frame then runs a slab of tiles at a time.
+size_t estimate_bytes(const mista_job& j, size_t budget, size_t most, size_t& table_limit)
 {
 	const mista_sta_config& c = j.config;
-	const uint64_t ntx = c.last_tx_elem - c.first_tx_elem + 1ull, nrx = c.num_elements;
-	const uint64_t L = static_cast<uint64_t>(j.num_samples) * c.upsampling_factor;
-	const uint64_t nf = hilbert_fft_size(static_cast<uint32_t>(L));
-	const uint64_t npix = static_cast<uint64_t>(j.n1) * j.n2;
-	const uint64_t tensor = ntx * nrx * L * storage_bytes(c.storage);
-	const uint64_t delays = nrx * npix * 4 + npix * 8;
-	const uint64_t ntx_pad = budget_pad_ntx(static_cast<uint32_t>(ntx));
-	const uint64_t tables = (npix / 256 + 1) * (nrx * ntx_pad * 8 + nrx * 8);
-	const uint64_t chunk = std::min<uint64_t>(ntx * nrx, 1024);
-	const uint64_t prep = chunk * nf * (4 + 8 + 16);
-	const uint64_t io = ntx * nrx * j.num_samples * 4 + npix * 8;
-	return tensor + delays + tables + prep + io + (16u << 20);
+	FrameGeom g{};
+	g.num_elements = g.nrx = c.num_elements;
+	g.first_tx = c.first_tx_elem;
+	g.ntx = c.last_tx_elem - c.first_tx_elem + 1U;
+	g.ns = j.num_samples;
+	g.up = c.upsampling_factor;
+	// (longer records are refused when the job runs)
+	g.L = static_cast<uint32_t>(std::min<uint64_t>(static_cast<uint64_t>(j.num_samples) * c.upsampling_factor, 1u << 20));
+	g.nf = hilbert_fft_size(g.L);
+	g.n1 = j.n1;
+	g.n2 = j.n2;
+	g.ny = 1;
+	g.npix = static_cast<uint64_t>(j.n1) * j.n2;
+	g.storage = c.storage;
+	const size_t nch = static_cast<size_t>(g.ntx) * g.nrx;
+	const size_t tensor = nch * (g.L * storage_bytes(c.storage) + sizeof(float)) + tensor_tail_padding();
+	const size_t delays = (g.nrx + 2) * g.npix * sizeof(float);
+	const size_t weights = (static_cast<size_t>(g.ntx) * pad_nrx(g.nrx) + g.nrx + g.ntx) * sizeof(float);
+	const size_t io = nch * j.num_samples * sizeof(float) + 2 * g.npix * sizeof(float);
+	const size_t rest = tensor + delays + weights + prep_estimate(g) + io + (16u << 20);
+	table_limit = most;
+	const size_t all = rest + das_table_bytes(g, most);
+	if (all <= budget) return all;
+	table_limit = std::min(most, budget > rest ? budget - rest : 0);
+	return rest + das_table_bytes(g, table_limit);
 }
 
 uint64_t job_key(const mista_job& j, const std::vector<float>& grid, const std::vector<float>& rx,
@@ -142,7 +158,7 @@ uint64_t job_key(const mista_job& j, const std::vector<float>& grid, const std::
 
 struct mista_engine {
 	mista_engine_config cfg{};
-	size_t budget = 0;
+	size_t budget = 0, table_limit = 0;
 	uint32_t per_shape = 2;
 	std::mutex mu;
 	std::condition_variable cv_work, cv_done, cv_build;
@@ -553,6 +569,7 @@ void mista_engine::build_one(BuildTask& t, std::unique_lock<std::mutex>& lk)
 		c.device = cfg.device;
 		const int rc = mista_create(&c, &h);
 		if (rc != MISTA_OK) MISTA_THROW(rc, mista_last_error(nullptr));
+		handle_limit_tables(h, t.job ? t.job->table_limit : t.table_limit);
 		ok(mista_set_grid(h, grid.data(), q.n1, q.n2));
 		ok(mista_set_rx_apod(h, rx.data(), static_cast<uint32_t>(rx.size())));
 		ok(mista_set_tx_apod(h, tx.empty() ? nullptr : tx.data(), static_cast<uint32_t>(tx.size())));
@@ -625,6 +642,7 @@ void mista_engine::build_one(BuildTask& t, std::unique_lock<std::mutex>& lk)
 			c.grid = t.job->grid;
 			c.rx_apod = t.job->rx_apod;
 			c.tx_apod = t.job->tx_apod;
+			c.table_limit = t.job->table_limit;
 			builds.push_back(std::move(c));
 		}
 	}
@@ -661,6 +679,7 @@ int mista_engine_create(const mista_engine_config* config, mista_engine** out)
 		if (config->handles_per_shape > 8) MISTA_THROW(MISTA_E_INVALID_PARAM, "handles_per_shape must be in [0, 8].");
 		auto e = std::make_unique<mista_engine>();
 		e->cfg = *config;
+		e->table_limit = das_table_limit(config->device);
 		e->per_shape = config->handles_per_shape ? config->handles_per_shape : 2u;
 		if (config->hbm_budget) {
 			e->budget = config->hbm_budget;
@@ -734,7 +753,7 @@ int mista_engine_submit(mista_engine* e, const mista_job* job, uint64_t* ticket)
 	j->rx_apod.assign(job->rx_apod, job->rx_apod + c.num_elements);
 	if (job->tx_apod) j->tx_apod.assign(job->tx_apod, job->tx_apod + (c.last_tx_elem - c.first_tx_elem + 1));
 	j->key = job_key(*job, j->grid, j->rx_apod, j->tx_apod);
-	j->estimate = estimate_bytes(*job);
+	j->estimate = estimate_bytes(*job, e->budget, e->table_limit, j->table_limit);
 	j->t_submit = Clock::now();
 	{
 		std::lock_guard<std::mutex> lk(e->mu);
