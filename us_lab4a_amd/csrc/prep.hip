@@ -2166,6 +2166,9 @@ constexpr int kRfUp = 4, kRfJ = 21;   // rf4x_filter's factor and taps per phase
 // Bound by writing the tensor.  fir_dc_kernel, whose every tap reads both
 // operands from LDS, took 0.49 ms for 128 x 128 channels of 2048 samples in 16
 // launches (537 MB out); this takes 0.113 ms.
+// The matrix product also multiplies samples just past an output's taps, by zeros.
+// A record with an infinity or NaN, which would come out of that as NaN (and which
+// the mean does not spread where it lies before dz), takes the taps one by one.
 template<int NT, int TILES>
 __global__ void __launch_bounds__(NT) rf_fir_kernel(const float* __restrict__ raw, uint32_t ns, uint32_t dz,
 		const float* __restrict__ hpoly, uint32_t off, float* __restrict__ out)
@@ -2174,17 +2177,48 @@ __global__ void __launch_bounds__(NT) rf_fir_kernel(const float* __restrict__ ra
 	extern __shared__ float xs[];   // the echo: [PADL + ns + PADR]
 	constexpr uint32_t NW = NT / 64;
 	__shared__ double red[NW];
+	__shared__ uint32_t odd[NW];   // the wave has seen an infinity or NaN
 	const uint32_t tid = threadIdx.x, lane = tid & 63, L = ns * kRfUp, ntl = (L + 255) / 256;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const uint32_t in_tile = 16 * (lane % 16) + 4 * (lane / 16);
 	const float* src = raw + static_cast<uint64_t>(blockIdx.x) * ns;
+	float* dst = out + static_cast<uint64_t>(blockIdx.x) * L;
 	const Fir fir(hpoly, off, tid);
 	if (tid < Fir::PADL) xs[tid] = 0.0f;
 	if (tid < Fir::PADR) xs[Fir::PADL + ns + tid] = 0.0f;
-	copy_batched<NT, 8>(tid, ns, [&](uint32_t q) { return src[q]; }, [&](uint32_t q, float v) { xs[Fir::PADL + q] = v; });
+	uint32_t top = 0;   // the largest exponent
+	copy_batched<NT, 8>(tid, ns, [&](uint32_t q) { return src[q]; }, [&](uint32_t q, float v) {
+		xs[Fir::PADL + q] = v;
+		top = max(top, __float_as_uint(v) & 0x7F800000u);
+	});
+	const bool wave_odd = __any(top == 0x7F800000u);
+	if (lane == 0) odd[wave] = wave_odd;
 	__syncthreads();
-	f32x4 x[TILES];
+	uint32_t any_odd = 0;
+	for (uint32_t w = 0; w < NW; ++w) any_odd |= odd[w];
 	double part = 0.0;
+	auto mean = [&]() {
+		for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
+		if (lane == 0) red[wave] = part;
+		__syncthreads();
+		double sum = red[0];
+		for (uint32_t w = 1; w < NW; ++w) sum += red[w];
+		return static_cast<float>(sum / static_cast<double>(L - dz));
+	};
+	if (any_odd) {
+		const uint32_t taps = 2 * off + 1;
+		for (uint32_t i = tid; i < L; i += NT) {
+			const uint32_t ph = (i + off) % kRfUp, q0 = (i + off) / kRfUp;
+			float acc = 0.0f;
+			for (uint32_t j = 0; kRfUp * j + ph < taps; ++j) acc = fmaf(hpoly[ph * kRfJ + j], xs[Fir::PADL + q0 - j], acc);
+			if (i >= dz) part += static_cast<double>(acc);
+			dst[i] = acc;
+		}
+		const float m = mean();
+		for (uint32_t i = tid; i < L; i += NT) dst[i] -= m;
+		return;
+	}
+	f32x4 x[TILES];
 #pragma unroll
 	for (uint32_t k = 0; k < TILES; ++k) {
 		const uint32_t t = wave + k * NW, i = 256 * t + in_tile;
@@ -2194,18 +2228,12 @@ __global__ void __launch_bounds__(NT) rf_fir_kernel(const float* __restrict__ ra
 		for (uint32_t q = 0; q < 4; ++q)
 			if (i + q >= dz && i + q < L) part += static_cast<double>(x[k][q]);
 	}
-	for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
-	if (lane == 0) red[wave] = part;
-	__syncthreads();
-	double sum = red[0];
-	for (uint32_t w = 1; w < NW; ++w) sum += red[w];
-	const float mean = static_cast<float>(sum / static_cast<double>(L - dz));
-	float* dst = out + static_cast<uint64_t>(blockIdx.x) * L;
+	const float m = mean();
 #pragma unroll
 	for (uint32_t k = 0; k < TILES; ++k) {
 		const uint32_t i = 256 * (wave + k * NW) + in_tile;
 		if (i >= L) continue;   // (L is a multiple of 4)
-		*reinterpret_cast<f32x4*>(dst + i) = f32x4{x[k][0] - mean, x[k][1] - mean, x[k][2] - mean, x[k][3] - mean};
+		*reinterpret_cast<f32x4*>(dst + i) = f32x4{x[k][0] - m, x[k][1] - m, x[k][2] - m, x[k][3] - m};
 	}
 }
 
