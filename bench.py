@@ -558,7 +558,8 @@ def tile_name(ran):
              9: "64x32", 10: "16x8x8", 11: "16x16x8"}.get(p0, "16x16")
     tc, nb, kb = p1 & 0xFF, (p1 >> 8) & 0xFF, (p1 >> 16) & 0xFF
     budget = f"{kb} KiB budget" if kb else "smallest fitting budget"
-    return f"{shape} tile, {tc} pairs per chunk, {nb} ring buffers ({budget})"
+    lanes = {1: ", 1024 lanes", 2: ", 1024 lanes in chunks of two receive elements"}.get((p1 >> 24) & 3, "")
+    return f"{shape} tile, {tc} pairs per transmit step, {nb} ring buffers ({budget}{lanes})"
 
 
 if __name__ == "__main__":

@@ -259,8 +259,9 @@ int mista_tuned_kernel(const mista_handle* h, int* tile_param0, int* tile_param1
 /* The configuration of the last DAS launch: tile shape (-1 when the gather
  * kernel ran, -2 the rx-parallel form that runs where no tile fits: per-rx
  * sums by record or a lane per (pixel, rx), then the statistics a lane per pixel) and
- * pairs per transmit step | ring buffers << 8 | LDS budget in KiB << 16.  No
- * counterpart in the reference. */
+ * pairs per transmit step | ring buffers << 8 | LDS budget in KiB << 16 (0: the
+ * smallest that fits) | the lanes of 2048-point tiles << 24, the tile_param1 with
+ * which mista_set_kernel runs it again.  No counterpart in the reference. */
 int mista_last_kernel(const mista_handle* h, int* tile_param0, int* tile_param1);
 
 /*

@@ -614,7 +614,12 @@ struct Chunking {
 	uint32_t nbmax = 0;   // most chunk buffers
 	uint32_t lds = 0;     // LDS bytes
 	uint32_t nbuf = 0;    // chunk buffers of the tile with the longest window
-	int p1(int asked) const { return static_cast<int>(r | (nbuf << 8)) | (asked & 0xFF0000); }
+	// p1 that gives this chunking again, with the budget that was asked for
+	int p1(uint32_t npts, int asked) const
+	{
+		const uint32_t wide = npts != 2048u || nt == 512u ? 0u : rc == 2u ? 2u : 1u;
+		return static_cast<int>(r | (nbuf << 8) | (wide << 24)) | (asked & 0xFF0000);
+	}
 };
 
 // Chunking of the tiled kernel over windows of at most S slots.  p1: byte 0
@@ -887,7 +892,7 @@ bool launch_tiled(const FrameGeom& g, int p0, int p1, DasScratch& scratch, const
 		run_tiles(g, tp, A, a, t0, n, c, s);
 	}
 	scratch.last_p0 = reported_shape(tp, p0);
-	scratch.last_p1 = c.p1(p1);
+	scratch.last_p1 = c.p1(tp.npts, p1);
 	return true;
 }
 
@@ -1025,7 +1030,7 @@ void launch_das_noalloc(const FrameGeom& g, int tuned_p0, int tuned_p1, DasScrat
 			run_tiles(g, tp, A, a, t0, n, c, s);
 		}
 		last.last_p0 = reported_shape(tp, sh.first);
-		last.last_p1 = c.p1(sh.second);
+		last.last_p1 = c.p1(tp.npts, sh.second);
 		return;
 	}
 	if (!too_large)
@@ -1117,7 +1122,7 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 			first += r.tp.ntiles * A.ngrp;
 			args.push_back(a);
 			it.scratch->last_p0 = reported_shape(r.tp, r.p0);
-			it.scratch->last_p1 = c.p1(0);
+			it.scratch->last_p1 = c.p1(npts, 0);
 		}
 		B.first[B.njobs] = first;
 		B.total = first;

@@ -170,8 +170,8 @@ class HipSTAProcessor:
         return a.value, b.value
 
     def last_kernel(self):
-        """(tile shape, chunking) of the last DAS launch; shape -1: gather
-        kernel, -2: rx-parallel form (no tile fits)."""
+        """(tile shape, chunking) of the last DAS launch, as set_kernel(2, ...)
+        takes them; shape -1: gather kernel, -2: rx-parallel form (no tile fits)."""
         a, b = ctypes.c_int32(0), ctypes.c_int32(0)
         check(lib().mista_last_kernel(self._h, ctypes.byref(a), ctypes.byref(b)), self._h)
         return a.value, b.value
