@@ -54,3 +54,17 @@ def test_report_names_the_kernel():
         reports.append(ran)
     p.close()
     assert len(set(reports[:len(WIDE)])) == len(WIDE)
+
+
+@pytest.mark.parametrize("p0", [1, 2, 3])
+def test_eight_pairs_on_256_points_run_tiled(p0):
+    p, n = processor()
+    p.set_kernel(1)
+    gv, gf = image(p, n)
+    for p1 in (8, 8 | 52 << 16, 8 | 2 << 8 | 76 << 16):
+        p.set_kernel(2, p0, p1)
+        v, f = image(p, n)
+        say("asked", p0, hex(p1), "ran", p.last_kernel())
+        assert p.last_kernel()[0] == p0
+        assert np.array_equal(v, gv) and np.array_equal(f, gf)
+    p.close()

@@ -633,7 +633,9 @@ struct Chunking {
 bool choose_chunking(uint32_t npts, int p1, uint32_t S, Chunking& c)
 {
 	if (S > kMaxSlots) return false;
-	const uint32_t want_r = static_cast<uint32_t>(p1) & 0xFF, want_nb = (static_cast<uint32_t>(p1) >> 8) & 0xFF;
+	// (8 on 256 points: they have 4 only, whose ring is the smaller one)
+	const uint32_t asked_r = static_cast<uint32_t>(p1) & 0xFF, want_r = npts == 256u && asked_r == 8u ? 4u : asked_r;
+	const uint32_t want_nb = (static_cast<uint32_t>(p1) >> 8) & 0xFF;
 	const uint32_t want_kb = (static_cast<uint32_t>(p1) >> 16) & 0xFF;
 	const uint32_t wide = npts == 2048u ? static_cast<uint32_t>(p1) >> 24 & 3u : 0u;
 	c.nbmax = want_nb ? std::max(2u, std::min(want_nb, 4u)) : 4u;
