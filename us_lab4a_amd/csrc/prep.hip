@@ -2250,8 +2250,13 @@ void prepare_signals_rf(const FrameGeom& g, const float* d_raw, const float* d_f
 	auto go = [&](auto kern, uint32_t nt) {
 		HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
 				static_cast<int>(lds)));
-		hipLaunchKernelGGL(kern, dim3(nch), dim3(nt), lds, s, d_raw, g.ns, g.dz_up, d_filter_poly, off, d_tensor);
-		HIP_CHECK(hipGetLastError());
+		// (a launch holds fewer than 2^32 lanes)
+		constexpr uint32_t most = 1u << 21;
+		for (uint32_t c0 = 0; c0 < nch; c0 += most) {
+			hipLaunchKernelGGL(kern, dim3(std::min(most, nch - c0)), dim3(nt), lds, s, d_raw + static_cast<uint64_t>(c0) * g.ns, g.ns,
+					g.dz_up, d_filter_poly, off, d_tensor + static_cast<uint64_t>(c0) * g.L);
+			HIP_CHECK(hipGetLastError());
+		}
 	};
 	if (g.L <= 8192) go(rf_fir_kernel<256, 8>, 256);
 	else if (g.L <= 16384) go(rf_fir_kernel<512, 8>, 512);
