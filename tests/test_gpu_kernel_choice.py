@@ -68,3 +68,30 @@ def test_eight_pairs_on_256_points_run_tiled(p0):
         assert p.last_kernel()[0] == p0
         assert np.array_equal(v, gv) and np.array_equal(f, gf)
     p.close()
+
+
+def test_first_frame_does_not_time_what_cannot_win():
+    """256 elements over 512 x 512 points, frames of some 22 ms: the first one, which
+    times tile shapes and chunkings, takes no more than 5.5 of them and 15 ms (the
+    tables)."""
+    import time
+
+    import torch
+    wl = workloads.Workload2D(name="first", num_elements=256, num_samples=4096, upsampling=8, cf="phase_coherence_factor",
+                              grid_x=(-38 * MM, 38 * MM), grid_z=(5 * MM, 75 * MM), n_x=512, n_z=512)
+    e = torch.randn(256 * 256 * 4096, device="cuda")
+    v, f = (torch.empty(wl.n_x * wl.n_z, device="cuda") for _ in range(2))
+    first, steady = [], []
+    for _ in range(3):   # (the first handle also loads the kernels)
+        p = HipSTAProcessor(wl.sta_config(), None, wl.upsampling, CoherenceFactor(wl.cf, wl.cf_param), 0.0,
+                            wl.rx_apodization(), storage="f16")
+        p.set_grid(wl.grid())
+        for times in (first, steady):
+            torch.cuda.synchronize()
+            t = time.perf_counter()
+            p.process_device(e, wl.num_samples, v, f)
+            torch.cuda.synchronize()
+            times.append((time.perf_counter() - t) * 1e3)
+        p.close()
+    say("first frames", [round(t, 1) for t in first], "steady", [round(t, 1) for t in steady], "ms")
+    assert min(first) <= 5.5 * min(steady) + 15.0

@@ -614,6 +614,7 @@ struct Chunking {
 	uint32_t nbmax = 0;   // most chunk buffers
 	uint32_t lds = 0;     // LDS bytes
 	uint32_t nbuf = 0;    // chunk buffers of the tile with the longest window
+	bool same(const Chunking& o) const { return r == o.r && nt == o.nt && rc == o.rc && nbmax == o.nbmax && lds == o.lds; }
 	// p1 that gives this chunking again, with the budget that was asked for
 	int p1(uint32_t npts, int asked) const
 	{
@@ -1160,8 +1161,7 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 			// Autotuner: on the first frame of a geometry, time every
 			// candidate tile shape, LDS budget and chunk size (each writes
 			// the same images) and keep the fastest for the frames that
-			// follow.  The first run of a shape builds its window tables and
-			// is not timed.
+			// follow.
 			const uint64_t key = g.grid_version ^ (static_cast<uint64_t>(g.L) << 20) ^ (static_cast<uint64_t>(g.ntx) << 40) ^
 					(static_cast<uint64_t>(g.nrx) << 50) ^ (static_cast<uint64_t>(g.storage) << 60) ^
 					(static_cast<uint64_t>(g.cf_kind) << 62) ^ static_cast<uint64_t>(g.offset * 1024.0f);
@@ -1192,51 +1192,53 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 					const uint32_t npts = tile_plan(g, p0).npts;
 					const uint32_t won = bp0 >= 0 ? tile_plan(g, bp0).npts : 0u;
 					if (won > 512 && (npts == 256 || (npts == 512 && g.ny <= 1))) continue;
-					// the first run builds the shape's tables; not compared
-					HIP_CHECK(hipEventRecord(e0, s));
-					if (!launch_tiled(g, p0, 0, scratch, a, d_delay, s)) continue;
-					HIP_CHECK(hipEventRecord(e1, s));
-					last_p0 = p0;
-					HIP_CHECK(hipEventSynchronize(e1));
-					float first_ms = 0.0f;
-					HIP_CHECK(hipEventElapsedTime(&first_ms, e0, e1));
-					if (first_ms > 2.0f * kTuneLimitMs) long_frame = true;
-					// pairs per transmit step (4 or 8) in the LDS budgets worth
-					// a try, then the smallest budget that fits; a long frame
-					// takes that alone
-					std::vector<int> cands;
-					// 2048 points: 512 lanes with two workgroups a CU,
-					// 1024 lanes with two (4-byte entries: short windows,
-					// 100-element BF16 frame 0.66 -> 0.55 ms; 8-byte ones in
-					// chunks of two receive elements: 128-element frame 5.76
-					// -> 5.54 ms) or one; where none of them fits, the chunks
-					// of two in the whole LDS (192 elements of 65 536 samples
-					// 4.14 ms against 5.05 at 32x32).  1024 points: three
-					// workgroups a CU where they fit (128-element F16 frame
-					// 3.96 -> 3.55 ms, RF 1.03 -> 0.86), else two.
+					TileRun held;
+					if (!ensure_tables(g, tile_plan(g, p0), scratch, d_delay, s, held)) continue;
+					// The smallest LDS budget that fits, which is all that a long
+					// frame tries, then pairs per transmit step (4 or 8) in the
+					// budgets worth a try.  2048 points: 512 lanes with two
+					// workgroups a CU, 1024 lanes with two (4-byte entries: short
+					// windows, 100-element BF16 frame 0.66 -> 0.55 ms; 8-byte ones
+					// in chunks of two receive elements: 128-element frame 5.76 ->
+					// 5.54 ms) or one; where none of them fits, the chunks of two
+					// in the whole LDS (192 elements of 65 536 samples 4.14 ms
+					// against 5.05 at 32x32).  1024 points: three workgroups a CU
+					// where they fit (128-element F16 frame 3.96 -> 3.55 ms, RF
+					// 1.03 -> 0.86), else two.
 					const int wide = g.storage == MISTA_STORAGE_F32 ? 2 << 24 : 1 << 24;
-					if (!long_frame && npts == 2048) cands = {4 | (80 << 16), 4 | (80 << 16) | wide, 8 | (160 << 16)};
-					else if (!long_frame && npts == 1024) cands = {4 | (80 << 16)};
-					else if (!long_frame && npts == 512) cands = {8 | (52 << 16)};
-					cands.push_back(0);
-					bool any = false;
+					std::vector<int> cands = {0};
+					if (npts == 2048) cands.insert(cands.end(), {4 | (80 << 16), 4 | (80 << 16) | wide, 8 | (160 << 16)});
+					else if (npts == 1024) cands.push_back(4 | (80 << 16));
+					else if (npts == 512) cands.push_back(8 | (52 << 16));
+					std::vector<Chunking> tried;
 					for (const int p1 : cands) {
-						if (p1 == 0 && npts == 2048 && any) break;
-						// the best of three runs (the first may find cold caches)
+						Chunking c;
+						if (!choose_chunking(npts, p1, scratch.max_slots, c)) continue;
+						if (std::any_of(tried.begin(), tried.end(), [&](const Chunking& q) { return q.same(c); })) continue;
+						tried.push_back(c);
+						// Best of three runs, as the first may find cold caches;
+						// of two from 5 ms on, where runs agree within 2 % (the
+						// first: 12).  A first run of over 1 ms (shorter ones hold
+						// the load of the kernel) that is far enough behind the
+						// best ends a chunking, and a shape, whose chunkings differ
+						// by up to 1.42.  (256 elements, 512 x 512 points: first
+						// frame 176 -> 108 ms.)
 						float ms = 0.0f;
-						bool run = false;
-						for (int rep = 0; rep < 3; ++rep) {
+						for (int rep = 0; rep < (ms > 5.0f ? 2 : 3); ++rep) {
 							float t = 0.0f;
-							run = timed(p0, p1, t);
+							(void)timed(p0, p1, t);
 							ms = rep == 0 ? t : std::min(ms, t);
-							if (!run || t > kTuneLimitMs) break;
+							if (t > kTuneLimitMs || (bp0 >= 0 && t > 1.0f && t > 1.15f * best)) break;
 						}
-						any = any || run;
-						if (run && (bp0 < 0 || ms < best)) {
+						last_p0 = p0;
+						long_frame = long_frame || ms > kTuneLimitMs;
+						const bool lost = bp0 >= 0 && ms > 1.0f && ms > 1.5f * best;
+						if (bp0 < 0 || ms < best) {
 							best = ms;
 							bp0 = p0;
 							bp1 = p1;
 						}
+						if (p1 == 0 && (long_frame || lost)) break;
 					}
 				}
 				(void)hipEventDestroy(e0);
