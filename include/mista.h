@@ -202,9 +202,9 @@ int mista_das_batch_device(mista_handle* const* handles, uint32_t n, float* cons
  * images as mista_das_device with the tiled kernel; it calls no hipMalloc
  * or hipFree.  The handle must hold a prepared frame (the preparation sizes
  * every buffer the DAS reads).  The tile delays, window tables and per-rx
- * sums of the launch live in a static device array of 256 MiB that each GPU
- * holds once per process and that every call on that GPU rebuilds, a run of
- * tiles at a time: a geometry whose window tables need more than 80 MiB is
+ * sums of the launch live in a static device array of 256 MiB that the process's
+ * first call on a GPU loads (0.1 s: make one before time counts) and that every
+ * call on that GPU rebuilds, a run of tiles at a time: a geometry whose window tables need more than 80 MiB is
  * refused with MISTA_E_INVALID_PARAM, and calls that overlap on one GPU
  * (from several threads or streams) race.  Uses the tile shape tuned for the
  * geometry when there is one, else a default; it never tunes.  Stage timing

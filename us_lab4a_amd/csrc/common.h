@@ -224,6 +224,8 @@ size_t tensor_tail_padding();
 // as many tiles at a time as fit.
 constexpr size_t kNoAllocTableBytes = static_cast<size_t>(80) << 20;
 constexpr size_t kNoAllocScratchBytes = static_cast<size_t>(256) << 20;
+// The current device's scratch (looked up once per device, with the device current).
+unsigned char* noalloc_scratch();
 // DAS over the handle's resident tensor with its tables and sums in that
 // scratch: no device allocation; the tuned tile shape when there is one.
 void launch_das_noalloc(const FrameGeom& g, int tuned_p0, int tuned_p1, DasScratch& last, const void* d_tensor,

@@ -29,8 +29,6 @@
 #include "das_common.h"
 
 #include <algorithm>
-#include <map>
-#include <mutex>
 #include <cmath>
 #include <vector>
 
@@ -930,34 +928,6 @@ DasArgs das_args(const FrameGeom& g, const void* d_tensor, const float* d_delay,
 }
 
 // ---------------------------------------------------------------- no allocation
-
-// Device scratch of the no-allocation DAS: the tile delays, window tables and
-// per-rx sums of as many tiles as fit.  Every call on a GPU shares that GPU's
-// copy (each GPU the library runs on holds one until the process ends) and
-// rebuilds what it needs: calls that overlap on one GPU race.  In host code
-// `scratch` names a host-side stand-in; kernels get the device address from
-// hipGetSymbolAddress.
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
-
-namespace {
-std::mutex g_scratch_mu;
-std::map<int, unsigned char*> g_scratch_ptr;   // device ordinal -> that GPU's copy of scratch
-}  // namespace
-
-// The current device's copy of scratch (looked up once per device, with the
-// device current).
-static unsigned char* noalloc_scratch()
-{
-	int dev = 0;
-	HIP_CHECK(hipGetDevice(&dev));
-	std::lock_guard<std::mutex> g(g_scratch_mu);
-	auto it = g_scratch_ptr.find(dev);
-	if (it != g_scratch_ptr.end()) return it->second;
-	void* ptr = nullptr;
-	HIP_CHECK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch)));
-	g_scratch_ptr[dev] = static_cast<unsigned char*>(ptr);
-	return static_cast<unsigned char*>(ptr);
-}
 
 // Bytes of the window tables that decide whether the entry point takes a
 // geometry (its documented limit): transmits padded to 32, 64, 128 or equal
