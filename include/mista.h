@@ -285,12 +285,15 @@ int mista_create_rf(const mista_sta_config* config, mista_handle** out);
 int mista_envelope_device(mista_handle* h, float* d_data, uint32_t n1, uint32_t n2, void* stream);
 int mista_envelope(mista_handle* h, float* data, uint32_t n1, uint32_t n2);
 
-/* Select the signal-preparation implementation: 0 = automatic (fused LDS
- * kernel when the FFT fits on chip, else the four-step FFTs), 1 = library FFT
+/* Select the signal-preparation implementation: 0 = automatic, 1 = library FFT
  * (FIR kernel, hipFFT R2C, spectrum kernel, hipFFT C2C, store kernel),
- * 2 = fused LDS kernel (error if the frame does not fit), 3 = four-step FFTs
- * (FIR kernel, two-pass forward FFT, spectrum kernel, two-pass backward FFT,
- * store kernel; FFT sizes up to 2^20 whose two factors are 2-3-5 smooth). */
+ * 2 = fused LDS kernel (error if the frame does not fit: FFT sizes up to
+ * 36 864), 3 = not the fused kernel but what automatic takes where that does
+ * not fit: FFT sizes above 36 864 up to 73 728 on chip by halves (upsampling 1,
+ * 2, 4, 8 or 16, signal lengths that are multiples of 4), every other frame by
+ * four-step FFTs (FIR kernel, two-pass forward FFT, spectrum kernel, two-pass
+ * backward FFT, store kernel; FFT sizes up to 2^20 whose two factors are 2-3-5
+ * smooth). */
 int mista_set_prep(mista_handle* h, int method);
 
 /* Stage times of the last mista_das_device/mista_process_device frame (ms,

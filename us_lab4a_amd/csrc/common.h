@@ -163,7 +163,7 @@ void fft4_exec(const Fft4Plan& p, const float2* in, float2* tmp, float2* out, ui
 		uint32_t* ymax = nullptr, uint32_t npair = 0, bool odd = false);
 struct PrepState {
 	PrepPlan* plan = nullptr;  // owned; destroyed in prep.hip where PrepPlan is complete
-	int method = 0;            // 0 automatic (fused kernel, else four-step FFTs), 1 library FFT (hipFFT), 2 fused kernel, 3 four-step FFTs
+	int method = 0;            // 0 automatic (fused kernel, else as 3), 1 library FFT (hipFFT), 2 fused kernel, 3 on chip by halves, else four-step FFTs
 	bool last_fused = false;   // the last preparation ran the fused kernel
 	// called before the kernels of channels [c0, c0 + n) are launched (the
 	// host path uploads each chunk of echoes just in time)

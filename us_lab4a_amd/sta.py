@@ -152,8 +152,9 @@ class HipSTAProcessor:
         self._grid_xz = xz
 
     def set_prep(self, method):
-        """0 automatic, 1 library FFT (hipFFT), 2 fused LDS kernel,
-        3 four-step FFTs (long records)."""
+        """0 automatic, 1 library FFT (hipFFT), 2 fused LDS kernel, 3 what
+        automatic takes where the fused kernel does not fit (long records: on
+        chip by halves up to an FFT size of 73 728, else four-step FFTs)."""
         check(lib().mista_set_prep(self._h, method), self._h)
 
     def set_kernel(self, variant, p0=0, p1=0):
