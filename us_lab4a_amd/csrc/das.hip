@@ -110,8 +110,8 @@ __global__ void __launch_bounds__(256) das_gather_kernel(const DasArgs a)
 // workgroup take consecutive pixels of one rx (grid y), so the delay-table
 // and partial-sum accesses are coalesced and the weights uniform.  The sum
 // over the transmits is the tiled kernel's fma chain in transmit order (an
-// excluded position adds nothing, where the tiled kernel adds it with weight
-// 0); out to partial[rx][pixel].  With far more lanes than pixels this keeps
+// excluded position adds nothing, where the tiled kernel adds a zero entry);
+// out to partial[rx][pixel].  With far more lanes than pixels this keeps
 // the GPU busy on grids too coarse for any tile (a window past 64 KiB) or too
 // small to fill it one pixel per lane.
 template<int STORAGE>

@@ -28,50 +28,33 @@ __device__ __forceinline__ float2 load_sample(const void* __restrict__ t, uint64
 	}
 }
 
-// LDS entry type per storage kind and its conversion to FP32 complex.
+// LDS entry type per storage kind.  lerp2: v0 + k (v1 - v0) per component from the
+// raw words of two entries as one LDS read returns them (LdsPair), with FP32
+// arithmetic: the difference rounded once, then one fused multiply-add.
 template<int STORAGE> struct Entry;
-// get: one entry as FP32 (re, im).  lerp: v0 + k (v1 - v0) per component
-// for the entries e[0], e[1], with FP32 arithmetic: the difference rounded
-// once, then one fused multiply-add.
-// lerp2: the same from the raw words of the two entries as one LDS read
-// returns them (LdsPair).
 template<uint32_t ESZ> struct LdsPair;
 template<> struct LdsPair<8> { using T = float4; };   // two 8-byte entries
 template<> struct LdsPair<4> { using T = uint2; };    // two 4-byte entries
 
 template<> struct Entry<MISTA_STORAGE_F32> {
 	using T = float2;
-	static __device__ __forceinline__ float2 get(T v) { return v; }
 	static __device__ __forceinline__ float2 lerp2(float4 e, float k)
 	{
 		return make_float2(fmaf(k, e.z - e.x, e.x), fmaf(k, e.w - e.y, e.y));
 	}
-	static __device__ __forceinline__ float2 lerp(const T* e, float k)
-	{
-		const float2 v0 = e[0], v1 = e[1];
-		return make_float2(fmaf(k, v1.x - v0.x, v0.x), fmaf(k, v1.y - v0.y, v0.y));
-	}
 };
 template<> struct Entry<MISTA_STORAGE_F16> {
 	using T = __half2;
-	static __device__ __forceinline__ float2 get(T v) { return __half22float2(v); }
-	static __device__ __forceinline__ float2 lerp(const T* e, float k)
+	static __device__ __forceinline__ float2 lerp2(uint2 e, float k)
 	{
-		const T h0 = e[0], h1 = e[1];
-		const uint32_t u0 = __builtin_bit_cast(uint32_t, h0), u1 = __builtin_bit_cast(uint32_t, h1);
 		// v1 - v0 straight from the FP16 halves: the mixed-precision FMA
 		// widens both exactly and rounds 1 * v1 - v0 once to FP32, as the
 		// widen-then-subtract form does, in one instruction
 		float dx, dy;
-		asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(dx) : "v"(u1), "v"(u0));
-		asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(dy) : "v"(u1), "v"(u0));
-		const float2 v0 = __half22float2(h0);
+		asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,1]" : "=v"(dx) : "v"(e.y), "v"(e.x));
+		asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,1] op_sel_hi:[1,0,1]" : "=v"(dy) : "v"(e.y), "v"(e.x));
+		const float2 v0 = __half22float2(__builtin_bit_cast(__half2, e.x));
 		return make_float2(fmaf(k, dx, v0.x), fmaf(k, dy, v0.y));
-	}
-	static __device__ __forceinline__ float2 lerp2(uint2 e, float k)
-	{
-		T h[2] = {__builtin_bit_cast(T, e.x), __builtin_bit_cast(T, e.y)};
-		return lerp(h, k);
 	}
 };
 template<> struct Entry<MISTA_STORAGE_BF16> {
@@ -80,30 +63,18 @@ template<> struct Entry<MISTA_STORAGE_BF16> {
 	{
 		return make_float2(__uint_as_float(b << 16), __uint_as_float(b & 0xFFFF0000u));
 	}
-	static __device__ __forceinline__ float2 lerp(const T* e, float k)
+	static __device__ __forceinline__ float2 lerp2(uint2 e, float k)
 	{
-		const float2 v0 = get(e[0]), v1 = get(e[1]);
+		const float2 v0 = get(e.x), v1 = get(e.y);
 		return make_float2(fmaf(k, v1.x - v0.x, v0.x), fmaf(k, v1.y - v0.y, v0.y));
 	}
-	static __device__ __forceinline__ float2 lerp2(uint2 e, float k)
-	{
-		const T h[2] = {e.x, e.y};
-		return lerp(h, k);
-	}
 };
-
 template<> struct Entry<kStorageReal> {
 	using T = float;
-	static __device__ __forceinline__ float2 get(T v) { return make_float2(v, 0.0f); }
-	static __device__ __forceinline__ float2 lerp(const T* e, float k)
-	{
-		const float v0 = e[0], v1 = e[1];
-		return make_float2(fmaf(k, v1 - v0, v0), 0.0f);
-	}
 	static __device__ __forceinline__ float2 lerp2(uint2 e, float k)
 	{
-		const T h[2] = {__uint_as_float(e.x), __uint_as_float(e.y)};
-		return lerp(h, k);
+		const float v0 = __uint_as_float(e.x), v1 = __uint_as_float(e.y);
+		return make_float2(fmaf(k, v1 - v0, v0), 0.0f);
 	}
 };
 
@@ -250,7 +221,9 @@ struct TileGeom {
 constexpr uint32_t kEdgeBit = 1u << 31;
 constexpr uint32_t kWsMask = (1u << 24) - 1u;
 constexpr uint32_t kSlotShift = 24;
-constexpr uint32_t kMaxWindowL = 1u << 21;   // records up to here: every ws * ESZ fits the word
+// Records below this: every ws * ESZ fits the word.  (Prepared records end at 2^20
+// samples; longer ones, uploaded, take the record or the gather form.)
+constexpr uint32_t kMaxWindowL = 1u << 21;
 
 // Read-only tables (window words, weights) through the constant address
 // space: uniform indices then become scalar loads.

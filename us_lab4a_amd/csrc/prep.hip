@@ -550,14 +550,12 @@ __device__ __forceinline__ void fft_pass(float2* D, uint32_t M, uint32_t Ns, uin
 // u + i nb, and the partner M - k of bin i is bin R - 1 - i of butterfly
 // nb - u, so a lane takes both butterflies.  u = 0 (bin i with bin R - i) and
 // u = nb/2 (i with R - 1 - i) are their own partners.
-// Butterfly pairs a lane holds: two of radix 5 (u <= M / 10 <= 1.8 NT), one of
-// radix 8 or 9, whose registers would spill (longer transforms run
-// hilbert_in_place and a plain pass).
-template<int R> constexpr int hilbert_slots() { return R == 5 ? 2 : 1; }
-template<int NT, int R>
+// Radix 5 alone, two butterfly pairs a lane (u <= M / 10 <= 1.8 NT): with 8 or 9
+// the registers would spill (those transforms run hilbert_in_place and a plain pass).
+template<int NT>
 __device__ __forceinline__ void hilbert_pass(float2* D, uint32_t M, const float2* __restrict__ wpost)
 {
-	constexpr int MAXP = hilbert_slots<R>();
+	constexpr int R = 5, MAXP = 2;
 	const uint32_t nb = M / R;
 	float2 v1[MAXP][R], v2[MAXP][R];
 #pragma unroll
@@ -658,7 +656,7 @@ __device__ __forceinline__ void analytic_transforms(float2* D, const FftPlanArgs
 	for (uint32_t s = 0; s < 2 * np; ++s) {
 		const uint32_t p = s < np ? s : s - np;
 		if (s == np && pairs) {
-			hilbert_pass<NT, 5>(D, P.M, wpost);
+			hilbert_pass<NT>(D, P.M, wpost);
 			continue;
 		}
 		if (s == np) hilbert_in_place<NT>(D, P.M, wpost);
@@ -668,18 +666,16 @@ __device__ __forceinline__ void analytic_transforms(float2* D, const FftPlanArgs
 	}
 }
 
-// FIR x U output i (no DC removal): the generic polyphase loop over the
-// echo and the filter in LDS, or the raw sample when U = 1.  Deterministic,
-// so a second evaluation gives the same bits as the first.
-__device__ __forceinline__ float fir_at(const AnalyticArgs& A, const float* xs, const float* hs, const float* src,
-		uint32_t i)
+// FIR x U output i (no DC removal) of the 27-tap design: the polyphase loop over
+// the echo and the filter in LDS.  Deterministic, the same bits as the first
+// evaluation.
+__device__ __forceinline__ float fir_at(const AnalyticArgs& A, const float* xs, const float* hs, uint32_t i)
 {
-	if (A.up <= 1) return src[i];
 	const uint32_t m = i + A.off;
-	const float* hrow = hs + (m % A.up) * A.J;
-	const float* xrow = xs + A.J + m / A.up;
+	const float* hrow = hs + (m % A.up) * kFirJ;
+	const float* xrow = xs + kFirJ + m / A.up;
 	float acc = 0.0f;
-	for (uint32_t j = 0; j < A.J; ++j) acc = fmaf(hrow[j], xrow[-static_cast<int>(j)], acc);
+	for (uint32_t j = 0; j < kFirJ; ++j) acc = fmaf(hrow[j], xrow[-static_cast<int>(j)], acc);
 	return acc;
 }
 
@@ -771,17 +767,17 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 	__shared__ float redm[NW], redx[NW], redn[NW];
 	const uint32_t tid = threadIdx.x, ch = blockIdx.x;
 	const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-	const uint32_t M = A.plan.M, N = A.N, L = A.L, up = A.up, J = A.J;
+	const uint32_t M = A.plan.M, N = A.N, L = A.L, up = A.up;
 	float2* D = reinterpret_cast<float2*>(lds);
 	float* Df = reinterpret_cast<float*>(lds);
 	const uint32_t right = A.off / up + 2;
-	// The echo: UP = 0 [J + ns + right] and the taps [up][J] after the transform,
+	// The echo: UP = 0 [kFirJ + ns + right] and the taps [up][kFirJ] after the transform,
 	// UP > 1 [PADL + ns + PADR] after it, too, or (SHARE) in its space, staged
 	// again for the output: 256-lane workgroups, of which four instead of three
 	// then share a CU (64 x 1024 channels of 2048 x 4 samples 2.61 -> 2.34 ms).
 	constexpr bool SHARE = NT == 256 && UP > 1;
 	float* xs = SHARE ? Df : reinterpret_cast<float*>(lds + static_cast<size_t>(M) * sizeof(float2));
-	float* hs = xs + J + A.ns + right;
+	float* hs = xs + kFirJ + A.ns + right;
 	const float* src = A.raw + static_cast<uint64_t>(ch) * A.ns;
 	const uint32_t ntl = (L + 255) / 256;
 	const uint32_t in_tile = 16 * (lane % 16) + 4 * (lane / 16);
@@ -864,47 +860,36 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 		}
 		for (uint32_t i = 256 * ntl + tid; i < N; i += NT) Df[i] = 0.0f;
 	} else {
-		if (up > 1) {
-			for (uint32_t i = tid; i < J + A.ns + right; i += NT) {
-				const int q = static_cast<int>(i) - static_cast<int>(J);
-				xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
-			}
-			for (uint32_t i = tid; i < up * J; i += NT) hs[i] = A.hpoly[i];
-			__syncthreads();
+		for (uint32_t i = tid; i < kFirJ + A.ns + right; i += NT) {
+			const int q = static_cast<int>(i) - static_cast<int>(kFirJ);
+			xs[i] = (q >= 0 && q < static_cast<int>(A.ns)) ? src[q] : 0.0f;
 		}
-		if (up > 1 && J == kFirJ) {
-			// Lane per input position q: the window x[q-26..q] sits in
-			// registers and serves all U phases (outputs m = q*U + p,
-			// i = m - off); the taps, the same for every lane, come through
-			// the scalar cache.
-			const cf32_t hg = (cf32_t)A.hpoly;
-			const uint32_t q_lo = A.off / up, q_hi = (L - 1 + A.off) / up;
-			for (uint32_t q = q_lo + tid; q <= q_hi; q += NT) {
-				float xw[kFirJ];
-				const float* xrow = xs + J + q;
+		for (uint32_t i = tid; i < up * kFirJ; i += NT) hs[i] = A.hpoly[i];
+		__syncthreads();
+		// Lane per input position q: the window x[q-26..q] sits in registers
+		// and serves all U phases (outputs m = q*U + p, i = m - off); the
+		// taps, the same for every lane, come through the scalar cache.
+		const cf32_t hg = (cf32_t)A.hpoly;
+		const uint32_t q_lo = A.off / up, q_hi = (L - 1 + A.off) / up;
+		for (uint32_t q = q_lo + tid; q <= q_hi; q += NT) {
+			float xw[kFirJ];
+			const float* xrow = xs + kFirJ + q;
 #pragma unroll
-				for (int j = 0; j < static_cast<int>(kFirJ); ++j) xw[j] = xrow[-j];
-				const int ibase = static_cast<int>(q * up) - static_cast<int>(A.off);
-				for (uint32_t ph = 0; ph < up; ++ph) {
-					const cf32_t hrow = hg + ph * kFirJ;
-					float acc = 0.0f;
+			for (int j = 0; j < static_cast<int>(kFirJ); ++j) xw[j] = xrow[-j];
+			const int ibase = static_cast<int>(q * up) - static_cast<int>(A.off);
+			for (uint32_t ph = 0; ph < up; ++ph) {
+				const cf32_t hrow = hg + ph * kFirJ;
+				float acc = 0.0f;
 #pragma unroll
-					for (int j = 0; j < static_cast<int>(kFirJ); ++j) acc = fmaf(hrow[j], xw[j], acc);
-					const int i = ibase + static_cast<int>(ph);
-					if (i >= 0 && i < static_cast<int>(L)) {
-						if (static_cast<uint32_t>(i) >= A.dz) part += static_cast<double>(acc);
-						xmax = fmaxf(xmax, acc);
-						xmin = fminf(xmin, acc);
-						Df[i] = acc;
-					}
+				for (int j = 0; j < static_cast<int>(kFirJ); ++j) acc = fmaf(hrow[j], xw[j], acc);
+				const int i = ibase + static_cast<int>(ph);
+				if (i >= 0 && i < static_cast<int>(L)) {
+					if (static_cast<uint32_t>(i) >= A.dz) part += static_cast<double>(acc);
+					xmax = fmaxf(xmax, acc);
+					xmin = fminf(xmin, acc);
+					Df[i] = acc;
 				}
 			}
-		} else for (uint32_t i = tid; i < L; i += NT) {
-			const float acc = fir_at(A, xs, hs, src, i);
-			if (i >= A.dz) part += static_cast<double>(acc);
-			xmax = fmaxf(xmax, acc);
-			xmin = fminf(xmin, acc);
-			Df[i] = acc;
 		}
 		for (uint32_t i = L + tid; i < N; i += NT) Df[i] = 0.0f;
 		reduce_mean();
@@ -1023,7 +1008,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(4, 4)))
 	} else {
 		for (uint32_t i = tid; i < L; i += NT) {
 			const float2 v = D[i >> 1];
-			put1(i, fir_at(A, xs, hs, src, i) - mean, (i & 1u) ? -v.y * coef : v.x * coef);
+			put1(i, fir_at(A, xs, hs, i) - mean, (i & 1u) ? -v.y * coef : v.x * coef);
 		}
 	}
 }
@@ -1598,7 +1583,7 @@ static uint32_t fused_up(uint32_t up, uint32_t J, uint32_t off)
 // transform, the echo, and the taps where the generic FIR runs.
 static size_t fused_lds_bytes(const FrameGeom& g, uint32_t J, uint32_t off)
 {
-	if (g.nf % 2 != 0) return 0;
+	if (g.nf % 2 != 0 || (g.up > 1 && J != kFirJ)) return 0;
 	const uint32_t M = g.nf / 2;
 	if (M > kFftMaxM) return 0;
 	size_t b = static_cast<size_t>(M) * sizeof(float2);
