@@ -522,11 +522,11 @@ def main():
 
 def instruction_bounds(wl, storage, das_ms):
     """Issue-rate bounds of the DAS launch from the committed SQ counter
-    summary for this workload and storage (instructions per 64
-    pixel-pairs): the time the VALU, the scalar unit and the LDS would need
-    alone at one wave64 instruction per 4 cycles per SIMD (VALU, SALU) and
-    the LDS's cycles (instructions plus bank-conflict cycles) per CU, at
-    2.4 GHz over 256 CUs; each against the measured launch."""
+    summary for this workload and storage (per 64 pixel-pairs): the time the
+    VALU and the scalar unit would need alone at one wave64 instruction per 4
+    cycles per SIMD, and the LDS at the cycles that it was active with index
+    operations (bank conflicts among them), at 2.4 GHz over 256 CUs; and the
+    share of the CU cycles that the counters saw busy that each of them took."""
     path = os.path.join(ROOT, "profiles", f"sq_counters_{wl.name}_{storage}.md")
     if not os.path.exists(path):
         return None
@@ -536,16 +536,15 @@ def instruction_bounds(wl, storage, das_ms):
             for kv in line.split(":", 1)[1].split():
                 k, v = kv.split("=")
                 per[k] = float(v)
-    if not per:
+    if "lds_active" not in per or "busy_cu" not in per:
         return None
-    wave_pairs = wl.pixel_pairs / 64.0
-    simd_cycles = 256 * 4 * 2.4e9        # SIMD issue cycles per second
-    cu_cycles = 256 * 2.4e9
-    valu_ms = wave_pairs * per["valu"] * 4 / simd_cycles * 1e3
-    salu_ms = wave_pairs * per["salu"] * 4 / simd_cycles * 1e3
-    lds_ms = wave_pairs * (per["lds"] * per.get("lds_cycles_per_inst", 4.0) + per["lds_conflict"]) / cu_cycles * 1e3
-    return {"valu_ms": round(valu_ms, 3), "salu_ms": round(salu_ms, 3), "lds_ms": round(lds_ms, 3),
-            "launch_ms": round(das_ms, 3), "source": os.path.relpath(path, ROOT), "per_64_pixel_pairs": per}
+    # cycles of a CU: a SIMD issues an instruction in 4, and there are 4 SIMDs
+    cycles = {"valu": per["valu"], "salu": per["salu"], "lds": per["lds_active"]}
+    ms = wl.pixel_pairs / 64.0 / (256 * 2.4e9) * 1e3
+    out = {f"{k}_ms": round(v * ms, 3) for k, v in cycles.items()}
+    out["share_of_busy"] = {k: round(v / per["busy_cu"], 3) for k, v in cycles.items()}
+    out.update(launch_ms=round(das_ms, 3), source=os.path.relpath(path, ROOT), per_64_pixel_pairs=per)
+    return out
 
 
 def tile_name(ran):

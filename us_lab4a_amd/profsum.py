@@ -10,7 +10,7 @@ trace:   per-kernel calls / average / total / per-frame time from
 sq:      instruction mix of the kernel matching --kernel from rocprofv3 --pmc
          runs of SQ counters (any number of directories), per 64 of
          --units (pixel-pairs per dispatch); writes a line "per_wave_pair:
-         valu=.. salu=.. lds=.. lds_conflict=.." that bench.py reads.
+         valu=.. salu=.. lds_active=.. busy_cu=.. ..." that bench.py reads.
 traffic: HBM-side bytes of one dispatch of the kernel matching --kernel from
          two rocprofv3 --pmc runs (FETCH_SIZE, WRITE_SIZE; KiB per dispatch),
          each scaled by what the counter reads for a calibration kernel
@@ -114,7 +114,7 @@ def sq(args):
     for c in sorted(vals):
         out.append(f"| {c} | {vals[c]:.4g} | {vals[c] / wp:.4g} |")
     key = {"valu": "SQ_INSTS_VALU", "salu": "SQ_INSTS_SALU", "lds": "SQ_INSTS_LDS", "lds_conflict": "SQ_LDS_BANK_CONFLICT",
-           "smem": "SQ_INSTS_SMEM", "vmem": "SQ_INSTS_VMEM", "wait_any": "SQ_WAIT_ANY", "wave_cycles": "SQ_WAVE_CYCLES"}
+           "lds_active": "SQ_LDS_IDX_ACTIVE", "busy_cu": "SQ_BUSY_CU_CYCLES", "smem": "SQ_INSTS_SMEM", "vmem": "SQ_INSTS_VMEM", "wait_any": "SQ_WAIT_ANY", "wave_cycles": "SQ_WAVE_CYCLES"}
     kv = " ".join(f"{k}={vals[c] / wp:.4g}" for k, c in key.items() if c in vals)
     if args.note:
         out += ["", args.note]
