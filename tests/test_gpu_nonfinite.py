@@ -4,7 +4,7 @@ import pytest
 
 import oracle
 from us_lab4a_amd import workloads
-from us_lab4a_amd.sta import CoherenceFactor, HipSTARFProcessor
+from us_lab4a_amd.sta import CoherenceFactor, HipSTAProcessor, HipSTARFProcessor, das_batch_device
 
 from parity import say
 
@@ -40,3 +40,49 @@ def test_rf_dead_zone_sample_reaches_its_filter_only(samples, value):
     err = float(np.abs(a[~reach] - a64[~reach]).max() / np.abs(a64).max())
     say("error / peak", f"{err:.2e}")
     assert err <= 2e-6
+
+
+@pytest.mark.parametrize("weight", [np.inf, np.nan])
+def test_infinite_weight_of_an_unheard_element(weight):
+    """Pixels whose echoes by way of element 0 all lie past the record's end: its
+    weight does not matter to them in any form of the kernel."""
+    import torch
+    wl = workloads.Workload2D(name="unheard", num_elements=32, num_samples=512, upsampling=4, cf="sign_coherence_factor",
+                              grid_x=(-4 * MM, 4.5 * MM), grid_z=(8 * MM, 9.6 * MM), n_x=40, n_z=48, points=4,
+                              point_x=(-4 * MM, 4 * MM), point_z=(8 * MM, 9.6 * MM), seed_points=9, seed_noise=10)
+    n = wl.n_x * wl.n_z
+    say("element 0 has weight", weight)
+
+    def processor():
+        rx = np.ones(32, np.float32)
+        p = HipSTAProcessor(wl.sta_config(), None, 4, CoherenceFactor(wl.cf, 1.0), 0.0, rx)
+        p.set_grid(wl.grid())
+        p.process_echoes(wl.echoes_cpu())   # tuned
+        rx[0] = weight
+        p.set_rx_apod(rx)
+        return p
+
+    def out():
+        return [torch.full((n,), -1.0, dtype=torch.float32, device="cuda") for _ in range(2)]
+
+    p, q = processor(), processor()
+    p.set_kernel(1)
+    gather = out()
+    p.das_device(*gather)
+    frames = {}
+    for p0 in (0, 1, 6):
+        frames["tile", p0] = out()
+        p.set_kernel(2 if p0 else 0, p0)
+        p.das_device(*frames["tile", p0])
+    frames["noalloc"] = out()
+    p.das_device_noalloc(*frames["noalloc"])
+    frames["batch"], other = out(), out()
+    das_batch_device([p, q], [frames["batch"][0], other[0]], [frames["batch"][1], other[1]])
+    torch.cuda.synchronize()
+    finite = torch.isfinite(gather[0])
+    assert 0 < int(finite.sum()) < n
+    for name, f in frames.items():
+        for got, want in zip(f, gather):
+            assert np.array_equal(got.cpu().numpy(), want.cpu().numpy(), equal_nan=True), name
+    p.close()
+    q.close()

@@ -30,6 +30,7 @@ struct mista_handle {
 	// apodization (host copies + device copies)
 	std::vector<float> rx_apod, tx_apod;
 	bool tx_apod_set = false;
+	bool finite_apod = true;       // every product of the two
 	DeviceBuffer d_rx_apod, d_tx_apod, d_w;
 	bool weights_dirty = true;
 
@@ -251,6 +252,20 @@ void upload_apod(mista_handle* h, hipStream_t s)
 	h->weights_dirty = false;
 }
 
+// After a change of the apodization.
+void apod_changed(mista_handle* h)
+{
+	auto most = [](const std::vector<float>& w) {
+		float m = 0.0f;
+		for (float v : w) m = std::isfinite(v) ? std::max(m, std::fabs(v)) : INFINITY;
+		return m;
+	};
+	const float rx = most(h->rx_apod), tx = h->tx_apod_set ? most(h->tx_apod) : 1.0f;
+	h->finite_apod = std::isfinite(rx) && std::isfinite(tx) && std::isfinite(rx * tx);
+	h->weights_dirty = true;
+	++h->settings_epoch;
+}
+
 void ensure_events(mista_handle* h)
 {
 	for (auto& e : h->ev)
@@ -287,6 +302,7 @@ void run_das(mista_handle* h, float* d_value, float* d_factor, hipStream_t s)
 	h->geom.ny = h->ny;
 	h->geom.npix = static_cast<uint64_t>(h->n1) * h->n2;
 	h->geom.grid_version = h->grid_version;
+	h->geom.finite_weights = h->finite_apod;
 	upload_apod(h, s);
 	ensure_events(h);
 	// w[tx][rx] = rxApod * txApod * per-channel storage scale
@@ -579,9 +595,8 @@ int mista_set_rx_apod(mista_handle* h, const float* rx_apod, uint32_t n)
 		// unchanged weights (a request loop sets them for every job): no
 		// upload, no stream synchronisation, no new frame graph
 		if (h->rx_apod.size() == n && std::equal(h->rx_apod.begin(), h->rx_apod.end(), rx_apod)) return;
-		++h->settings_epoch;
 		h->rx_apod.assign(rx_apod, rx_apod + n);
-		h->weights_dirty = true;
+		apod_changed(h);
 	});
 }
 
@@ -601,8 +616,7 @@ int mista_set_tx_apod(mista_handle* h, const float* tx_apod, uint32_t n)
 			h->tx_apod.assign(tx_apod, tx_apod + n);
 			h->tx_apod_set = true;
 		}
-		++h->settings_epoch;
-		h->weights_dirty = true;
+		apod_changed(h);
 	});
 }
 
@@ -782,6 +796,7 @@ int mista_das_batch_device(mista_handle* const* handles, uint32_t n, float* cons
 			h->geom.ny = h->ny;
 			h->geom.npix = static_cast<uint64_t>(h->n1) * h->n2;
 			h->geom.grid_version = h->grid_version;
+			h->geom.finite_weights = h->finite_apod;
 			upload_apod(h, s);
 			launch_weights(h->geom, h->d_rx_apod.as<const float>(), h->tx_apod_set ? h->d_tx_apod.as<const float>() : nullptr,
 					h->d_scale.as<const float>(), h->d_w.as<float>(), s);
@@ -807,6 +822,7 @@ int mista_das_device_noalloc(mista_handle* h, float* d_value, float* d_factor, v
 		h->geom.ny = h->ny;
 		h->geom.npix = static_cast<uint64_t>(h->n1) * h->n2;
 		h->geom.grid_version = h->grid_version;
+		h->geom.finite_weights = h->finite_apod;
 		upload_apod(h, s);   // into buffers the preparation reserved
 		launch_weights(h->geom, h->d_rx_apod.as<const float>(), h->tx_apod_set ? h->d_tx_apod.as<const float>() : nullptr,
 				h->d_scale.as<const float>(), h->d_w.as<float>(), s);

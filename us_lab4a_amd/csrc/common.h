@@ -109,6 +109,9 @@ struct FrameGeom {
 	float cf_param;
 	int storage;
 	uint64_t grid_version;  // bumped whenever the grid / delay table changes
+	// The apodization's products are finite.  Else no tiles: there a position
+	// outside the record adds a zero entry times its weight, which has to be zero.
+	bool finite_weights = true;
 };
 
 // Size helpers (FFTUtil.h:100-135, HilbertEnvelope.h:127).

@@ -951,6 +951,7 @@ void launch_das_noalloc(const FrameGeom& g, int tuned_p0, int tuned_p1, DasScrat
 	if (tuned_p0 >= 0) shapes.emplace_back(tuned_p0, tuned_p1);
 	const std::vector<int> defaults = g.ny > 1 ? std::vector<int>{4, 7} : std::vector<int>{1, 5, 6};
 	for (int p0 : defaults) shapes.emplace_back(p0, 0);
+	if (!g.finite_weights) shapes.clear();
 	size_t need_min = ~size_t(0);
 	for (int p0 : defaults) {
 		FrameGeom gl = g;
@@ -961,7 +962,8 @@ void launch_das_noalloc(const FrameGeom& g, int tuned_p0, int tuned_p1, DasScrat
 	if (need_min != ~size_t(0) && need_min > kNoAllocTableBytes)
 		MISTA_THROW(MISTA_E_INVALID_PARAM, "The DAS window tables of this geometry need " << need_min
 				<< " bytes; the no-allocation entry point holds at most " << kNoAllocTableBytes << '.');
-	bool too_large = g.L >= kMaxWindowL;   // no tile of the frame fits the scratch (or the record the window words)
+	// no tile of the frame fits the scratch, or the record the window words, or none may run
+	bool too_large = g.L >= kMaxWindowL || !g.finite_weights;
 	for (const auto& sh : shapes) {
 		const TilePlan tp = tile_plan(g, sh.first);
 		if (!tp.ok) continue;
@@ -1030,7 +1032,9 @@ uint32_t launch_das_batch(const std::vector<DasBatchItem>& items, hipStream_t s)
 		const DasBatchItem& it = items[i];
 		const FrameGeom& g = *it.g;
 		int p0 = -1, p1 = 0;
-		if (it.t->variant != 1 && (it.t->variant == 2 || it.t->p0 || it.t->p1)) {
+		if (!g.finite_weights) {
+			// no tiles
+		} else if (it.t->variant != 1 && (it.t->variant == 2 || it.t->p0 || it.t->p1)) {
 			p0 = it.t->p0;
 			p1 = it.t->p1;
 		} else if (it.t->variant != 1 && it.scratch->tuned_p0 >= 0) {
@@ -1123,7 +1127,7 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 {
 	const DasArgs a = das_args(g, d_tensor, d_delay, d_w, d_value, d_factor);
 
-	const bool can_tile = t.variant != 1 && g.L < kMaxWindowL;
+	const bool can_tile = t.variant != 1 && g.L < kMaxWindowL && g.finite_weights;
 	if (can_tile) {
 		if (t.variant == 2 || t.p0 || t.p1) {
 			if (launch_tiled(g, t.p0, t.p1, scratch, a, d_delay, s)) return;
