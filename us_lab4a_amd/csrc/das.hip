@@ -1198,12 +1198,15 @@ void launch_das(const FrameGeom& g, const DasTuning& t, DasScratch& scratch, con
 						// by up to 1.42.  (256 elements, 512 x 512 points: first
 						// frame 176 -> 108 ms.)
 						float ms = 0.0f;
+						bool run = false;
 						for (int rep = 0; rep < (ms > 5.0f ? 2 : 3); ++rep) {
 							float t = 0.0f;
-							(void)timed(p0, p1, t);
+							run = timed(p0, p1, t);
+							if (!run) break;
 							ms = rep == 0 ? t : std::min(ms, t);
 							if (t > kTuneLimitMs || (bp0 >= 0 && t > 1.0f && t > 1.15f * best)) break;
 						}
+						if (!run) continue;
 						last_p0 = p0;
 						long_frame = long_frame || ms > kTuneLimitMs;
 						const bool lost = bp0 >= 0 && ms > 1.0f && ms > 1.5f * best;
