@@ -235,7 +235,8 @@ int mista_query(const mista_handle* h, uint32_t* signal_length, uint32_t* fft_si
  * workgroup: 4, 8, or 16 on 512-point tiles; 256-point tiles run 4 for 8) |
  * ring buffers << 8 | LDS budget in KiB << 16 | on 2048-point tiles 1 << 24
  * (1024 lanes) or 2 << 24 (1024 lanes, chunks of two receive elements).  Where
- * the variant's tiles do not fit, the rx-parallel form runs instead. */
+ * the variant's tiles do not fit, or an apodization weight is infinite or NaN,
+ * the rx-parallel form runs instead. */
 int mista_set_kernel(mista_handle* h, int variant, int tile_param0, int tile_param1);
 
 /* Frame graphs for mista_process_device (no counterpart in the reference:

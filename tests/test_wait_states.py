@@ -37,7 +37,7 @@ def early_loads(listing):
     return early, loads
 
 
-def test_checker_finds_an_early_load():
+def test_an_early_load_is_found():
     bad = ["0000 <k>:\n", "\ts_mov_b32 m0, s4    // 0: 00\n", "\tglobal_load_lds_dwordx4 v1, s[2:3]    // 4: 00\n"]
     good = bad[:2] + ["\ts_nop 0    // 4: 00\n", bad[2]]
     assert early_loads(bad) == ([("k", "global_load_lds_dwordx4")], 1)
